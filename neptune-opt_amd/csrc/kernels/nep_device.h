@@ -172,6 +172,26 @@ __device__ __forceinline__ u32x4 load16_cached(const void* p) {
 __device__ __forceinline__ void store16(void* p, const u32x4& w) {
   __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(p));
 }
+// The same store at any element alignment: gfx950 runs with unaligned global access on, so
+// this is one global_store_dwordx4 too.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+__device__ __forceinline__ void store16_any(void* p, const u32x4& w) {
+  __builtin_nontemporal_store(w, reinterpret_cast<u32x4_any*>(p));
+}
+
+// How a row kernel walks its rows.
+//   kStrided  one element per load, any column stride
+//   kAligned  16-byte vectors: unit column stride, every row 16-byte aligned, width a multiple
+//             of the vector
+//   kRagged   unit column stride, any alignment and width: the aligned vectors inside the row,
+//             and the elements before and behind them one at a time
+constexpr int kStrided = 0, kAligned = 1, kRagged = 2;
+// A contiguous output row need not share its input row's alignment.
+template <int ACCESS>
+__device__ __forceinline__ void store_vec(void* p, const u32x4& w) {
+  if constexpr (ACCESS == kRagged) store16_any(p, w);
+  else store16(p, w);
+}
 
 // ---------------------------------------------------------------- cross-lane exchange
 // partner<S>(v) returns the value of a lane in the partner group of size S inside the

@@ -18,7 +18,8 @@
 // TPR > 64: several wavefronts per row, merged through LDS).  A row is walked in tiles of
 // TPR*UNROLL*VEC elements; lane t of the row owns slot (u, t) = elements
 // [tile + (u*TPR + t)*VEC, +VEC), so one wavefront-wide load instruction reads consecutive
-// 16-byte segments.  VECTOR=false is the general strided path (one element per slot).
+// 16-byte segments.  VECTOR is the row access (nep_device.h): kAligned, kStrided (one element per
+// slot) or kRagged (see Span).
 #pragma once
 
 namespace nep {
@@ -106,7 +107,7 @@ __device__ __forceinline__ LogLane log_merge(const LogLane& A, const LogLane& B)
 
 
 // ---------------------------------------------------------------- tile access
-template <class St, int TPR, int UNROLL, bool VECTOR>
+template <class St, int TPR, int UNROLL, int VECTOR>
 struct Tiles {
   typedef typename St::T T;
   static constexpr int VEC = VECTOR ? St::kVec : 1;
@@ -125,6 +126,71 @@ struct Tiles {
       v[u] = St::load(row + e * stride_col);
     }
     return true;
+  }
+};
+
+// Raw slots of one tile: 16-byte words (VECTOR) or one element each (strided path).  Slots
+// past the row's end hold -inf elements, so a fold whose phi is the identity needs no per-element
+// test of `ok` (-inf neither raises a max nor adds to an exponential sum).
+template <class St, int UNROLL, int VECTOR>
+struct RawTile {
+  u32x4 w[VECTOR ? UNROLL : 1];
+  float s[VECTOR ? 1 : UNROLL];
+  bool ok[UNROLL];
+};
+
+// Columns [c0, c1) of a row as its access walks them: whole vectors over [v0, v1) and, for a
+// ragged row, the `rest` elements before and behind them (at most VEC-1 each), which form one
+// short tile of one element per slot.  v0 is the row's first 16-byte aligned element, so the
+// vector loads are aligned whatever the row's own alignment.
+//
+// Rows that are not 16-byte aligned or whose width is no multiple of a vector used to take one
+// element per load: a wavefront's load instruction then covers 128 or 256 bytes instead of 1 KB,
+// and the fold is bound by load issue (1.6 TB/s in 16 bits).  Measured on MI355X, cold inputs:
+// logsumexp fp16 8192 x 10007 102.7 -> 34.9 us (4.7 TB/s), bf16 4096 x 50257 217 -> 77 us;
+// log_softmax bf16 4096 x 32003 432 -> 92 us; variance bf16 16384 x 4095 84 -> 29 us.  Vectors
+// from the row's own start, unaligned, measured 42.4, 86 and 110 us for the first three: a
+// wavefront's 1 KB then straddles nine 128-byte lines instead of eight.
+template <class St, int TPR, int VECTOR>
+struct Span {
+  typedef typename St::T T;
+  static constexpr int kRest = 2 * (St::kVec - 1);
+  static constexpr int RU = VECTOR == kRagged ? (kRest + TPR - 1) / TPR : 1;
+  typedef RawTile<St, RU, kStrided> Rest;
+  i64 v0, v1;
+  int head, rest;
+
+  __device__ __forceinline__ Span(const T* row, i64 c0, i64 c1) {
+    v0 = c0;
+    v1 = c1;
+    head = rest = 0;
+    if constexpr (VECTOR == kRagged) {
+      if (c0 >= c1) return;
+      const u64 at = (u64)(row + c0) / sizeof(T);
+      const int n = (int)(c1 - c0 < kRest ? c1 - c0 : kRest);
+      head = (int)(-at & (St::kVec - 1));
+      head = head < n ? head : n;
+      v0 = c0 + head;
+      const int tail = (int)((c1 - v0) & (St::kVec - 1));
+      v1 = c1 - tail;
+      rest = head + tail;
+    }
+  }
+  // Column of rest element i.
+  __device__ __forceinline__ i64 column(int i) const { return i < head ? v0 - head + i : v1 + (i - head); }
+  __device__ __forceinline__ void load_rest(Rest& r, const T* row, int t) const {
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      const int i = u * TPR + t;
+      r.ok[u] = i < rest;
+      r.s[u] = r.ok[u] ? St::load(row + column(i)) : -kInf;
+    }
+  }
+  template <class F>
+  __device__ __forceinline__ void store_rest(const Rest& r, T* out, int t, F value) const {
+#pragma unroll
+    for (int u = 0; u < RU; ++u)
+      if (r.ok[u]) St::store(out + column(u * TPR + t), value(r.s[u]));
   }
 };
 
@@ -181,24 +247,17 @@ __device__ __forceinline__ State log_chunk(Slot slot, float n) {
   return c;
 }
 
-// The reference chunk over one thread's slots of one tile, merged into the running state.
-// Used by every non-exponential fold and, for exponential folds, only on rows whose fast path
-// met NaN or +inf.
-template <class F, class St, int TPR, int UNROLL, bool VECTOR>
-__device__ __forceinline__ void exact_tile(State& s, const typename St::T* row, i64 stride_col,
-                                           i64 tile, i64 c1, int t, float n) {
-  typedef Tiles<St, TPR, UNROLL, VECTOR> TL;
-  float v[TL::K];
-  bool ok[UNROLL];
-#pragma unroll
-  for (int u = 0; u < UNROLL; ++u) ok[u] = TL::load_slot(row, stride_col, tile, c1, t, u, v);
+// The reference chunk over one lane's UNROLL slots of VEC values (slot u valid when ok[u]),
+// merged into the running state.
+template <class F, int UNROLL, int VEC>
+__device__ __forceinline__ void exact_fold(State& s, const float* v, const bool* ok, float n) {
   if constexpr (F::kLog) {
     auto slot = [&](int u, float* w) {
 #pragma unroll
-      for (int j = 0; j < TL::VEC; ++j) w[j] = v[u * TL::VEC + j];
+      for (int j = 0; j < VEC; ++j) w[j] = v[u * VEC + j];
       return ok[u];
     };
-    s = merge_state<F>(s, log_chunk<F, UNROLL, TL::VEC>(slot, n));
+    s = merge_state<F>(s, log_chunk<F, UNROLL, VEC>(slot, n));
   } else {
     // Streaming update (one repair per tile instead of merge_state's two): the tile's terms
     // are taken at the combined producer value, and only the carried accumulator is
@@ -211,8 +270,8 @@ __device__ __forceinline__ void exact_tile(State& s, const typename St::T* row, 
       if (!ok[u]) continue;
       any = true;
 #pragma unroll
-      for (int j = 0; j < TL::VEC; ++j) {
-        const float o = F::phi(v[u * TL::VEC + j], n);
+      for (int j = 0; j < VEC; ++j) {
+        const float o = F::phi(v[u * VEC + j], n);
         mt = F::kProducerSum ? (mt + o) : __builtin_fmaxf(mt, o);
       }
     }
@@ -226,8 +285,8 @@ __device__ __forceinline__ void exact_tile(State& s, const typename St::T* row, 
     for (int u = 0; u < UNROLL; ++u) {
       if (!ok[u]) continue;
 #pragma unroll
-      for (int j = 0; j < TL::VEC; ++j) {
-        const float tv = F::term(v[u * TL::VEC + j], den, n);
+      for (int j = 0; j < VEC; ++j) {
+        const float tv = F::term(v[u * VEC + j], den, n);
         acc = F::kConsumerMax ? __builtin_fmaxf(acc, tv) : (acc + tv);
       }
     }
@@ -241,6 +300,20 @@ __device__ __forceinline__ void exact_tile(State& s, const typename St::T* row, 
     s.acc = acc;
     s.seen = 1;
   }
+}
+
+// The reference chunk over one thread's slots of one tile, merged into the running state.
+// Used by every non-exponential fold and, for exponential folds, only on rows whose fast path
+// met NaN or +inf.
+template <class F, class St, int TPR, int UNROLL, int VECTOR>
+__device__ __forceinline__ void exact_tile(State& s, const typename St::T* row, i64 stride_col,
+                                           i64 tile, i64 c1, int t, float n) {
+  typedef Tiles<St, TPR, UNROLL, VECTOR> TL;
+  float v[TL::K];
+  bool ok[UNROLL];
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u) ok[u] = TL::load_slot(row, stride_col, tile, c1, t, u, v);
+  exact_fold<F, UNROLL, TL::VEC>(s, v, ok, n);
 }
 
 // A row's lane states merged (lanes in order, then waves in order), complete in every lane.
@@ -272,14 +345,20 @@ __device__ __forceinline__ State empty_state() {
 }
 
 // Exact state of the columns [c0, c1) of one row, complete in every lane of the row.
-template <class F, class St, int TPR, int UNROLL, bool VECTOR>
+template <class F, class St, int TPR, int UNROLL, int VECTOR>
 __device__ __forceinline__ State exact_row_state(const typename St::T* row, i64 stride_col,
                                                  i64 c0, i64 c1, int t, float n,
                                                  State* lds_state) {
   typedef Tiles<St, TPR, UNROLL, VECTOR> TL;
   State s = empty_state<F>();
-  for (i64 tile = c0; tile < c1; tile += TL::TILE)
-    exact_tile<F, St, TPR, UNROLL, VECTOR>(s, row, stride_col, tile, c1, t, n);
+  const Span<St, TPR, VECTOR> sp(row, c0, c1);
+  for (i64 tile = sp.v0; tile < sp.v1; tile += TL::TILE)
+    exact_tile<F, St, TPR, UNROLL, VECTOR>(s, row, stride_col, tile, sp.v1, t, n);
+  if constexpr (VECTOR == kRagged) {
+    typename Span<St, TPR, VECTOR>::Rest rest;
+    sp.load_rest(rest, row, t);
+    exact_fold<F, Span<St, TPR, VECTOR>::RU, 1>(s, rest.s, rest.ok, n);
+  }
   return row_state<F, TPR>(s, lds_state);
 }
 
@@ -297,17 +376,7 @@ __device__ __forceinline__ float finalize_state(const State& s, float n) {
 }
 
 // ---------------------------------------------------------------- fast exponential path
-// Raw slots of one tile: 16-byte words (VECTOR) or one element each (strided path).  Slots
-// past the row's end hold -inf elements, so a fold whose phi is the identity needs no per-element
-// test of `ok` (-inf neither raises a max nor adds to an exponential sum).
-template <class St, int UNROLL, bool VECTOR>
-struct RawTile {
-  u32x4 w[VECTOR ? UNROLL : 1];
-  float s[VECTOR ? 1 : UNROLL];
-  bool ok[UNROLL];
-};
-
-template <class St, int TPR, int UNROLL, bool VECTOR>
+template <class St, int TPR, int UNROLL, int VECTOR>
 __device__ __forceinline__ void load_raw(RawTile<St, UNROLL, VECTOR>& r,
                                          const typename St::T* row, i64 stride_col, i64 tile,
                                          i64 c1, int t) {
@@ -319,7 +388,8 @@ __device__ __forceinline__ void load_raw(RawTile<St, UNROLL, VECTOR>& r,
     if constexpr (VECTOR) {
       // a uniform base plus a 32-bit lane offset (the tile is below 2^31 elements)
       const u32 f = St::kNegInfWord;
-      r.w[u] = r.ok[u] ? load16(row + tile + (u32)((u * TPR + t) * TL::VEC)) : u32x4{f, f, f, f};
+      r.w[u] = r.ok[u] ? load16(row + tile + (u32)((u * TPR + t) * TL::VEC))
+                       : u32x4{f, f, f, f};
     } else {
       r.s[u] = r.ok[u] ? St::load(row + e * stride_col) : -kInf;
     }
@@ -329,7 +399,7 @@ __device__ __forceinline__ void load_raw(RawTile<St, UNROLL, VECTOR>& r,
 // The held words of a raw tile, made opaque to the compiler: unpacks after this point cannot
 // reuse values unpacked before it, so a pass over a held row re-derives its fp32 values from
 // the 16-bit words instead of keeping them live (no instruction is emitted).
-template <class St, int UNROLL, bool VECTOR>
+template <class St, int UNROLL, int VECTOR>
 __device__ __forceinline__ void reopen(RawTile<St, UNROLL, VECTOR>& r) {
   if constexpr (VECTOR) {
 #pragma unroll
@@ -351,7 +421,7 @@ __device__ __forceinline__ void reopen(RawTile<St, UNROLL, VECTOR>& r) {
 // CU); the terms and their order are the same.  Only the identity term is recomputed: a
 // term with arithmetic in it (softcap's tanh) is evaluated once and held, since evaluating it
 // twice cost softcap_lse a quarter of its time (fp32 16384x4096: 41.8 -> 51.5 us).
-template <class F, class St, int TPR, int UNROLL, bool VECTOR, bool CENTERED>
+template <class F, class St, int TPR, int UNROLL, int VECTOR, bool CENTERED>
 __device__ __forceinline__ void log_fold_tile(LogLane& s, RawTile<St, UNROLL, VECTOR>& cur,
                                               float n) {
   typedef Tiles<St, TPR, UNROLL, VECTOR> TL;
@@ -422,7 +492,7 @@ __device__ __forceinline__ void log_fold_tile(LogLane& s, RawTile<St, UNROLL, VE
 
 // One lane's exponential fold over its slots of [c0, c1).  The next tile's loads are issued
 // before the current tile is folded, so each lane keeps up to 2*UNROLL loads in flight.
-template <class F, class St, int TPR, int UNROLL, bool VECTOR, bool CENTERED = false>
+template <class F, class St, int TPR, int UNROLL, int VECTOR, bool CENTERED = false>
 __device__ __forceinline__ LogLane log_row_lane(const typename St::T* row, i64 stride_col,
                                                 i64 c0, i64 c1, int t, float n) {
   typedef Tiles<St, TPR, UNROLL, VECTOR> TL;
@@ -431,15 +501,20 @@ __device__ __forceinline__ LogLane log_row_lane(const typename St::T* row, i64 s
   s.acc = 0.0f;
   s.flag = 0;
   if (c0 >= c1) return s;
+  const Span<St, TPR, VECTOR> sp(row, c0, c1);
+  typename Span<St, TPR, VECTOR>::Rest rest;   // issued first: its latency is the first tile's
+  if constexpr (VECTOR == kRagged) sp.load_rest(rest, row, t);
   RawTile<St, UNROLL, VECTOR> cur;
-  load_raw<St, TPR, UNROLL, VECTOR>(cur, row, stride_col, c0, c1, t);
-  for (i64 tile = c0; tile < c1; tile += TL::TILE) {
+  load_raw<St, TPR, UNROLL, VECTOR>(cur, row, stride_col, sp.v0, sp.v1, t);
+  for (i64 tile = sp.v0; tile < sp.v1; tile += TL::TILE) {
     RawTile<St, UNROLL, VECTOR> nxt;
-    const bool more = tile + TL::TILE < c1;
-    if (more) load_raw<St, TPR, UNROLL, VECTOR>(nxt, row, stride_col, tile + TL::TILE, c1, t);
+    const bool more = tile + TL::TILE < sp.v1;
+    if (more) load_raw<St, TPR, UNROLL, VECTOR>(nxt, row, stride_col, tile + TL::TILE, sp.v1, t);
     log_fold_tile<F, St, TPR, UNROLL, VECTOR, CENTERED>(s, cur, n);
     if (more) cur = nxt;
   }
+  if constexpr (VECTOR == kRagged)
+    log_fold_tile<F, St, TPR, Span<St, TPR, VECTOR>::RU, kStrided, CENTERED>(s, rest, n);
   return s;
 }
 
@@ -498,7 +573,7 @@ __device__ __forceinline__ float log_row_result(LogLane s, float n, LogLane* lds
 }
 
 // The same with the exact path re-reading the row from memory.
-template <class F, class St, int TPR, int UNROLL, bool VECTOR>
+template <class F, class St, int TPR, int UNROLL, int VECTOR>
 __device__ __forceinline__ float log_row_finish(LogLane s, const typename St::T* rp,
                                                 i64 stride_col, i64 c1, int t, float n,
                                                 State* lds_state, LogLane* lds_lane) {
@@ -508,7 +583,7 @@ __device__ __forceinline__ float log_row_finish(LogLane s, const typename St::T*
   });
 }
 
-template <class F, class St, int TPR, int UNROLL, bool VECTOR, bool CENTERED = false>
+template <class F, class St, int TPR, int UNROLL, int VECTOR, bool CENTERED = false>
 __device__ __forceinline__ float row_result(const typename St::T* rp, i64 stride_col, i64 c1,
                                             int t, float n, State* lds_state,
                                             LogLane* lds_lane) {
@@ -524,7 +599,7 @@ __device__ __forceinline__ float row_result(const typename St::T* rp, i64 stride
   }
 }
 
-template <class F, class St, int TPR, int UNROLL, bool VECTOR, int WG>
+template <class F, class St, int TPR, int UNROLL, int VECTOR, int WG>
 __device__ __forceinline__ void fold_serial(const typename St::T* __restrict__ x,
                                             typename St::T* __restrict__ out, i64 rows,
                                             i64 ncols, i64 stride_row, i64 stride_col) {
@@ -551,7 +626,7 @@ __device__ __forceinline__ void fold_serial(const typename St::T* __restrict__ x
 // which stay in registers between the fold and the readout (one HBM read); the others take
 // any width and read the row twice.  The two are separate kernels so that each is allocated
 // the registers of its own path.
-template <class F, class St, int TPR, int UNROLL, bool VECTOR, int WG, bool NAN_POSINF,
+template <class F, class St, int TPR, int UNROLL, int VECTOR, int WG, bool NAN_POSINF,
           bool RESIDENT>
 __device__ __forceinline__ void fold_readout(const typename St::T* __restrict__ x,
                                              typename St::T* __restrict__ out, i64 rows,
@@ -570,14 +645,19 @@ __device__ __forceinline__ void fold_readout(const typename St::T* __restrict__ 
   typename St::T* op = out + (live ? row : 0) * ncols;
   const i64 c1 = live ? ncols : 0;
   const float n = (float)ncols;
+  const Span<St, TPR, VECTOR> sp(rp, 0, c1);
+  constexpr int RU = Span<St, TPR, VECTOR>::RU;
+  typename Span<St, TPR, VECTOR>::Rest rest;
   if constexpr (RESIDENT) {
+    if constexpr (VECTOR == kRagged) sp.load_rest(rest, rp, t);
     RawTile<St, UNROLL, VECTOR> keep;
-    load_raw<St, TPR, UNROLL, VECTOR>(keep, rp, stride_col, 0, c1, t);
+    load_raw<St, TPR, UNROLL, VECTOR>(keep, rp, stride_col, sp.v0, sp.v1, t);
     LogLane s;
     s.m = -kInf;
     s.acc = 0.0f;
     s.flag = 0;
     log_fold_tile<F, St, TPR, UNROLL, VECTOR, true>(s, keep, n);
+    if constexpr (VECTOR == kRagged) log_fold_tile<F, St, TPR, RU, kStrided, true>(s, rest, n);
     // The exact fallback takes the row from the registers too: its state equals
     // exact_row_state's over the one tile (same slots, same order), without a second set of
     // fp32 values live beside `keep`.
@@ -593,6 +673,13 @@ __device__ __forceinline__ void fold_readout(const typename St::T* __restrict__ 
           return keep.ok[u];
         };
         e = merge_state<F>(e, log_chunk<F, UNROLL, TL::VEC>(slot, n));
+        if constexpr (VECTOR == kRagged) {
+          auto last = [&](int u, float* w) {
+            w[0] = rest.s[u];
+            return rest.ok[u];
+          };
+          e = merge_state<F>(e, log_chunk<F, RU, 1>(last, n));
+        }
       }
       return row_state<F, TPR>(e, lds_state);
     });
@@ -603,43 +690,49 @@ __device__ __forceinline__ void fold_readout(const typename St::T* __restrict__ 
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       if (!keep.ok[u]) continue;
-      const i64 e = (i64)(u * TPR + t) * TL::VEC;
+      const i64 e = sp.v0 + (i64)(u * TPR + t) * TL::VEC;
       if constexpr (VECTOR) {
         float v[TL::VEC];
         St::unpack(keep.w[u], v);
 #pragma unroll
         for (int j = 0; j < TL::VEC; ++j) v[j] = F::phi(v[j], n) - rr;
-        store16(op + (u32)((u * TPR + t) * TL::VEC), St::pack(v));
+        store_vec<VECTOR>(op + sp.v0 + (u32)((u * TPR + t) * TL::VEC), St::pack(v));
       } else {
         St::store(op + e, F::phi(keep.s[u], n) - rr);
       }
     }
+    if constexpr (VECTOR == kRagged)
+      sp.store_rest(rest, op, t, [&](float v) { return F::phi(v, n) - rr; });
   } else {
     const float r = row_result<F, St, TPR, UNROLL, VECTOR, true>(rp, stride_col, c1, t, n,
                                                                 lds_state, lds_lane);
     const float rr = (NAN_POSINF && r == kInf) ? __builtin_nanf("") : r;
-    for (i64 tile = 0; tile < c1; tile += TL::TILE) {
+    for (i64 tile = sp.v0; tile < sp.v1; tile += TL::TILE) {
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
         const i64 e = tile + (i64)(u * TPR + t) * TL::VEC;
-        if (e >= c1) continue;
+        if (e >= sp.v1) continue;
         if constexpr (VECTOR) {
           float v[TL::VEC];
           St::unpack(load16(rp + e), v);
 #pragma unroll
           for (int j = 0; j < TL::VEC; ++j) v[j] = F::phi(v[j], n) - rr;
-          store16(op + e, St::pack(v));
+          store_vec<VECTOR>(op + e, St::pack(v));
         } else {
           St::store(op + e, F::phi(St::load(rp + e * stride_col), n) - rr);
         }
       }
+    }
+    if constexpr (VECTOR == kRagged) {
+      sp.load_rest(rest, rp, t);
+      sp.store_rest(rest, op, t, [&](float v) { return F::phi(v, n) - rr; });
     }
   }
 }
 
 // Split plan, partial kernel (template.py:137-148): virtual row vr = row*nparts + part covers
 // columns [part*block, min(ncols, (part+1)*block)) and writes its exact chunk state.
-template <class F, class St, int TPR, int UNROLL, bool VECTOR, int WG>
+template <class F, class St, int TPR, int UNROLL, int VECTOR, int WG>
 __device__ __forceinline__ void fold_split_partial(const typename St::T* __restrict__ x,
                                                    float* __restrict__ pm,
                                                    float* __restrict__ pa,
@@ -738,7 +831,7 @@ __device__ __forceinline__ void fold_split_merge(const float* __restrict__ pm,
 
 // Two-pass plan (template.py:62-103): pass 1 reduces the producer over the row, pass 2 the
 // term with the producer held constant.  The second pass re-reads the row.
-template <class F, class St, int TPR, int UNROLL, bool VECTOR, int WG>
+template <class F, class St, int TPR, int UNROLL, int VECTOR, int WG>
 __device__ __forceinline__ void fold_two_pass(const typename St::T* __restrict__ x,
                                               typename St::T* __restrict__ out, i64 rows,
                                               i64 ncols, i64 stride_row, i64 stride_col) {
@@ -755,15 +848,20 @@ __device__ __forceinline__ void fold_two_pass(const typename St::T* __restrict__
   const int wave = threadIdx.x >> 6, first = (wave / RC::WPR) * RC::WPR;
   // A row that fits in one tile stays in registers: pass 2 reads what pass 1 loaded, so the
   // row crosses HBM once (same values, same order as reading it twice).
+  const Span<St, TPR, VECTOR> sp(rp, 0, c1);
+  constexpr int RU = Span<St, TPR, VECTOR>::RU;
   const bool resident = ncols <= TL::TILE;
   float keep[TL::K];
   bool kept[UNROLL];
+  // a ragged row's last elements, held from here to the second pass
+  typename Span<St, TPR, VECTOR>::Rest rest;
+  if constexpr (VECTOR == kRagged) sp.load_rest(rest, rp, t);
   // pass 1: the producer
   float m = F::kProducerSum ? 0.0f : -kInf;
   if (resident) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      kept[u] = TL::load_slot(rp, stride_col, 0, c1, t, u, keep);
+      kept[u] = TL::load_slot(rp, stride_col, sp.v0, sp.v1, t, u, keep);
       if (!kept[u]) continue;
 #pragma unroll
       for (int j = 0; j < TL::VEC; ++j) {
@@ -772,17 +870,25 @@ __device__ __forceinline__ void fold_two_pass(const typename St::T* __restrict__
       }
     }
   } else {
-    for (i64 tile = 0; tile < c1; tile += TL::TILE) {
+    for (i64 tile = sp.v0; tile < sp.v1; tile += TL::TILE) {
       float v[TL::K];
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
-        if (!TL::load_slot(rp, stride_col, tile, c1, t, u, v)) continue;
+        if (!TL::load_slot(rp, stride_col, tile, sp.v1, t, u, v)) continue;
 #pragma unroll
         for (int j = 0; j < TL::VEC; ++j) {
           const float o = F::phi(v[u * TL::VEC + j], n);
           m = F::kProducerSum ? (m + o) : __builtin_fmaxf(m, o);
         }
       }
+    }
+  }
+  if constexpr (VECTOR == kRagged) {
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      if (!rest.ok[u]) continue;
+      const float o = F::phi(rest.s[u], n);
+      m = F::kProducerSum ? (m + o) : __builtin_fmaxf(m, o);
     }
   }
   m = F::kProducerSum ? group_sum<RC::G>(m) : group_max<RC::G>(m);
@@ -809,17 +915,25 @@ __device__ __forceinline__ void fold_two_pass(const typename St::T* __restrict__
       }
     }
   } else {
-    for (i64 tile = 0; tile < c1; tile += TL::TILE) {
+    for (i64 tile = sp.v0; tile < sp.v1; tile += TL::TILE) {
       float v[TL::K];
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u) {
-        if (!TL::load_slot(rp, stride_col, tile, c1, t, u, v)) continue;
+        if (!TL::load_slot(rp, stride_col, tile, sp.v1, t, u, v)) continue;
 #pragma unroll
         for (int j = 0; j < TL::VEC; ++j) {
           const float tv = F::term(v[u * TL::VEC + j], m, n);
           acc = F::kConsumerMax ? __builtin_fmaxf(acc, tv) : (acc + tv);
         }
       }
+    }
+  }
+  if constexpr (VECTOR == kRagged) {
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      if (!rest.ok[u]) continue;
+      const float tv = F::term(rest.s[u], m, n);
+      acc = F::kConsumerMax ? __builtin_fmaxf(acc, tv) : (acc + tv);
     }
   }
   acc = F::kConsumerMax ? group_max<RC::G>(acc) : group_sum<RC::G>(acc);

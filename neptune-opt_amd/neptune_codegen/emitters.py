@@ -193,22 +193,36 @@ def emit_fold_policy(sk: Skeleton, values: dict | None = None, *, struct_name: s
 """
 
 
+def access_name(vector: bool, ragged: bool) -> str:
+    """The row access of a launch shape, as nep_device.h names it."""
+    return ("nep::kRagged" if ragged else "nep::kAligned") if vector else "nep::kStrided"
+
+
+def access_tag(vector: bool, ragged: bool) -> str:
+    return ("r" if ragged else "v") if vector else "s"
+
+
 @dataclasses.dataclass(frozen=True)
 class FoldVariant:
     """One launch shape of a scalar fold kernel."""
 
     dtype: str          # "float32" | "bfloat16" | "float16"
-    vector: bool        # 16-byte loads (unit column stride, aligned rows)
+    vector: bool        # 16-byte loads (unit column stride)
     tpr: int            # lanes per row (or per split partial)
     unroll: int = 4     # slots per lane per tile
     waves: int = 4      # wave64s per workgroup (at least one row)
+    ragged: bool = False    # vector rows of any alignment and width (nep_device.h kRagged)
 
     @property
     def wg(self) -> int:
         return max(64 * self.waves, self.tpr)
 
+    @property
+    def access(self) -> str:
+        return access_name(self.vector, self.ragged)
+
     def tag(self) -> str:
-        return (f"{dtype_tag(self.dtype)[0]}_{'v' if self.vector else 's'}{self.tpr}"
+        return (f"{dtype_tag(self.dtype)[0]}_{access_tag(self.vector, self.ragged)}{self.tpr}"
                 f"u{self.unroll}w{self.waves}")
 
 
@@ -219,8 +233,7 @@ _FOLD_ARGS_SERIAL = ("const void* x, void* out, long long rows, long long ncols,
 def _fold_kernel(sk: Skeleton, plan: str, part: str, var: FoldVariant) -> tuple[str, str]:
     """(kernel name, extern "C" definition) for one plan stage and variant."""
     _, st = dtype_tag(var.dtype)
-    vec = "true" if var.vector else "false"
-    tmpl = f"Fold, {st}, {var.tpr}, {var.unroll}, {vec}, {var.wg}"
+    tmpl = f"Fold, {st}, {var.tpr}, {var.unroll}, {var.access}, {var.wg}"
     if plan == "serial":
         name = f"{sk.name}_serial_{var.tag()}"
         body = (f"nep::fold_serial<{tmpl}>((const {st}::T*)x, ({st}::T*)out, rows, ncols, "
@@ -317,7 +330,6 @@ def emit_readout_source(sk: Skeleton, values: dict | None = None, *, variants: t
     seen = set()
     for var in variants:
         _, st = dtype_tag(var.dtype)
-        vec = "true" if var.vector else "false"
         for resident in (True, False):
             name = readout_kernel_name(sk, var, nan_posinf_rows, resident)
             if name in seen:
@@ -325,7 +337,7 @@ def emit_readout_source(sk: Skeleton, values: dict | None = None, *, variants: t
             seen.add(name)
             parts.append(
                 f'extern "C" __global__ void __launch_bounds__({var.wg}) {name}({_FOLD_ARGS_SERIAL}) {{\n'
-                f"  nep::fold_readout<Fold, {st}, {var.tpr}, {var.unroll}, {vec}, {var.wg}, {flag}, "
+                f"  nep::fold_readout<Fold, {st}, {var.tpr}, {var.unroll}, {var.access}, {var.wg}, {flag}, "
                 f"{'true' if resident else 'false'}>("
                 f"(const {st}::T*)x, ({st}::T*)out, rows, ncols, stride_row, stride_col);\n}}\n")
     return "\n".join(parts)

@@ -241,6 +241,13 @@ def _is_vector(x2, ncols: int, vec: int, extra_align: int = 0) -> bool:
             and x2.data_ptr() % 16 == 0 and (extra_align == 0 or extra_align % vec == 0))
 
 
+def _is_ragged(x2, ncols: int, vec: int) -> bool:
+    """Rows of unit column stride and at least one vector wide, whatever their alignment: the
+    vectors inside the row are loaded whole (nep_fold.h Span, with both sides measured).  A
+    narrower row may hold no vector at all."""
+    return x2.dim() == 2 and x2.stride(1) == 1 and ncols >= vec
+
+
 def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: int = 0,
                   resident: bool = False, merge_heavy: bool = False,
                   heavy_phi: bool = False) -> FoldVariant:
@@ -269,8 +276,10 @@ def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: in
     (bf16 and fp32)."""
     vec = vec_of(x2.dtype)
     vector = _is_vector(x2, ncols, vec, split_block)
+    ragged = not vector and _is_ragged(x2, ncols, vec)
+    vector = vector or ragged
     if vector and split_block and split_block < vec:
-        vector = False
+        vector = ragged = False
     tpr = lanes_per_row(block, vec if vector else 1)
     waves = max(1, min(16, int(num_warps)))
     waves = 1 << (waves - 1).bit_length()
@@ -303,7 +312,7 @@ def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: in
             tpr *= 2
     if per_slot == 8 and (merge_heavy or resident) and not split_block and tpr == 64:
         waves = 1              # one row per 64-lane workgroup (bf16 8192 wide: 54.0 -> 48.7 us)
-    return FoldVariant(str(x2.dtype).replace("torch.", ""), vector, tpr, unroll, waves)
+    return FoldVariant(str(x2.dtype).replace("torch.", ""), vector, tpr, unroll, waves, ragged)
 
 
 def _grid_1d(items: int, per_wg: int) -> int:
