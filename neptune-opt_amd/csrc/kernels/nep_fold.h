@@ -19,7 +19,7 @@
 // TPR*UNROLL*VEC elements; lane t of the row owns slot (u, t) = elements
 // [tile + (u*TPR + t)*VEC, +VEC), so one wavefront-wide load instruction reads consecutive
 // 16-byte segments.  VECTOR is the row access (nep_device.h): kAligned, kStrided (one element per
-// slot) or kRagged (see Span).
+// slot) or kRagged (see Span there).
 #pragma once
 
 namespace nep {
@@ -126,71 +126,6 @@ struct Tiles {
       v[u] = St::load(row + e * stride_col);
     }
     return true;
-  }
-};
-
-// Raw slots of one tile: 16-byte words (VECTOR) or one element each (strided path).  Slots
-// past the row's end hold -inf elements, so a fold whose phi is the identity needs no per-element
-// test of `ok` (-inf neither raises a max nor adds to an exponential sum).
-template <class St, int UNROLL, int VECTOR>
-struct RawTile {
-  u32x4 w[VECTOR ? UNROLL : 1];
-  float s[VECTOR ? 1 : UNROLL];
-  bool ok[UNROLL];
-};
-
-// Columns [c0, c1) of a row as its access walks them: whole vectors over [v0, v1) and, for a
-// ragged row, the `rest` elements before and behind them (at most VEC-1 each), which form one
-// short tile of one element per slot.  v0 is the row's first 16-byte aligned element, so the
-// vector loads are aligned whatever the row's own alignment.
-//
-// Rows that are not 16-byte aligned or whose width is no multiple of a vector used to take one
-// element per load: a wavefront's load instruction then covers 128 or 256 bytes instead of 1 KB,
-// and the fold is bound by load issue (1.6 TB/s in 16 bits).  Measured on MI355X, cold inputs:
-// logsumexp fp16 8192 x 10007 102.7 -> 34.9 us (4.7 TB/s), bf16 4096 x 50257 217 -> 77 us;
-// log_softmax bf16 4096 x 32003 432 -> 92 us; variance bf16 16384 x 4095 84 -> 29 us.  Vectors
-// from the row's own start, unaligned, measured 42.4, 86 and 110 us for the first three: a
-// wavefront's 1 KB then straddles nine 128-byte lines instead of eight.
-template <class St, int TPR, int VECTOR>
-struct Span {
-  typedef typename St::T T;
-  static constexpr int kRest = 2 * (St::kVec - 1);
-  static constexpr int RU = VECTOR == kRagged ? (kRest + TPR - 1) / TPR : 1;
-  typedef RawTile<St, RU, kStrided> Rest;
-  i64 v0, v1;
-  int head, rest;
-
-  __device__ __forceinline__ Span(const T* row, i64 c0, i64 c1) {
-    v0 = c0;
-    v1 = c1;
-    head = rest = 0;
-    if constexpr (VECTOR == kRagged) {
-      if (c0 >= c1) return;
-      const u64 at = (u64)(row + c0) / sizeof(T);
-      const int n = (int)(c1 - c0 < kRest ? c1 - c0 : kRest);
-      head = (int)(-at & (St::kVec - 1));
-      head = head < n ? head : n;
-      v0 = c0 + head;
-      const int tail = (int)((c1 - v0) & (St::kVec - 1));
-      v1 = c1 - tail;
-      rest = head + tail;
-    }
-  }
-  // Column of rest element i.
-  __device__ __forceinline__ i64 column(int i) const { return i < head ? v0 - head + i : v1 + (i - head); }
-  __device__ __forceinline__ void load_rest(Rest& r, const T* row, int t) const {
-#pragma unroll
-    for (int u = 0; u < RU; ++u) {
-      const int i = u * TPR + t;
-      r.ok[u] = i < rest;
-      r.s[u] = r.ok[u] ? St::load(row + column(i)) : -kInf;
-    }
-  }
-  template <class F>
-  __device__ __forceinline__ void store_rest(const Rest& r, T* out, int t, F value) const {
-#pragma unroll
-    for (int u = 0; u < RU; ++u)
-      if (r.ok[u]) St::store(out + column(u * TPR + t), value(r.s[u]));
   }
 };
 

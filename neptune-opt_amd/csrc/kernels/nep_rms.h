@@ -32,7 +32,7 @@ __device__ __forceinline__ float row_sum(float v, float* lds) {
   return v;
 }
 
-template <class St, bool VECTOR>
+template <class St, int VECTOR>
 struct RowIO {
   typedef typename St::T T;
   static constexpr int VEC = VECTOR ? St::kVec : 1;
@@ -98,11 +98,57 @@ __device__ __forceinline__ float rms_scale(float total, float count, float eps) 
   }
 }
 
+// One row held as packed 16-byte words (word u at column `first(u)`, valid when `first(u) < end`),
+// plus, for a ragged row, the span's rest: reads out every element of the row.  L2 divides
+// through div_by_row; a lane holding an element outside its exact range, or a row whose norm (or
+// its reciprocal) is not a normal number -- an infinite sum of squares, a denormal eps under an
+// underflowed sum, an eps of 2^126 or more -- stores div_rn results over them afterwards.
+template <class St, int NV, int VECTOR, bool L2, class First, class Gamma>
+__device__ __forceinline__ void rms_store_words(typename St::T* op, const u32x4* xr, float scale,
+                                                i64 end, First first, Gamma gamma) {
+  constexpr int VEC = St::kVec;
+  const float inv = L2 ? 1.0f / scale : 0.0f;
+  const float tiny = L2 ? __builtin_fmaxf(0x1p-100f, scale * 0x1p-125f) : 0.0f;
+  bool redo = L2 && !(scale >= 0x1p-126f && scale <= 0x1p126f);
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    const i64 e = first(u);
+    if (e >= end) continue;
+    float v[VEC], g[VEC], y[VEC];
+    St::unpack(xr[u], v);
+    if constexpr (!L2) St::unpack(gamma(u), g);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      if constexpr (L2) {
+        y[j] = div_by_row(v[j], scale, inv);
+        redo |= (__builtin_fabsf(v[j]) < tiny) & (v[j] != 0.0f);
+      } else {
+        y[j] = rms_readout<St, L2>(v[j], g[j], scale);
+      }
+    }
+    store_vec<VECTOR>(op + e, St::pack(y));
+  }
+  if constexpr (L2) {
+    if (redo) {
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        const i64 e = first(u);
+        if (e >= end) continue;
+        float v[VEC], y[VEC];
+        St::unpack(xr[u], v);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) y[j] = div_rn(v[j], scale);
+        store_vec<VECTOR>(op + e, St::pack(y));
+      }
+    }
+  }
+}
+
 // Serial plan: x [rows, ncols] strided -> out [rows, ncols] contiguous.
 // Requires ncols <= TPR * NV * VEC (checked by the host).  The vector path keeps the row and
 // gamma as packed 16-byte words (NV words each per lane) and unpacks on use, which halves the
 // registers of holding them as fp32.
-template <class St, int TPR, int NV, bool VECTOR, bool L2, int WG>
+template <class St, int TPR, int NV, int VECTOR, bool L2, int WG>
 __device__ __forceinline__ void rms_serial(const typename St::T* __restrict__ x,
                                            const typename St::T* __restrict__ gamma,
                                            typename St::T* __restrict__ out, i64 rows,
@@ -114,7 +160,7 @@ __device__ __forceinline__ void rms_serial(const typename St::T* __restrict__ x,
   __shared__ float lds[WG / 64];
   const int t = threadIdx.x % TPR;
   const float count = (float)ncols;
-  if constexpr (VECTOR) {
+  if constexpr (VECTOR == kAligned) {
     // gamma stays in registers as packed words (NV per lane) and is unpacked at its use: no LDS
     // staging and no barrier before the first row (84.1 -> 83.7 us at cfg3).
     u32x4 gr[L2 ? 1 : NV];
@@ -164,45 +210,62 @@ __device__ __forceinline__ void rms_serial(const typename St::T* __restrict__ x,
       total = row_sum<TPR>(total, lds);
       const float scale = rms_scale<L2>(total, count, eps);
       typename St::T* op = out + (live ? row : 0) * ncols;
-      // L2: the row's elements are divided through div_by_row; a lane holding an element
-      // outside its exact range, or a row whose norm (or its reciprocal) is not a normal
-      // number -- an infinite sum of squares, a denormal eps under an underflowed sum, an
-      // eps of 2^126 or more -- stores div_rn results over them afterwards.
-      const float inv = L2 ? 1.0f / scale : 0.0f;
-      const float tiny = L2 ? __builtin_fmaxf(0x1p-100f, scale * 0x1p-125f) : 0.0f;
-      bool redo = L2 && !(scale >= 0x1p-126f && scale <= 0x1p126f);
+      rms_store_words<St, NV, VECTOR, L2>(
+          op, xr, scale, c1, [&](int u) { return (i64)(u * TPR + t) * VEC; },
+          [&](int u) { return gr[u]; });
+    }
+  } else if constexpr (VECTOR == kRagged) {
+    // The row's aligned vectors as packed words and the elements around them one per slot; each
+    // row has its own alignment, so gamma's words (unaligned, cached) are loaded per row.  Bound
+    // by HBM: bf16 8192 x 3001 95.6 us with one element per load, 21.3 us (4.6 TB/s) so.
+    typedef Span<St, TPR, kRagged> Sp;
+    for (i64 base = (i64)blockIdx.x * RPW; base < rows; base += (i64)gridDim.x * RPW) {
+      const i64 row = base + threadIdx.x / TPR;
+      const bool live = row < rows;
+      const typename St::T* rp = x + (live ? row : 0) * stride_row;
+      const Sp sp(rp, 0, live ? ncols : 0);
+      u32x4 xr[NV], gr[L2 ? 1 : NV];
+      typename Sp::Rest rest;
+      float g_rest[L2 ? 1 : Sp::RU];
 #pragma unroll
       for (int u = 0; u < NV; ++u) {
-        const i64 e = (i64)(u * TPR + t) * VEC;
-        if (e >= c1) continue;
-        float v[VEC], g[VEC], y[VEC];
+        const i64 e = sp.v0 + (i64)(u * TPR + t) * VEC;
+        xr[u] = e < sp.v1 ? load16(rp + e) : u32x4{0u, 0u, 0u, 0u};
+      }
+      sp.load_rest(rest, rp, t);
+      if constexpr (!L2) {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+          const i64 e = sp.v0 + (i64)(u * TPR + t) * VEC;
+          gr[u] = e < sp.v1 ? load16_any(gamma + e) : u32x4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int u = 0; u < Sp::RU; ++u)
+          g_rest[u] = rest.ok[u] ? St::load(gamma + sp.column(u * TPR + t)) : 0.0f;
+      }
+      float total = 0.0f;
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        float v[VEC];
         St::unpack(xr[u], v);
-        if constexpr (!L2) St::unpack(gr[u], g);
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) {
-          if constexpr (L2) {
-            y[j] = div_by_row(v[j], scale, inv);
-            redo |= (__builtin_fabsf(v[j]) < tiny) & (v[j] != 0.0f);
-          } else {
-            y[j] = rms_readout<St, L2>(v[j], g[j], scale);
-          }
-        }
-        store16(op + e, St::pack(y));
+        for (int j = 0; j < VEC; ++j) total += v[j] * v[j];
       }
-      if constexpr (L2) {
-        if (redo) {
 #pragma unroll
-          for (int u = 0; u < NV; ++u) {
-            const i64 e = (i64)(u * TPR + t) * VEC;
-            if (e >= c1) continue;
-            float v[VEC], y[VEC];
-            St::unpack(xr[u], v);
+      for (int u = 0; u < Sp::RU; ++u) total += rest.ok[u] ? rest.s[u] * rest.s[u] : 0.0f;
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) y[j] = div_rn(v[j], scale);
-            store16(op + e, St::pack(y));
-          }
-        }
-      }
+      for (int u = 0; u < NV; ++u) asm volatile("" : "+v"(xr[u]));
+      total = row_sum<TPR>(total, lds);
+      const float scale = rms_scale<L2>(total, count, eps);
+      typename St::T* op = out + (live ? row : 0) * ncols;
+      rms_store_words<St, NV, VECTOR, L2>(
+          op, xr, scale, sp.v1, [&](int u) { return sp.v0 + (i64)(u * TPR + t) * VEC; },
+          [&](int u) { return gr[u]; });
+#pragma unroll
+      for (int u = 0; u < Sp::RU; ++u)
+        if (rest.ok[u])
+          St::store(op + sp.column(u * TPR + t),
+                    rms_readout<St, L2>(rest.s[u], L2 ? 0.0f : g_rest[L2 ? 0 : u], scale));
     }
   } else {
     float g[L2 ? 1 : NV];
@@ -235,7 +298,7 @@ __device__ __forceinline__ void rms_serial(const typename St::T* __restrict__ x,
 
 // Split plan, partial statistics (emitters.py:597-610): virtual row vr = row*nparts + part
 // covers columns [part*block, min(ncols, (part+1)*block)); writes (total fp32, count int64).
-template <class St, int TPR, int NV, bool VECTOR, int WG>
+template <class St, int TPR, int NV, int VECTOR, int WG>
 __device__ __forceinline__ void rms_split_partial(const typename St::T* __restrict__ x,
                                                   float* __restrict__ totals,
                                                   i64* __restrict__ counts, i64 rows,
@@ -273,7 +336,7 @@ __device__ __forceinline__ void rms_split_partial(const typename St::T* __restri
 
 // Split plan, map kernel (emitters.py:613-627): every (row, tile) merges all of the row's
 // partial statistics, then normalizes its own tile of `block` columns.
-template <class St, int TPR, int NV, bool VECTOR, bool L2, int WG>
+template <class St, int TPR, int NV, int VECTOR, bool L2, int WG>
 __device__ __forceinline__ void rms_split_map(const typename St::T* __restrict__ x,
                                               const typename St::T* __restrict__ gamma,
                                               const float* __restrict__ totals,

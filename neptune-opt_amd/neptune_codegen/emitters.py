@@ -357,13 +357,19 @@ class RowVariant:
     vector: bool
     tpr: int
     nv: int             # 16-byte slots (or elements) per lane
+    ragged: bool = False    # vector rows of any alignment and width (nep_device.h kRagged)
 
     @property
     def wg(self) -> int:
         return max(256, self.tpr)
 
+    @property
+    def access(self) -> str:
+        return access_name(self.vector, self.ragged)
+
     def tag(self) -> str:
-        return f"{dtype_tag(self.dtype)[0]}_{'v' if self.vector else 's'}{self.tpr}n{self.nv}"
+        return (f"{dtype_tag(self.dtype)[0]}_{access_tag(self.vector, self.ragged)}{self.tpr}"
+                f"n{self.nv}")
 
 
 def _check_eps(params: dict) -> float:
@@ -405,7 +411,7 @@ def emit_rms_state_source(spec, params=None, *, plan: str = "serial",
              f"constexpr float kEps = {f32_literal(eps)};  // eps={eps!r}\n"]
     for var in variants:
         _, st = dtype_tag(var.dtype)
-        vec = "true" if var.vector else "false"
+        vec = var.access
         if plan == "serial":
             name = f"{spec.name}_serial_{var.tag()}"
             parts.append(

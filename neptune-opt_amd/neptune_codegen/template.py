@@ -557,16 +557,27 @@ def _row_variant(flat, gamma, width: int, *, tile: int | None = None) -> RowVari
     width 4096: 4 slots 85.7 / 86.9, 2 slots 86.1 / 87.8, 8 slots 87.9 / 89.1 (a second run:
     4 slots 85.4-85.6 / 86.4-86.8, 8 slots 86.8-88.0 / 87.8-88.7);
     width 8192: 4 slots 87.4 / 88.6, 8 slots 89.0 / 90.5;
-    width 16384: 8 slots 88.4 / 89.0, 4 slots 89.0 / 88.9."""
+    width 16384: 8 slots 88.4 / 89.0, 4 slots 89.0 / 88.9.
+
+    Ragged rows (nep_device.h Span; gamma of unit stride, any alignment) take 2 slots in fp32 and
+    4 in 16 bits, 8 above 4096 elements: fp32 L2 20000 x 2999 78.7 us (3 slots 82.0, 6 84.4),
+    bf16 RMSNorm 32768 x 1001 27.3 (2 slots 27.2, 8 32.0), fp16 8192 x 8191 50.3 (4 slots 54.4).
+    One element per load, as these rows were read before: fp32 20000 x 2999 82.3, bf16
+    8192 x 3001 95.6 (now 21.3), fp16 4096 x 8192 in rows of 8205 124 (now 29.8)."""
     vec = vec_of(flat.dtype)
     vector = _is_vector(flat, width, vec, tile or 0)
     if vector and gamma is not None:
         vector = gamma.stride(0) == 1 and gamma.data_ptr() % 16 == 0
+    ragged = (not vector and tile is None and _is_ragged(flat, width, vec)
+              and (gamma is None or gamma.stride(0) == 1))
+    vector = vector or ragged
     span = tile if tile is not None else width
     slots = (span + vec - 1) // vec if vector else span
     nv = 8 if vector else 16
     if vector and vec == 8 and 128 <= slots <= 1024:
         nv = 4 if slots >= 256 else 2
+    if ragged:
+        nv = 2 if vec == 4 else (4 if slots <= 512 else 8)
     if tile is not None:
         nv = 2 if vector else 8
     tpr = 1 << max(0, (max(1, -(-slots // nv)) - 1).bit_length())
@@ -574,8 +585,7 @@ def _row_variant(flat, gamma, width: int, *, tile: int | None = None) -> RowVari
         nv *= 2
         tpr = 1 << max(0, (max(1, -(-slots // nv)) - 1).bit_length())
     nv = max(1, min(nv, -(-slots // tpr)))
-    nv = 1 << (nv - 1).bit_length()
-    return RowVariant(str(flat.dtype).replace("torch.", ""), vector, tpr, nv)
+    return RowVariant(str(flat.dtype).replace("torch.", ""), vector, tpr, nv, ragged)
 
 
 def _persistent_grid(items_per_wg: int, items: int, device) -> int:

@@ -109,3 +109,49 @@ def test_ragged_rule():
     assert access(x) == "Aligned"
     assert access(x[:, :1001]) == "Ragged" and access(x[:, 1:1001]) == "Ragged"
     assert access(x[:, :7]) == "Strided" and access(x[:, ::2]) == "Strided"
+
+
+def _ulps(got, want, dtype):
+    """Largest distance in units of the last place (as ordered integers) over finite values."""
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    a, b = got.view(bits).long(), want.view(bits).long()
+    low = torch.iinfo(bits).min
+    a, b = torch.where(a < 0, low - a, a), torch.where(b < 0, low - b, b)
+    return int((a - b).abs().max())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_ragged_norms(dtype):
+    """RMSNorm and L2-normalize at ragged rows, gamma at another alignment than its rows, against
+    fp64 statistics with the same rounding stages: the fp32 sum's order moves the scale by at most
+    a few fp32 units (4 here), which in 16 bits can flip one rounding at each of two stages."""
+    for width, offset, pad in SHAPES + [(16383, 1, 0), (32767, 0, 1)]:
+        x, dev = _rows(21, width, dtype, offset, pad)
+        gamma = (1 + 0.1 * torch.randn(width + 3, generator=torch.Generator().manual_seed(4))).to(dtype)
+        g_dev = gamma.cuda()[3:]
+        gamma = gamma[3:]
+        _say(f"ragged norms {dtype} width={width} offset={offset} pad={pad}")
+        xd = x.double()
+        scale = torch.rsqrt(xd.square().mean(-1, True) + 1e-6).float()
+        want = ((x.float() * scale).to(dtype).float() * gamma.float()).to(dtype)
+        got = CG.run_rms_norm(dev, g_dev, eps=1e-6).cpu()
+        assert _ulps(got, want, dtype) <= (8 if dtype == torch.float32 else 2)
+        want = (x.float() / xd.square().sum(-1, True).sqrt().float()).to(dtype)
+        got = CG.run_l2_normalize(dev, eps=1e-6).cpu()
+        assert _ulps(got, want, dtype) <= (8 if dtype == torch.float32 else 1)
+
+
+def test_ragged_l2_exact_division_of_tiny_and_huge_norms():
+    """Rows whose norm is not a normal number, or that hold denormal quotients, take the exact
+    division in the vector part too; a zero row divides by eps."""
+    width = 1001
+    x, dev = _rows(5, width, torch.float32, 1, 0)
+    x[0] = 0.0
+    x[1] *= 2.0 ** 66           # the sum of squares overflows: x / inf = 0
+    x[2] *= 2.0 ** -80          # the sum of squares underflows to a denormal or 0
+    x[3, 1:-1] *= 2.0 ** -120   # quotients in the denormal range beside ordinary ones
+    dev.copy_(x)
+    got = CG.run_l2_normalize(dev, eps=1e-6).cpu()
+    norm = x.square().sum(-1, True).sqrt().clamp_min(1e-6)
+    assert torch.equal(got[1], torch.zeros(width)) and torch.equal(got[0], torch.zeros(width))
+    assert _ulps(got[2:], (x / norm)[2:], torch.float32) <= 8
