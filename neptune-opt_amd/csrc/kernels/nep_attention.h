@@ -651,6 +651,303 @@ __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* 
 }
 
 
+// ---------------------------------------------------------------- short query ranges
+// Attention of few queries over many keys (decoding; the query heads that share a key head folded
+// into the query axis).  The kernels above give a head's queries one workgroup of 256 query slots
+// and stage V twice; here a head's keys are split over workgroups and waves instead, and K and V
+// are read once, in place, without LDS or a V^T image:
+//  * one workgroup = 4 independent wave64s x 16 query slots over one chunk of keys of one head; wave
+//    w takes the chunk's 32-key tiles w, w+4, ..., its next K tile in flight while it computes;
+//  * S^T = K Q^T on v_mfma_f32_16x16x32: lane (g = l/16, c = l%16) loads 8 head dims of key c, and
+//    ends up with the scores of query c for the keys 4g+r of each 16-key block;
+//  * O^T += V^T P^T in fp32 on v_mfma_f32_16x16x4: k slot g of step r is key 4g+r, so P is the
+//    score register r as it stands, and row m of V^T stands for the D/16 head dims from
+//    m*D/16 on, which are one contiguous load of the lane, one MFMA per dim.  P and V enter in
+//    fp32, exactly, so every V value has its IEEE result without a tile exponent;
+//  * the four waves' (m, l, O) meet in LDS; with the keys in one chunk the workgroup writes O / l,
+//    otherwise its fp32 state, and attention_short_merge combines the chunks.
+// Bound by HBM: the fp32 MFMAs take 2048 cycles per wave and 32 keys of head dim 128 (16 KB),
+// about twice the chip's HBM rate.  bf16, 512 heads x 3000 keys, one query: 312 us with the
+// kernels above, 128 us here (6.1 TB/s); K and V are loaded non-temporally (133 us without).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kShortBM = 16, kShortTK = 32, kShortWaves = 4;
+constexpr int kShortNt = 2;              // buffer loads of K and V: non-temporal
+
+template <typename T>
+struct AttnIn16;
+template <>
+struct AttnIn16<__bf16> {
+  __device__ static __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <>
+struct AttnIn16<_Float16> {
+  __device__ static __forceinline__ f32x4 mfma(f16x8 a, f16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+};
+
+// `chunks` key chunks of `per` 32-key tiles each.  Workgroups with the same chunk of the same
+// head (their query blocks differ) sit on one XCD (id % 8), so they share its L2.
+template <typename T, int D, bool CAUSAL>
+__device__ __forceinline__ void attention_short(const T* __restrict__ q, const T* __restrict__ k,
+                                                const T* __restrict__ v, T* __restrict__ o,
+                                                float* __restrict__ lse, float* __restrict__ po,
+                                                float* __restrict__ pml, int batch, int heads,
+                                                int sq, int sk, int chunks, int per, i64 qsb,
+                                                i64 qsh, i64 qss, i64 ksb, i64 ksh, i64 kss,
+                                                i64 vsb, i64 vsh, i64 vss, float scale_log2) {
+  typedef AttnIn<T> In;
+  typedef typename In::vec8 vec8;
+  constexpr int NB = kShortTK / 16;      // 16-key blocks of a tile
+  constexpr int KS = D / 32;             // MFMA k-steps of S^T
+  constexpr int DPL = D / 16;            // head dims per lane of a V row (and MFMAs per V step)
+  constexpr int W = kShortWaves, PAD = 4;
+  __shared__ __attribute__((aligned(16))) float so[W][kShortBM][D + PAD];
+  __shared__ float sm[W][kShortBM], sl[W][kShortBM];
+
+  const int nqb = (sq + kShortBM - 1) / kShortBM, bh_count = batch * heads;
+  const int slot = blockIdx.x >> 3;
+  const int unit = (slot / nqb) * 8 + (blockIdx.x & 7), q0 = (slot % nqb) * kShortBM;
+  if (unit >= bh_count * chunks) return;
+  const int chunk = unit / bh_count, bh = unit % bh_count;
+  const int b = bh / heads, h = bh % heads;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int my_q = q0 + c;
+  const T* kp = k + b * ksb + h * ksh;
+  const T* vp = v + b * vsb + h * vsh;
+
+  vec8 qreg[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    if (my_q < sq) qreg[s] = *(const vec8*)(q + b * qsb + h * qsh + my_q * qss + 32 * s + 8 * g);
+    else qreg[s] = vec8{};
+  }
+  const int kend = CAUSAL ? min(sk, q0 + kShortBM) : sk;
+  const int t_end = min((kend + kShortTK - 1) / kShortTK, (chunk + 1) * per);
+
+  // Byte offsets inside a tile; rows past the last key are sent out of the descriptor's range
+  // and read as zero.
+  constexpr u32 kOut = 0x80000000u;
+  u32 koff[NB], voff[NB][4];
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+    koff[n] = (u32)((16 * n + c) * (int)kss * 2 + 16 * g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) voff[n][r] = (u32)((16 * n + 4 * g + r) * (int)vss * 2 + c * DPL * 2);
+  }
+  auto tile_rsrc = [&](const T* base, i64 stride, int t) {
+    const int k0 = t * kShortTK, rows = min(kShortTK, sk - k0);
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(base + (i64)k0 * stride), (short)0,
+                                             (int)(((i64)(rows - 1) * stride + D) * 2),
+                                             (int)kRawBufferWord3);
+  };
+  u32x4 kreg[NB][KS];
+  auto load_k = [&](int t) {
+    const auto rs = tile_rsrc(kp, kss, t);
+    const int rem = sk - t * kShortTK;
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      const u32 off = 16 * n + c < rem ? koff[n] : kOut;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) kreg[n][s] = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 64 * s, 0, kShortNt);
+    }
+  };
+
+  f32x4 oacc[DPL];
+#pragma unroll
+  for (int j = 0; j < DPL; ++j) oacc[j] = f32x4{};
+  float m = -kInf, l = 0.0f;
+  int t = chunk * per + wave;
+  if (t < t_end) load_k(t);
+  for (; t < t_end; t += W) {
+    // ---- V of this tile: in flight through S and the softmax
+    constexpr int VW = DPL / 2;          // 32-bit words per lane and row
+    u32 vreg[NB][4][VW];
+    {
+      const auto rs = tile_rsrc(vp, vss, t);
+      const int rem = sk - t * kShortTK;
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const u32 off = 16 * n + 4 * g + r < rem ? voff[n][r] : kOut;
+          if constexpr (VW == 2) {
+            const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, kShortNt);
+            vreg[n][r][0] = w.x;
+            vreg[n][r][1] = w.y;
+          } else {
+#pragma unroll
+            for (int i = 0; i < VW / 4; ++i) {
+              const u32x4 w = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 * i, 0, kShortNt);
+              vreg[n][r][4 * i] = w.x;
+              vreg[n][r][4 * i + 1] = w.y;
+              vreg[n][r][4 * i + 2] = w.z;
+              vreg[n][r][4 * i + 3] = w.w;
+            }
+          }
+        }
+    }
+    // ---- S^T
+    f32x4 s[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      s[n] = f32x4{};
+#pragma unroll
+      for (int i = 0; i < KS; ++i) s[n] = AttnIn16<T>::mfma(__builtin_bit_cast(vec8, kreg[n][i]), qreg[i], s[n]);
+    }
+    const int k0 = t * kShortTK;
+    if (t + W < t_end) load_k(t + W);
+    if (k0 + kShortTK > sk || (CAUSAL && k0 + kShortTK - 1 > q0)) {
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = k0 + 16 * n + 4 * g + r;
+          if (key >= sk || (CAUSAL && key > my_q)) s[n][r] = -kInf;
+        }
+    }
+    float tmax = -kInf;
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tmax = __builtin_fmaxf(tmax, s[n][r]);
+    tmax = pair_max<32>(pair_max<16>(tmax)) * scale_log2;
+    const float m_new = __builtin_fmaxf(m, tmax);
+    if (__builtin_amdgcn_ballot_w64(m_new > m) != 0) {
+      const float alpha = m == -kInf ? 0.0f : __builtin_amdgcn_exp2f(m - m_new);
+      l *= alpha;
+#pragma unroll
+      for (int j = 0; j < DPL; ++j) oacc[j] *= alpha;
+      m = m_new;
+    }
+    const float shift = m == -kInf ? 0.0f : m;
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[n][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[n][r], scale_log2, -shift));
+        l += s[n][r];
+      }
+    // ---- O^T += V^T P^T
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int i = 0; i < VW; ++i) {
+          const u32 w = vreg[n][r][i];
+          oacc[2 * i] = __builtin_amdgcn_mfma_f32_16x16x4f32(In::lo(w), s[n][r], oacc[2 * i], 0, 0, 0);
+          oacc[2 * i + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(In::hi(w), s[n][r], oacc[2 * i + 1], 0, 0, 0);
+        }
+  }
+  // ---- the waves' states meet: row q of wave w is so[w][q], (m, l) in sm, sl
+  l = pair_sum<32>(pair_sum<16>(l));
+  if (g == 0) {
+    sm[wave][c] = m;
+    sl[wave][c] = l;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int j = 0; j < DPL; j += 4)
+      *(f32x4*)&so[wave][c][DPL * (4 * g + r) + j] =
+          f32x4{oacc[j][r], oacc[j + 1][r], oacc[j + 2][r], oacc[j + 3][r]};
+  __syncthreads();
+  constexpr int QUADS = kShortBM * D / 4;
+#pragma unroll
+  for (int e = tid; e < QUADS; e += 64 * W) {
+    const int row = e / (D / 4), d = (e % (D / 4)) * 4;
+    if (q0 + row >= sq) continue;
+    float mm = -kInf;
+#pragma unroll
+    for (int w = 0; w < W; ++w) mm = __builtin_fmaxf(mm, sm[w][row]);
+    float ll = 0.0f;
+    f32x4 acc = f32x4{};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float f = sm[w][row] == -kInf ? 0.0f : __builtin_amdgcn_exp2f(sm[w][row] - mm);
+      ll += sl[w][row] * f;
+      acc += *(const f32x4*)&so[w][row][d] * f;
+    }
+    const i64 out_row = (i64)bh * sq + q0 + row;
+    if (chunks == 1) {
+      const float inv = 1.0f / ll;
+      u32x2 w;
+      w.x = In::pack2(acc[0] * inv, acc[1] * inv);
+      w.y = In::pack2(acc[2] * inv, acc[3] * inv);
+      *(u32x2*)(o + out_row * D + d) = w;
+      if (lse != nullptr && d == 0) lse[out_row] = (mm + __builtin_log2f(ll)) * 0.6931471805599453f;
+    } else {
+      const i64 part = (i64)chunk * bh_count * sq + out_row;
+      *(f32x4*)(po + part * D + d) = acc;
+      if (d == 0) {
+        pml[2 * part] = mm;
+        pml[2 * part + 1] = ll;
+      }
+    }
+  }
+}
+
+// The chunks' states of one query row combined by one workgroup: D/4 lanes per chunk, the
+// workgroup's lane groups taking the chunks in turn and meeting in LDS.
+template <typename T, int D>
+__device__ __forceinline__ void attention_short_merge(const float* __restrict__ po,
+                                                      const float* __restrict__ pml,
+                                                      T* __restrict__ o, float* __restrict__ lse,
+                                                      i64 rows, int chunks) {
+  typedef AttnIn<T> In;
+  constexpr int LANES = D / 4, G = 256 / LANES;
+  __shared__ __attribute__((aligned(16))) float so[G][D];
+  __shared__ float sm[G], sl[G];
+  const i64 row = blockIdx.x;
+  const int grp = threadIdx.x / LANES, d = (threadIdx.x % LANES) * 4;
+  float mm = -kInf, ll = 0.0f;
+  f32x4 acc = f32x4{};
+  auto add = [&](float m2, float l2, const f32x4& a2) {
+    const float mn = __builtin_fmaxf(mm, m2);
+    const float f0 = mm == -kInf ? 0.0f : __builtin_amdgcn_exp2f(mm - mn);
+    const float f1 = m2 == -kInf ? 0.0f : __builtin_amdgcn_exp2f(m2 - mn);
+    ll = ll * f0 + l2 * f1;
+    acc = acc * f0 + a2 * f1;
+    mm = mn;
+  };
+  constexpr int PRE = 4;                 // chunks in flight per lane
+  for (int c0 = grp; c0 < chunks; c0 += PRE * G) {
+    float pm[PRE], pl[PRE];
+    f32x4 pa[PRE];
+#pragma unroll
+    for (int i = 0; i < PRE; ++i) {
+      if (c0 + i * G >= chunks) break;
+      const i64 part = (i64)(c0 + i * G) * rows + row;
+      pm[i] = pml[2 * part];
+      pl[i] = pml[2 * part + 1];
+      pa[i] = *(const f32x4*)(po + part * D + d);
+    }
+#pragma unroll
+    for (int i = 0; i < PRE; ++i)
+      if (c0 + i * G < chunks) add(pm[i], pl[i], pa[i]);
+  }
+  *(f32x4*)&so[grp][d] = acc;
+  if (d == 0) {
+    sm[grp] = mm;
+    sl[grp] = ll;
+  }
+  __syncthreads();
+  if (grp != 0) return;
+  const int live = min(G, chunks);
+  for (int j = 1; j < live; ++j) add(sm[j], sl[j], *(const f32x4*)&so[j][d]);
+  const float inv = 1.0f / ll;
+  u32x2 w;
+  w.x = In::pack2(acc[0] * inv, acc[1] * inv);
+  w.y = In::pack2(acc[2] * inv, acc[3] * inv);
+  *(u32x2*)(o + row * D + d) = w;
+  if (lse != nullptr && d == 0) lse[row] = (mm + __builtin_log2f(ll)) * 0.6931471805599453f;
+}
+
 #ifdef NEP_ATTN_W64_ASM
 typedef u32 u32x8 __attribute__((ext_vector_type(8)));
 typedef u32 u32x32 __attribute__((ext_vector_type(32)));

@@ -11,6 +11,9 @@ fp16), unit stride on D; other strides are honoured (rows must be 16-byte aligne
 contiguous).  Output is a fresh contiguous [B, H, Sq, D] tensor of the input dtype;
 `return_lse` adds the fp32 [B, H, Sq] natural-log logsumexp of the scaled, masked scores.
 
+Calls of at most 16 queries (decoding) run kernels of their own, which split a head's keys over
+workgroups and take P and V in fp32 (see SHORT_MAX_SQ); what follows is about the others.
+
 Every input has a result; nothing is refused at run time and no device-side assert is used.
 The MFMA path feeds V to the P.V product as fp16 images scaled per 64-key tile by a power of
 two (exact for |v| < 2^28 in a tile, see V_EXPONENT_MAX).  A workgroup whose keys include a
@@ -20,13 +23,16 @@ a non-finite V value become non-finite.
 """
 from __future__ import annotations
 
+import functools
 import math
 import threading
 
 from neptune_codegen import hip
-from neptune_codegen.emitters import (ATTN_HEAD_DIMS, BASE_OPTIONS, attention_block_m,
+from neptune_codegen.emitters import (ATTN_HEAD_DIMS, ATTN_SHORT_BLOCK_M, ATTN_SHORT_TILE,
+                                      ATTN_SHORT_WAVES, BASE_OPTIONS, attention_block_m,
                                       attention_fold_threads, attention_kernel_name,
-                                      attention_pack_kernel_name, attention_w64,
+                                      attention_pack_kernel_name, attention_short_kernel_names,
+                                      attention_w64, emit_attention_short_source,
                                       emit_attention_source)
 
 _PROGRAMS: dict = {}
@@ -74,6 +80,56 @@ def _program(head_dim: int, causal: bool, dtype="bfloat16", w64: bool | None = N
         return prog
 
 
+def _short_program(head_dim: int, causal: bool, dtype) -> hip.Program:
+    key = ("short", head_dim, causal, str(dtype))
+    with _lock:
+        prog = _PROGRAMS.get(key)
+        if prog is None:
+            name = attention_short_kernel_names(head_dim, causal, dtype)[0]
+            prog = hip.Program(emit_attention_short_source(head_dim, causal, dtype),
+                               f"{name}.hip", BASE_OPTIONS)
+            _PROGRAMS[key] = prog
+        return prog
+
+
+# Calls of at most 16 queries run the short-query kernels: K and V are read once, by as many
+# workgroups as the keys allow, where the others give a head one workgroup with 240 idle query
+# slots and stage V twice.  Measured on MI355X (graph replays, cold; the kernels above -> these):
+# bf16 B*H=512 sq=1 sk=3000 d=128 312 -> 128 us (6.1 TB/s of K and V); B*H=32 sq=1 sk=32768 784 ->
+# 87; B*H=256 sq=8 sk=4096 201 -> 95; fp16 B*H=64 sq=16 sk=5000 d=64 106 -> 25; B*H=8 sq=4 sk=8192
+# d=256 383 -> 23; B*H=8 sq=1 sk=512 20 -> 8.5.
+SHORT_MAX_SQ = 16
+# Chunks of a head's keys: a workgroup's 4 waves pass a 32-key tile in about 0.6 us when each CU
+# has one, and a split costs a second launch and its chunks' states (3 us + 0.05 us a chunk).
+# `short_chunks` takes the cheapest count; against a sweep of 1 to 64 chunks over fourteen shapes
+# it is within 4% of the best but for two (d=64, 4 chunks 25 us for 8 at 20.6; sq=1 sk=8192 B*H=1
+# 12.4 for 10.7).  At B*H=32 sk=32768 1 chunk takes 556 us, 8 take 87 and 64 take 94.
+SHORT_MAX_CHUNKS = 64
+SHORT_TILE_US, SHORT_MERGE_US, SHORT_CHUNK_US = 0.6, 3.0, 0.05
+CUS = 256
+
+
+def use_short(head_dim: int, causal: bool, sq: int, sk: int) -> bool:
+    """Whether a call of this shape runs the short-query kernels (attention_short)."""
+    return sq <= SHORT_MAX_SQ
+
+
+@functools.lru_cache(maxsize=4096)
+def short_chunks(units: int, sk: int) -> tuple[int, int]:
+    """(chunks, tiles per chunk) of a head's keys for `units` (head, query block) pairs."""
+    tiles = -(-sk // ATTN_SHORT_TILE)
+
+    def cost(chunks):
+        rounds = -(-units * chunks // CUS)
+        return (rounds * -(-tiles // chunks) * SHORT_TILE_US
+                + (SHORT_MERGE_US + chunks * SHORT_CHUNK_US if chunks > 1 else 0.0))
+
+    most = max(1, min(SHORT_MAX_CHUNKS, tiles // ATTN_SHORT_WAVES))
+    chunks = min(range(1, most + 1), key=cost)
+    per = -(-tiles // chunks)
+    return -(-tiles // per), per
+
+
 def validate_attention_inputs(q, k, v, *, metadata: bool = False):
     import torch
 
@@ -107,7 +163,10 @@ def _kernel_ready(t):
 def run_attention(q, k, v, *, scale: float | None = None, causal: bool = True,
                   return_lse: bool = False):
     """Attention fold on the current stream; see the module docstring for the contract."""
-    out, lse, _ = launch_attention(q, k, v, scale=scale, causal=causal, return_lse=return_lse)
+    if q.ndim == 4 and use_short(q.shape[3], causal, q.shape[2], k.shape[2]):
+        out, lse = _launch_short(q, k, v, scale, causal, return_lse)
+    else:
+        out, lse, _ = launch_attention(q, k, v, scale=scale, causal=causal, return_lse=return_lse)
     return (out, lse) if return_lse else out
 
 
@@ -119,24 +178,75 @@ def launch_attention(q, k, v, *, scale: float | None = None, causal: bool = True
     return _launch(q, k, v, scale, causal, return_lse, V_EXPONENT_MAX)
 
 
+def _outputs(q, k, v, scale, return_lse):
+    """(out, lse or None, scale, whether nothing is to be launched) after validation."""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensor
+
+    metadata = isinstance(q, FakeTensor) or q.device.type == "meta"
+    shape = validate_attention_inputs(q, k, v, metadata=metadata)
+    out = torch.empty(shape, dtype=q.dtype, device=q.device)
+    lse = torch.empty(shape[:3], dtype=torch.float32, device=q.device) if return_lse else None
+    if metadata or out.numel() == 0:
+        return out, lse, scale, True
+    scale = 1.0 / math.sqrt(shape[3]) if scale is None else float(scale)
+    if not math.isfinite(scale) or scale <= 0:
+        raise ValueError("attention scale must be finite and positive")
+    return out, lse, scale, False
+
+
+def _launch_short(q, k, v, scale, causal, return_lse):
+    """(out, lse or None) through the short-query kernels."""
+    import torch
+
+    out, lse, scale, done = _outputs(q, k, v, scale, return_lse)
+    if done:
+        return out, lse
+    B, H, Sq, D = q.shape
+    q, k, v = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)
+    if k.stride(2) >= K_ROW_STRIDE_MAX:
+        k = k.contiguous()
+    if v.stride(2) >= K_ROW_STRIDE_MAX:
+        v = v.contiguous()
+    device = q.device.index if q.device.index is not None else torch.cuda.current_device()
+    Sk = k.shape[2]
+    nqb = -(-Sq // ATTN_SHORT_BLOCK_M)
+    chunks, per = short_chunks(B * H * nqb, min(Sk, Sq) if causal else Sk)
+    rows = B * H * Sq
+    po = pml = 0
+    if chunks > 1:   # fp32 O, then (max, sum), of every chunk and query
+        part = torch.empty(chunks * rows * (D + 2), dtype=torch.float32, device=q.device)
+        po = part.data_ptr()
+        pml = po + 4 * chunks * rows * D
+    names = attention_short_kernel_names(D, causal, q.dtype)
+    prog = _short_program(D, causal, q.dtype)
+    fold = prog.kernel(names[0], (hip.PTR,) * 7 + (hip.I32,) * 6 + (hip.I64,) * 9 + (hip.F32,),
+                       64 * ATTN_SHORT_WAVES, device)
+    stream = hip.current_stream(q.device)
+    lse_ptr = lse.data_ptr() if lse is not None else 0
+    grid = -(-B * H * chunks // 8) * nqb * 8
+    fold.launch((grid,), (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse_ptr, po, pml,
+                          B, H, Sq, Sk, chunks, per, q.stride(0), q.stride(1), q.stride(2),
+                          k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1),
+                          v.stride(2), scale * LOG2E), stream)
+    if chunks > 1:
+        merge = prog.kernel(names[1], (hip.PTR,) * 4 + (hip.I64, hip.I32), 256, device)
+        merge.launch((rows,), (po, pml, out.data_ptr(), lse_ptr, rows, chunks),
+                     stream)
+    return out, lse
+
+
 def _launch(q, k, v, scale, causal, return_lse, e_max: int, w64: bool | None = None):
     """The launches with the exact path's threshold as a parameter: e_max = -1 sends every
     query block through the exact fp32 path (the tests compare the two paths with it).
     `w64=False` runs the compiler-scheduled 32-queries-per-wave kernel at head dim 128 instead
     of the instruction-scheduled one (the tests compare the two bit for bit)."""
     import torch
-    from torch._subclasses.fake_tensor import FakeTensor
 
-    metadata = isinstance(q, FakeTensor) or q.device.type == "meta"
-    shape = validate_attention_inputs(q, k, v, metadata=metadata)
-    B, H, Sq, D = shape
-    out = torch.empty(shape, dtype=q.dtype, device=q.device)
-    lse = torch.empty((B, H, Sq), dtype=torch.float32, device=q.device) if return_lse else None
-    if metadata or out.numel() == 0:
+    out, lse, scale, done = _outputs(q, k, v, scale, return_lse)
+    if done:
         return out, lse, None
-    scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
-    if not math.isfinite(scale) or scale <= 0:
-        raise ValueError("attention scale must be finite and positive")
+    B, H, Sq, D = q.shape
     if w64 is None:
         w64 = use_w64(D, causal, Sq, k.shape[2])
     q, k, v = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)

@@ -632,3 +632,37 @@ def attention_kernel_name(head_dim: int, causal: bool, dtype="bfloat16", w64: bo
 def attention_pack_kernel_name(head_dim: int, dtype="bfloat16") -> str:
     tag, _ = _attn_dtype(dtype)
     return f"attention_vt_pack_{tag}_d{head_dim}"
+
+
+# Short query ranges: 16 queries per workgroup, the head's keys split over workgroups in tiles of 32.
+ATTN_SHORT_BLOCK_M, ATTN_SHORT_TILE, ATTN_SHORT_WAVES = 16, 32, 4
+
+
+def attention_short_kernel_names(head_dim: int, causal: bool, dtype="bfloat16") -> tuple[str, str]:
+    """(fold, merge) symbols of the short-query kernels."""
+    tag, _ = _attn_dtype(dtype)
+    return (f"attention_short_{tag}_d{head_dim}_{'causal' if causal else 'full'}",
+            f"attention_short_merge_{tag}_d{head_dim}")
+
+
+def emit_attention_short_source(head_dim: int, causal: bool, dtype="bfloat16") -> str:
+    """hiprtc unit of attention for few queries (nep_attention.h attention_short)."""
+    if head_dim not in ATTN_HEAD_DIMS:
+        raise NotImplementedError("attention fold supports head_dim 64, 128 and 256")
+    _, ctype = _attn_dtype(dtype)
+    fold, merge = attention_short_kernel_names(head_dim, causal, dtype)
+    return "\n".join([
+        "// AUTO-GENERATED by neptune_codegen (HIP emitter) -- do not edit.\n"
+        f"// attention of few queries: head_dim={head_dim}, causal={causal}, {ctype} inputs\n",
+        kernel_header("nep_device.h", "nep_attention.h"),
+        f'extern "C" __global__ void __launch_bounds__({64 * ATTN_SHORT_WAVES}) {fold}(const void* q, '
+        "const void* k, const void* v, void* o, float* lse, float* po, float* pml, int batch, "
+        "int heads, int sq, int sk, int chunks, int per, long long qsb, long long qsh, long long qss, "
+        "long long ksb, long long ksh, long long kss, long long vsb, long long vsh, long long vss, "
+        "float scale_log2) {\n"
+        f"  nep::attention_short<{ctype}, {head_dim}, {'true' if causal else 'false'}>((const {ctype}*)q, "
+        f"(const {ctype}*)k, (const {ctype}*)v, ({ctype}*)o, lse, po, pml, batch, heads, sq, sk, chunks, "
+        "per, qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, scale_log2);\n}\n",
+        f'extern "C" __global__ void __launch_bounds__(256) {merge}(const float* po, const float* pml, '
+        "void* o, float* lse, long long rows, int chunks) {\n"
+        f"  nep::attention_short_merge<{ctype}, {head_dim}>(po, pml, ({ctype}*)o, lse, rows, chunks);\n}}\n"])
