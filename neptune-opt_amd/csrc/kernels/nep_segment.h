@@ -11,9 +11,9 @@
 // 24 >= 2*11+2 significand bits, so double rounding is innocuous); the vector path therefore
 // adds packed halves (v_pk_add_f16).  bf16 and fp32 add in fp32 and round explicitly.
 //
-// Mapping: vector path -- LPS lanes per segment, each lane owns one 16-byte channel vector,
-// 64/LPS segments per wavefront, UNR token rows prefetched per step; generic path -- one lane
-// per channel, 64-channel tiles, any strides.
+// Mapping: vector path -- one lane per (segment, chunk of 1, 2 or 4 words of channels), several
+// token rows in flight per lane; generic path -- one lane per channel, 64-channel tiles, any
+// strides.
 //
 // Descriptor validation (the reference's device-side span asserts, torch_op.py:378-386) is
 // fused into the fold: with `status` non-null, a lane whose span is malformed, or the last
@@ -24,66 +24,96 @@
 
 namespace nep {
 
-template <class St>
+// Ordered sums of the elements of W 32-bit words.
+template <class St, int W>
 struct SegAcc;
 
-template <>
-struct SegAcc<F32> {
-  float a[4];
+template <int W>
+struct SegAcc<F32, W> {
+  float a[W];
   __device__ __forceinline__ void init(float v) {
-    a[0] = a[1] = a[2] = a[3] = v;
-  }
-  __device__ __forceinline__ void add(const u32x4& w) {
-    a[0] = a[0] + as_f32(w.x);
-    a[1] = a[1] + as_f32(w.y);
-    a[2] = a[2] + as_f32(w.z);
-    a[3] = a[3] + as_f32(w.w);
-  }
-  __device__ __forceinline__ void get(float* o) const {
-    for (int j = 0; j < 4; ++j) o[j] = a[j];
-  }
-};
-
-template <>
-struct SegAcc<BF16> {
-  float a[8];
-  __device__ __forceinline__ void init(float v) {
-    for (int j = 0; j < 8; ++j) a[j] = v;
-  }
-  __device__ __forceinline__ void add(const u32x4& w) {
-    float v[8];
-    BF16::unpack(w, v);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) a[j] = BF16::round(a[j] + v[j]);
+    for (int j = 0; j < W; ++j) a[j] = v;
+  }
+  template <class V>
+  __device__ __forceinline__ void add(const V& w) {
+#pragma unroll
+    for (int j = 0; j < W; ++j) a[j] = a[j] + as_f32(w[j]);
   }
   __device__ __forceinline__ void get(float* o) const {
-    for (int j = 0; j < 8; ++j) o[j] = a[j];
+#pragma unroll
+    for (int j = 0; j < W; ++j) o[j] = a[j];
   }
+  __device__ static __forceinline__ u32 pack(const float* r) { return as_u32(r[0]); }
 };
 
-template <>
-struct SegAcc<F16> {
-  half2_t a[4];
+template <int W>
+struct SegAcc<BF16, W> {
+  u32 a[W];    // packed pairs, rounded after every token
+  __device__ __forceinline__ void init(float v) {
+#pragma unroll
+    for (int j = 0; j < W; ++j) a[j] = bf16x2_rne(v, v);
+  }
+  template <class V>
+  __device__ __forceinline__ void add(const V& w) {
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+      a[j] = bf16x2_rne(as_f32(a[j] << 16) + as_f32(w[j] << 16),
+                        as_f32(a[j] & 0xffff0000u) + as_f32(w[j] & 0xffff0000u));
+  }
+  __device__ __forceinline__ void get(float* o) const {
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+      o[2 * j] = as_f32(a[j] << 16);
+      o[2 * j + 1] = as_f32(a[j] & 0xffff0000u);
+    }
+  }
+  __device__ static __forceinline__ u32 pack(const float* r) { return bf16x2_rne(r[0], r[1]); }
+};
+
+template <int W>
+struct SegAcc<F16, W> {
+  half2_t a[W];
   __device__ __forceinline__ void init(float v) {
     half2_t h;
     h.x = (_Float16)v;
     h.y = h.x;
-    a[0] = a[1] = a[2] = a[3] = h;
+#pragma unroll
+    for (int j = 0; j < W; ++j) a[j] = h;
   }
-  __device__ __forceinline__ void add(const u32x4& w) {
-    a[0] = a[0] + as_half2(w.x);
-    a[1] = a[1] + as_half2(w.y);
-    a[2] = a[2] + as_half2(w.z);
-    a[3] = a[3] + as_half2(w.w);
+  template <class V>
+  __device__ __forceinline__ void add(const V& w) {
+#pragma unroll
+    for (int j = 0; j < W; ++j) a[j] = a[j] + as_half2(w[j]);
   }
   __device__ __forceinline__ void get(float* o) const {
-    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
       o[2 * j] = (float)a[j].x;
       o[2 * j + 1] = (float)a[j].y;
     }
   }
+  __device__ static __forceinline__ u32 pack(const float* r) {
+    half2_t h;
+    h.x = (_Float16)r[0];
+    h.y = (_Float16)r[1];
+    return half2_bits(h);
+  }
 };
 
+// W consecutive 32-bit words, non-temporally; ALIGNED: the address is a multiple of 4*W bytes,
+// otherwise only of the element size.
+template <int W, bool ALIGNED>
+struct Words {
+  typedef u32 V __attribute__((ext_vector_type(W)));
+  typedef V VA __attribute__((aligned(ALIGNED ? 4 * W : 2)));
+  __device__ static __forceinline__ V load(const void* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const VA*>(p));
+  }
+  __device__ static __forceinline__ void store(void* p, const V& v) {
+    __builtin_nontemporal_store(v, reinterpret_cast<VA*>(p));
+  }
+};
 template <class SpanT>
 __device__ __forceinline__ bool read_span(const SpanT* spans, i64 stride_span, i64 seg,
                                           i64 nrows, i64* start, i64* end) {
@@ -111,41 +141,72 @@ __device__ __forceinline__ float segment_readout(float acc, bool valid, i64 star
   return valid ? r : __builtin_nanf("");
 }
 
-// Vector path: channels == LPS * VEC, data rows 16-byte aligned with unit channel stride.
-template <class St, class SpanT, bool MEAN, bool INIT_NONE, int LPS, int UNR, int WG>
+// Vector path (unit channel stride, at least one lane's worth of channels): lane L of the launch
+// owns the W-word channel chunk L % chunks of segment L / chunks.  When the chunks do not divide
+// the channels the last one ends at the last channel, overlapping its neighbour: both compute
+// and store the same values for the channels they share.  UNR token rows are loaded per step.
+// NEAR: the data spans less than 4 GiB, so a load is a uniform row base plus the lane's 32-bit
+// offset, without address arithmetic of its own.
+// Bound by HBM with many segments, by the latency of a segment's steps with few.  Measured on
+// MI355X, cold, kernel alone, against 16-byte chunks for power-of-two lane counts and one element
+// per lane for the rest: bf16 5000 segments x 26 tokens x 768 channels 117 -> 38 us, 3000 x 40 x
+// 300 46 -> 18, fp16 16 x 400 x 1024 106 -> 14, 64 x 400 x 128 42 -> 13 (whole steps without
+// per-row bounds and 64-bit addresses: 21 of those 42).
+template <class St, class SpanT, bool MEAN, bool INIT_NONE, int W, int UNR, bool ALIGNED,
+          bool NEAR, int WG>
 __device__ __forceinline__ void segment_vector(const typename St::T* __restrict__ data,
                                                const SpanT* __restrict__ spans,
                                                typename St::T* __restrict__ out, i64 nrows,
                                                i64 channels, i64 nsegments, i64 stride_row,
                                                i64 stride_span, float initial, int* status,
                                                i64 cover) {
-  constexpr int VEC = St::kVec;
-  constexpr int SPW = WG / LPS;  // segments per workgroup
-  const int l = threadIdx.x % LPS;
-  const i64 seg = (i64)blockIdx.x * SPW + threadIdx.x / LPS;
+  typedef Words<W, ALIGNED> IO;
+  constexpr int SIZE = (int)sizeof(typename St::T);
+  constexpr int VE = 4 * W / SIZE;   // channels per lane
+  const u32 chunks = (u32)((channels + VE - 1) / VE);
+  const u32 id = blockIdx.x * (u32)WG + threadIdx.x;        // nsegments * chunks < 2^32 (host)
+  const i64 seg = id / chunks;
   if (seg >= nsegments) return;
+  i64 c0 = (i64)(id % chunks) * VE;
+  if constexpr (!ALIGNED) c0 = c0 + VE <= channels ? c0 : channels - VE;
   i64 start, end;
   const bool valid = read_span(spans, stride_span, seg, nrows, &start, &end);
   segment_check(status, valid, seg, nsegments, end, cover);
-  SegAcc<St> acc;
+  SegAcc<St, W> acc;
   acc.init(St::round(initial));
   if (valid) {
-    const typename St::T* col = data + (i64)l * VEC;
-    for (i64 t = start; t < end; t += UNR) {
-      u32x4 w[UNR];
+    const char* base = (const char*)data;
+    const i64 pitch = stride_row * SIZE;
+    typedef __typeof__(sizeof(0)) word;
+    const word at = (word)(start * pitch + c0 * SIZE);
+    u32 near = (u32)at;
+    const char* far = base + at;
+    auto row = [&](int i) { return NEAR ? base + i * pitch + near : far + i * pitch; };
+    i64 left = end - start;
+    typename IO::V w[UNR];
+    for (; left >= UNR; left -= UNR) {
 #pragma unroll
-      for (int i = 0; i < UNR; ++i)
-        if (t + i < end) w[i] = load16(col + (t + i) * stride_row);
+      for (int i = 0; i < UNR; ++i) w[i] = IO::load(row(i));
 #pragma unroll
-      for (int i = 0; i < UNR; ++i)
-        if (t + i < end) acc.add(w[i]);
+      for (int i = 0; i < UNR; ++i) acc.add(w[i]);
+      near += (u32)(UNR * pitch);
+      far += UNR * pitch;
     }
+#pragma unroll
+    for (int i = 0; i < UNR - 1; ++i)
+      if (i < left) w[i] = IO::load(row(i));
+#pragma unroll
+    for (int i = 0; i < UNR - 1; ++i)
+      if (i < left) acc.add(w[i]);
   }
-  float a[VEC], r[VEC];
+  float a[VE];
   acc.get(a);
 #pragma unroll
-  for (int j = 0; j < VEC; ++j) r[j] = segment_readout<St, MEAN, INIT_NONE>(a[j], valid, start, end);
-  store16(out + seg * channels + (i64)l * VEC, St::pack(r));
+  for (int j = 0; j < VE; ++j) a[j] = segment_readout<St, MEAN, INIT_NONE>(a[j], valid, start, end);
+  typename IO::V r;
+#pragma unroll
+  for (int j = 0; j < W; ++j) r[j] = SegAcc<St, W>::pack(a + j * (VE / W));
+  IO::store(out + seg * channels + c0, r);
 }
 
 // Generic path: grid (nsegments, ceil(channels / 64)), one lane per channel.

@@ -454,12 +454,15 @@ class SegmentVariant:
     dtype: str
     span_dtype: str     # "int32" | "int64"
     vector: bool
-    lps: int            # lanes per segment (vector path); 64 for the generic path
-    unroll: int = 8
+    words: int          # 32-bit words of channels per lane (vector path; 0 otherwise)
+    unroll: int = 4     # token rows loaded per step
+    aligned: bool = True    # rows and chunks are aligned to the lane's words
+    near: bool = True       # the data spans less than 4 GiB
 
     def tag(self) -> str:
         sd = "i32" if self.span_dtype == "int32" else "i64"
-        return f"{dtype_tag(self.dtype)[0]}_{sd}_{'v' if self.vector else 's'}{self.lps}u{self.unroll}"
+        kind = ("v" if self.aligned else "r") + ("" if self.near else "f") if self.vector else "s"
+        return f"{dtype_tag(self.dtype)[0]}_{sd}_{kind}{self.words}u{self.unroll}"
 
 
 def initial_bits(initial: float | None) -> tuple[int, float]:
@@ -486,7 +489,7 @@ def emit_segment_source(name: str, *, initial=None, offsets=False, plan="serial"
     mean = "true" if name == "segment_mean" else "false"
     none = "true" if params["initial"] is None else "false"
     if variants is None:
-        variants = tuple(SegmentVariant(d, "int64", False, 64) for d in DTYPE_TAGS)
+        variants = tuple(SegmentVariant(d, "int64", False, 0) for d in DTYPE_TAGS)
     parts = [f"// AUTO-GENERATED by neptune_codegen (HIP emitter) -- do not edit.\n"
              f"// segment state=(sum,count); exact-real additive certificate only.\n"
              f"// Numeric contract: ordered per-token storage-dtype RTNE; no IEEE reassociation.\n"
@@ -500,7 +503,8 @@ def emit_segment_source(name: str, *, initial=None, offsets=False, plan="serial"
         span_t = "int" if var.span_dtype == "int32" else "long long"
         kname = f"{name}_{var.tag()}"
         if var.vector:
-            body = (f"nep::segment_vector<{st}, {span_t}, {mean}, {none}, {var.lps}, {var.unroll}, 256>("
+            body = (f"nep::segment_vector<{st}, {span_t}, {mean}, {none}, {var.words}, {var.unroll}, "
+                    f"{str(var.aligned).lower()}, {str(var.near).lower()}, 256>("
                     f"(const {st}::T*)data, (const {span_t}*)spans, ({st}::T*)out, nrows, channels, "
                     "nsegments, stride_row, stride_span, __builtin_bit_cast(float, kInitialBits), "
                     "status, cover);")

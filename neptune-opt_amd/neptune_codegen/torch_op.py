@@ -365,20 +365,38 @@ def _segment_spans(data, segments, *, offsets, unsafe):
 
 
 def _segment_variant(flat, spans, channels: int) -> SegmentVariant:
-    from neptune_codegen.autotune import vec_of
-
+    """Channel words per lane and token rows per step.  A lane's adds are ordered, so a segment's
+    rows are only in flight together, never split over lanes: with few (segment, chunk) lanes
+    narrow chunks put more of them to work, and with rows of whole 256-byte wavefronts (one
+    4-byte word per lane) a wavefront holds one segment and its lanes stop together; otherwise
+    wide chunks take the fewest instructions.  Measured on MI355X, cold, words/rows per step:
+    fp16 65536 segments x 20 tokens x 128 channels 1/16 56.8 us, 2/16 61.7, 4/16 58.9;
+    bf16 5000 x 26 x 768 37.6, 37.4, 39.9; fp32 50000 x 10 x 128 45.3, 46.3, 48.0;
+    bf16 20000 x 20 x 100 23.8, 20.9, 20.2; bf16 3000 x 40 x 300 19.6, 18.1, 17.8;
+    bf16 4096 x 16 x 64 6.4, 5.4, 8.5; bf16 300 x 200 x 512 17.4, 18.1, 24.3 (1/32 19.1);
+    fp16 16 x 400 x 1024 20.0, 22.2, 30.0 (1/32 14.4); fp16 64 x 400 x 128 17.2, 19.5, 29.3
+    (1/32 12.8); fp32 347 x 13 x 246 4.1, 4.4, 4.9."""
     dtype = str(flat.dtype).replace("torch.", "")
     span_dtype = str(spans.dtype).replace("torch.", "")
-    vec = vec_of(flat.dtype)
-    lanes = channels // vec if channels % vec == 0 else 0
-    vector = (lanes > 0 and lanes <= 64 and lanes & (lanes - 1) == 0
-              and (flat.stride(1) == 1 or channels == 1) and flat.stride(0) % vec == 0
-              and flat.data_ptr() % 16 == 0)
-    if vector:
-        # 16 tokens in flight per lane: cfg4 (Poisson(20) segments, 128 fp16 channels) 55.8 us
-        # against 58.6 us at 8 tokens and 57.3 us at 32, bit-identical results
-        return SegmentVariant(dtype, span_dtype, True, lanes, 16)
-    return SegmentVariant(dtype, span_dtype, False, 64, 4)
+    size = flat.element_size()
+    nseg, nrows = spans.shape[0] - 1, flat.shape[0]
+    waves = nseg * channels * size / 256     # of one 4-byte word per lane
+    words, unroll = 1, 16
+    if waves < 512 and nrows >= 64 * nseg:
+        unroll = 32
+    elif waves >= 2048 and channels * size % 256:
+        words = 2 if waves < 4096 else 4
+    while words > 1 and channels * size < 4 * words:
+        words //= 2
+    per_lane = 4 * words // size
+    chunks = -(-channels // per_lane)
+    if (channels < per_lane or (flat.stride(1) != 1 and channels > 1)
+            or nseg * chunks > (1 << 32) - 256):
+        return SegmentVariant(dtype, span_dtype, False, 0, 4)
+    aligned = (channels % per_lane == 0 and flat.stride(0) % per_lane == 0
+               and flat.data_ptr() % (4 * words) == 0)
+    near = (nrows * flat.stride(0) + channels) * size < 1 << 32
+    return SegmentVariant(dtype, span_dtype, True, words, unroll, aligned, near)
 
 
 DESCRIPTOR_MESSAGE = ("segment descriptor is invalid: lengths must be nonnegative, within data bounds "
@@ -530,7 +548,8 @@ def launch_segment_kernel(program, flat, spans, out, *, status=None, cover=-1):
     device = flat.device.index if flat.device.index is not None else torch.cuda.current_device()
     kernel = program.kernel(var, device)
     if var.vector:
-        grid = (max(1, -(-nseg // (256 // var.lps))),)
+        per_lane = 4 * var.words // flat.element_size()
+        grid = (max(1, -(-(nseg * -(-channels // per_lane)) // 256)),)
     else:
         grid = (nseg, -(-channels // 64))
     tail = (flat.shape[0], channels, nseg, flat.stride(0), flat.stride(1), spans.stride(0),
