@@ -50,11 +50,8 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// wave64s per fold workgroup (32 queries each): two per SIMD up to head dim 128; at head dim
-// 256 a wave's O^T and Q^T operands alone take 192 registers, so one wave per SIMD
-template <int D>
-constexpr int attn_waves() { return D <= 128 ? 8 : 4; }
 constexpr int kAttnBN = 64;            // keys per tile
 constexpr int kAttnThreads = 256;      // V^T pack workgroup: 4 wave64s
 constexpr float kRescaleSlack = 8.0f;  // base-2 headroom before the reference max moves
@@ -305,12 +302,16 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc, void* dst, in
 // throughout: a query's row is held by 4 adjacent lanes (D/4 head dims each); per key the
 // score is the group sum of their partial dot products, and (m, l, O) are moved to every new
 // maximum exactly (not lazily).  Masked keys contribute nothing, so only the rows that see a
-// non-finite V value turn non-finite, as IEEE arithmetic on the visible keys gives.
+// non-finite V value turn non-finite, as IEEE arithmetic on the visible keys gives.  Of the keys
+// [k_begin, k_end); with po0 the unnormalised state goes to the part's fp32 rows instead.
 template <typename T, int D, bool CAUSAL, int W, int BM = 32 * W>
 __device__ void attention_exact_rows(const T* __restrict__ qp, const T* __restrict__ kp,
                                      const T* __restrict__ vp, T* __restrict__ orow0,
                                      float* __restrict__ lse_row0, int sq, int sk, int q0,
-                                     i64 qss, i64 kss, i64 vss, float scale_log2) {
+                                     i64 qss, i64 kss, i64 vss, float scale_log2,
+                                     int k_begin = 0, int k_end = 0x7fffffff,
+                                     float* __restrict__ po0 = nullptr,
+                                     float* __restrict__ pml0 = nullptr) {
   typedef AttnIn<T> In;
   constexpr int DQ = D / 4;                    // head dims per lane
   constexpr int ROWS = W * 64 / 4;             // queries per round
@@ -332,10 +333,10 @@ __device__ void attention_exact_rows(const T* __restrict__ qp, const T* __restri
 #pragma unroll
     for (int d = 0; d < DQ; ++d) ov[d] = 0.0f;
     float m = -kInf, l = 0.0f;
-    const int kend = CAUSAL ? min(sk, r0 + ROWS) : sk;
+    const int kend = min(k_end, CAUSAL ? min(sk, r0 + ROWS) : sk);
     const int last = !active ? -1 : (CAUSAL ? min(my_q, sk - 1) : sk - 1);
 #pragma unroll 2
-    for (int j = 0; j < kend; ++j) {
+    for (int j = k_begin; j < kend; ++j) {
       const T* kr = kp + (i64)j * kss + c * DQ;
       const T* vr = vp + (i64)j * vss + c * DQ;
       u32x4 kw[DQ / 8], vw[DQ / 8];
@@ -373,7 +374,14 @@ __device__ void attention_exact_rows(const T* __restrict__ qp, const T* __restri
           }
       }
     }
-    if (active) {
+    if (active && po0 != nullptr) {
+#pragma unroll
+      for (int d = 0; d < DQ; ++d) po0[(i64)my_q * D + c * DQ + d] = ov[d];
+      if (c == 0) {
+        pml0[2 * (i64)my_q] = m;
+        pml0[2 * (i64)my_q + 1] = l;
+      }
+    } else if (active) {
       T* orow = orow0 + (i64)my_q * D + c * DQ;
 #pragma unroll
       for (int d8 = 0; d8 < DQ; d8 += 8) {
@@ -388,7 +396,14 @@ __device__ void attention_exact_rows(const T* __restrict__ qp, const T* __restri
   }
 }
 
-template <typename T, int D, bool CAUSAL>
+// kAttnWaves wave64s of 32 queries: 8 share each staged tile among most queries, 4 make twice the
+// workgroups where 8 leave CUs idle or uneven.
+// A head's keys may be split into `parts` of `per` tiles: each workgroup takes one part of one
+// query block, and a block that has more than one part leaves its unnormalised fp32 state
+// (O, m, l) for attention_parts_merge (causal blocks differ in their parts).  Both are for calls
+// whose time is their longest workgroup's: bf16 full, 36 heads x 100 queries x 4000 keys, d=128
+// 108 us with 8 waves, 92 with 4, 44 in 6 parts; causal, 8 heads x 4096 103, 84, 63.
+template <typename T, int D, bool CAUSAL, int kAttnWaves>
 __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* __restrict__ k,
                                               const u16* __restrict__ vt,
                                               const int* __restrict__ exps,
@@ -396,11 +411,11 @@ __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* 
                                               float* __restrict__ lse, int heads, int sq, int sk,
                                               i64 qsb, i64 qsh, i64 qss, i64 ksb, i64 ksh,
                                               i64 kss, i64 vsb, i64 vsh, i64 vss, int e_max,
-                                              float scale_log2) {
+                                              float scale_log2, float* __restrict__ po,
+                                              float* __restrict__ pml, int parts, int per) {
   static_assert(D == 64 || D == 128 || D == 256, "head dim must be 64, 128 or 256");
   typedef AttnIn<T> In;
   typedef typename In::vec8 vec8;
-  constexpr int kAttnWaves = attn_waves<D>();
   constexpr int kAttnBM = 32 * kAttnWaves;           // queries per workgroup
   constexpr int CH = D / 8;                          // 16-byte chunks per K row
   constexpr int KSTEPS = D / 16;                     // MFMA k-steps of S^T
@@ -417,10 +432,16 @@ __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* 
   __shared__ __attribute__((aligned(1024))) unsigned char vbuf1[TILE];
 
   const int nqb = (sq + kAttnBM - 1) / kAttnBM;
-  const int bh_count = gridDim.x / nqb;
-  const int id = blockIdx.x;
-  const int qb = nqb - 1 - id / bh_count;   // heaviest query block first
-  const int bh = id % bh_count;
+  const int bh_count = gridDim.x / (nqb * parts);
+  const int id = blockIdx.x / bh_count;
+  const int qb = nqb - 1 - id / parts;      // heaviest query block first
+  const int part = id % parts;
+  const int bh = blockIdx.x % bh_count;
+  int kv_end = sk;
+  if constexpr (CAUSAL) kv_end = min(sk, (qb + 1) * kAttnBM);
+  const int block_tiles = (kv_end + kAttnBN - 1) / kAttnBN;
+  const int t0 = part * per, ntiles = min(block_tiles, t0 + per);
+  if (t0 >= block_tiles) return;            // a causal block with fewer parts
   const int b = bh / heads, h = bh % heads;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -441,10 +462,6 @@ __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* 
     if (my_q < sq) qreg[s] = *(const vec8*)(qp + (i64)my_q * qss + 16 * s + 8 * hi);
     else qreg[s] = vec8{};
   }
-
-  int kv_end = sk;
-  if constexpr (CAUSAL) kv_end = min(sk, q0 + kAttnBM);
-  const int ntiles = (kv_end + kAttnBN - 1) / kAttnBN;
 
   // DMA addressing.  LDS chunk L = (i*W + wave)*64 + lane (W waves) of a K tile is key L / CH, position
   // L % CH, and holds head-dim chunk (L % CH) ^ swizzle<CH>(key) of that key; piece i moves
@@ -580,9 +597,9 @@ __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* 
   // e_pending (per lane, the same in all) is loaded one iteration ahead and made uniform only
   // after the next wait_dma, which retires it with the DMA: the load's latency is never waited
   // for on its own.
-  int e_pending = ntiles > 0 ? eh[0] : 0;
-  if (ntiles > 0) issue(0, kbuf0, vbuf0);
-  for (int tile = 0; tile < ntiles;) {
+  int e_pending = eh[t0];
+  issue(t0, kbuf0, vbuf0);
+  for (int tile = t0; tile < ntiles;) {
     wait_dma();
     __syncthreads();
     asm volatile("" : "+v"(e_pending));
@@ -606,10 +623,31 @@ __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* 
   }
   T* orow0 = o + (i64)bh * sq * D;
   float* lse_row0 = lse != nullptr ? lse + (i64)bh * sq : nullptr;
+  const bool whole = per >= block_tiles;
+  const i64 part_row0 = ((i64)part * bh_count + bh) * sq;
   if (exact) {
-    attention_exact_rows<T, D, CAUSAL, kAttnWaves>(qp, kp, v + b * vsb + h * vsh, orow0,
-                                                   lse_row0, sq, sk, q0, qss, kss, vss,
-                                                   scale_log2);
+    attention_exact_rows<T, D, CAUSAL, kAttnWaves>(
+        qp, kp, v + b * vsb + h * vsh, orow0, lse_row0, sq, sk, q0, qss, kss, vss, scale_log2,
+        t0 * kAttnBN, ntiles * kAttnBN, whole ? nullptr : po + part_row0 * D,
+        whole ? nullptr : pml + 2 * part_row0);
+    return;
+  }
+  if (!whole) {
+    const float l_part = l_even + l_odd;
+    const float l_sum = l_part + partner<32>(l_part);
+    if (my_q < sq) {
+      float* prow = po + (part_row0 + my_q) * D + 4 * hi;
+#pragma unroll
+      for (int a = 0; a < DBLK; ++a)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *(f32x4*)(prow + 32 * a + 8 * g) = f32x4{oacc[a][4 * g], oacc[a][4 * g + 1],
+                                                   oacc[a][4 * g + 2], oacc[a][4 * g + 3]};
+      if (hi == 0) {
+        pml[2 * (part_row0 + my_q)] = m_ref;
+        pml[2 * (part_row0 + my_q) + 1] = l_sum;
+      }
+    }
     return;
   }
   // ---- readout: O / l, and the natural-log LSE of the scaled scores.  The wave's 32 output
@@ -650,6 +688,60 @@ __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* 
   }
 }
 
+// Query rows whose block was split: the parts' states combined, D/4 lanes per row.
+template <typename T, int D, bool CAUSAL, int BM>
+__device__ __forceinline__ void attention_parts_merge(const float* __restrict__ po,
+                                                      const float* __restrict__ pml,
+                                                      T* __restrict__ o, float* __restrict__ lse,
+                                                      i64 rows, int sq, int sk, int per) {
+  typedef AttnIn<T> In;
+  constexpr int LANES = D / 4;
+  const i64 row = (i64)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+  const int d = (threadIdx.x % LANES) * 4;
+  if (row >= rows) return;
+  const int qb = (int)(row % sq) / BM;
+  const int kv_end = CAUSAL ? min(sk, (qb + 1) * BM) : sk;
+  const int parts = ((kv_end + kAttnBN - 1) / kAttnBN + per - 1) / per;
+  if (parts == 1) return;                // written by its workgroup
+  float mm = -kInf, ll = 0.0f;
+  f32x4 acc = f32x4{};
+  constexpr int PRE = 4;                 // parts in flight per lane
+  for (int p0 = 0; p0 < parts; p0 += PRE) {
+    float pm[PRE], pl[PRE];
+    f32x4 pa[PRE];
+#pragma unroll
+    for (int i = 0; i < PRE; ++i) {
+      pm[i] = -kInf;
+      pl[i] = 0.0f;
+      pa[i] = f32x4{};
+      if (p0 + i < parts) {
+        const i64 at = (i64)(p0 + i) * rows + row;
+        pm[i] = pml[2 * at];
+        pl[i] = pml[2 * at + 1];
+        pa[i] = *(const f32x4*)(po + at * D + d);
+      }
+    }
+    float mn = mm;
+#pragma unroll
+    for (int i = 0; i < PRE; ++i) mn = __builtin_fmaxf(mn, pm[i]);
+    const float f0 = mm == -kInf ? 0.0f : __builtin_amdgcn_exp2f(mm - mn);
+    ll *= f0;
+    acc *= f0;
+#pragma unroll
+    for (int i = 0; i < PRE; ++i) {
+      const float f1 = pm[i] == -kInf ? 0.0f : __builtin_amdgcn_exp2f(pm[i] - mn);
+      ll += pl[i] * f1;
+      acc += pa[i] * f1;
+    }
+    mm = mn;
+  }
+  const float inv = 1.0f / ll;
+  u32x2 w;
+  w.x = In::pack2(acc[0] * inv, acc[1] * inv);
+  w.y = In::pack2(acc[2] * inv, acc[3] * inv);
+  *(u32x2*)(o + row * D + d) = w;
+  if (lse != nullptr && d == 0) lse[row] = (mm + __builtin_log2f(ll)) * 0.6931471805599453f;
+}
 
 // ---------------------------------------------------------------- short query ranges
 // Attention of few queries over many keys (decoding; the query heads that share a key head folded
@@ -669,7 +761,6 @@ __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* 
 // Bound by HBM: the fp32 MFMAs take 2048 cycles per wave and 32 keys of head dim 128 (16 KB),
 // about twice the chip's HBM rate.  bf16, 512 heads x 3000 keys, one query: 312 us with the
 // kernels above, 128 us here (6.1 TB/s); K and V are loaded non-temporally (133 us without).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kShortBM = 16, kShortTK = 32, kShortWaves = 4;
 constexpr int kShortNt = 2;              // buffer loads of K and V: non-temporal
 

@@ -68,14 +68,16 @@ def use_w64(head_dim: int, causal: bool, sq: int, sk: int) -> bool:
     return sq >= W64_CAUSAL_MIN_SQ if causal else sk >= W64_MIN_SK
 
 
-def _program(head_dim: int, causal: bool, dtype="bfloat16", w64: bool | None = None) -> hip.Program:
+def _program(head_dim: int, causal: bool, dtype="bfloat16", w64: bool | None = None,
+             waves: int | None = None) -> hip.Program:
     w64 = attention_w64(head_dim, w64)
-    key = (head_dim, causal, str(dtype), w64)
+    key = (head_dim, causal, str(dtype), w64, waves)
     with _lock:
         prog = _PROGRAMS.get(key)
         if prog is None:
-            prog = hip.Program(emit_attention_source(head_dim, causal, dtype, w64=w64),
-                               f"{attention_kernel_name(head_dim, causal, dtype, w64)}.hip", BASE_OPTIONS)
+            prog = hip.Program(emit_attention_source(head_dim, causal, dtype, w64=w64, waves=waves),
+                               f"{attention_kernel_name(head_dim, causal, dtype, w64, waves)}.hip",
+                               BASE_OPTIONS)
             _PROGRAMS[key] = prog
         return prog
 
@@ -98,6 +100,7 @@ def _short_program(head_dim: int, causal: bool, dtype) -> hip.Program:
 # bf16 B*H=512 sq=1 sk=3000 d=128 312 -> 128 us (6.1 TB/s of K and V); B*H=32 sq=1 sk=32768 784 ->
 # 87; B*H=256 sq=8 sk=4096 201 -> 95; fp16 B*H=64 sq=16 sk=5000 d=64 106 -> 25; B*H=8 sq=4 sk=8192
 # d=256 383 -> 23; B*H=8 sq=1 sk=512 20 -> 8.5.
+# Longer query ranges take them where `_short_wins` finds them cheaper (few heads, few keys).
 SHORT_MAX_SQ = 16
 # Chunks of a head's keys: a workgroup's 4 waves pass a 32-key tile in about 0.6 us when each CU
 # has one, and a split costs a second launch and its chunks' states (3 us + 0.05 us a chunk).
@@ -107,11 +110,6 @@ SHORT_MAX_SQ = 16
 SHORT_MAX_CHUNKS = 64
 SHORT_TILE_US, SHORT_MERGE_US, SHORT_CHUNK_US = 0.6, 3.0, 0.05
 CUS = 256
-
-
-def use_short(head_dim: int, causal: bool, sq: int, sk: int) -> bool:
-    """Whether a call of this shape runs the short-query kernels (attention_short)."""
-    return sq <= SHORT_MAX_SQ
 
 
 @functools.lru_cache(maxsize=4096)
@@ -128,6 +126,89 @@ def short_chunks(units: int, sk: int) -> tuple[int, int]:
     chunks = min(range(1, most + 1), key=cost)
     per = -(-tiles // chunks)
     return -(-tiles // per), per
+
+
+# What `_fold_choice` and `_short_wins` price a call with, in us on MI355X, by head dim (fits of graph-replayed calls over
+# 24 shapes, cold): one workgroup's pass over a 64-key tile with a CU to itself -- the 256-query
+# kernels (two workgroups on a CU pass theirs hardly faster; at head dim 128 from 1.45 us on a
+# nearly empty chip to 2.05 on a full one, whose clock drops) and the 128-query one (4 waves x 32
+# queries) --, a workgroup's start and readout, and the merge launch with its state's traffic.
+TILE_256_US = {64: (1.1, 0.0), 128: (1.45, 0.6), 256: None}
+TILE_128_US = {64: 0.6, 128: 1.15, 256: 3.3}
+BLOCK_US, MERGE_US, STATE_BYTES_PER_US, PACK_US, PACK_BYTES_PER_US = 2.5, 6.0, 8e6, 4.0, 5e6
+MAX_STATE_BYTES = 256 << 20
+# The short-query kernels: launch, a workgroup's start and end, its 4 waves' pass over 4 tiles of
+# 32 keys, and the workgroups the chip holds at once.
+SHORT_LAUNCH_US, SHORT_BLOCK_US = 3.0, 3.0
+SHORT_PASS_US = {64: 1.2, 128: 1.8, 256: 2.5}
+SHORT_RESIDENT = {64: 1024, 128: 512, 256: 256}
+
+
+def _fold_cost(bh, sq, sk, head_dim, causal, bm, tile_us, per):
+    """us of the fold (and merge) with query blocks of `bm` and keys in parts of `per` tiles."""
+    nqb = -(-sq // bm)
+    blocks = [-(-(min(sk, (i + 1) * bm) if causal else sk) // BLOCK_N) for i in range(nqb)]
+    per = min(per, blocks[-1])
+    items = bh * sum(-(-t // per) for t in blocks)
+    if causal:     # heaviest first: the last items to finish are about half a part apart
+        tiles = max(per, bh * sum(blocks) / CUS + per / 2)
+    else:
+        tiles = -(-items // CUS) * per
+    cost = tile_us * tiles + BLOCK_US * max(1.0, items / CUS)
+    if per < blocks[-1]:
+        state = 2 * 4 * items * sq / nqb * head_dim    # written and read, fp32
+        cost += MERGE_US + state / STATE_BYTES_PER_US
+    return cost
+
+
+@functools.lru_cache(maxsize=4096)
+def _fold_choice(bh: int, sq: int, sk: int, head_dim: int, causal: bool) -> tuple:
+    """(us, (w64, waves, tiles per part or None)) of the cheapest fold after the V^T pack.
+
+    The 256-query kernels pass a tile for fewest us per query and are best on a full chip; the
+    128-query one makes twice the workgroups, and parts of the keys make as many as it takes.
+    Measured, 256 queries / 128 / 128 in parts (us of the whole call): bf16 d=128 full B*H=36
+    sq=100 sk=4000 108 / 92 / 44; causal B*H=8 s=4096 103 / 84 / 63; full B*H=64 sq=333 sk=2000
+    67 / 57 / 59; causal B*H=128 s=1500 122 / 117 / 162; full B*H=128 s=512 33 / 34 / 64; causal
+    B*H=128 s=4096 592 / 645 / -; d=64 causal B*H=1 s=6000 110 / 82 / 28; d=256 full B*H=16 s=700
+    - / 45 / 43."""
+    most = -(-(min(sk, sq) if causal else sk) // BLOCK_N)
+    big = TILE_256_US[head_dim]
+    best = None
+    if big is not None:
+        tile_us = big[0] + big[1] * min(1.0, bh * -(-sq // 256) / CUS)
+        best = (_fold_cost(bh, sq, sk, head_dim, causal, 256, tile_us, most + 4),
+                (use_w64(head_dim, causal, sq, sk), 8, None))
+    for parts in (1, 2, 3, 4, 6, 8, 12, 16):
+        per = -(-most // parts)
+        if parts > 1 and (per < 2 or parts * bh * sq * (head_dim + 2) * 4 > MAX_STATE_BYTES):
+            break
+        cost = _fold_cost(bh, sq, sk, head_dim, causal, 128, TILE_128_US[head_dim], per if parts > 1 else most + 4)
+        if best is None or cost < best[0]:
+            best = (cost, (False, 4, per if parts > 1 else None))
+    return best
+
+
+def _fold_plan(bh, sq, sk, head_dim, causal):
+    return _fold_choice(bh, sq, sk, head_dim, causal)[1]
+
+
+@functools.lru_cache(maxsize=4096)
+def _short_wins(bh: int, sq: int, sk: int, head_dim: int, causal: bool) -> bool:
+    """Whether the short-query kernels run a call: always up to 16 queries; beyond, where they are
+    estimated 15% cheaper (bf16 causal B*H=8 s=512 13.3 us against 17.5, d=256 causal B*H=16 s=100
+    9.8 against 18.4; B*H=96 s=1000 d=64 full 34 against 21)."""
+    if sq <= SHORT_MAX_SQ:
+        return True
+    seen = min(sq, sk) if causal else sk
+    fold = (_fold_choice(bh, sq, sk, head_dim, causal)[0] + PACK_US
+            + bh * seen * head_dim * 4 / PACK_BYTES_PER_US)
+    units = bh * -(-sq // ATTN_SHORT_BLOCK_M)
+    chunks, per = short_chunks(units, seen)
+    short = (SHORT_LAUNCH_US + -(-units * chunks // SHORT_RESIDENT[head_dim])
+             * (SHORT_BLOCK_US + -(-per // ATTN_SHORT_WAVES) * SHORT_PASS_US[head_dim])
+             + (MERGE_US if chunks > 1 else 0.0))
+    return 1.15 * short < fold
 
 
 def validate_attention_inputs(q, k, v, *, metadata: bool = False):
@@ -163,17 +244,26 @@ def _kernel_ready(t):
 def run_attention(q, k, v, *, scale: float | None = None, causal: bool = True,
                   return_lse: bool = False):
     """Attention fold on the current stream; see the module docstring for the contract."""
-    if q.ndim == 4 and use_short(q.shape[3], causal, q.shape[2], k.shape[2]):
+    if _takes_short(q, k, causal):
         out, lse = _launch_short(q, k, v, scale, causal, return_lse)
     else:
         out, lse, _ = launch_attention(q, k, v, scale=scale, causal=causal, return_lse=return_lse)
     return (out, lse) if return_lse else out
 
 
+def _takes_short(q, k, causal) -> bool:
+    """Whether the call runs the short-query kernels (calls to be refused do not matter here)."""
+    if q.ndim != 4 or k.ndim != 4 or q.shape[3] not in ATTN_HEAD_DIMS or 0 in q.shape or 0 in k.shape:
+        return False
+    B, H, Sq, D = q.shape
+    return _short_wins(B * H, Sq, k.shape[2], D, bool(causal))
+
+
 def launch_attention(q, k, v, *, scale: float | None = None, causal: bool = True,
                      return_lse: bool = False):
-    """(out, lse or None, exps or None): the fold's two launches.  `exps` is the int32 tile
-    exponent table [B*H*ceil(Sk/64)] the V^T pack wrote (None when nothing was launched);
+    """(out, lse or None, exps or None): the V^T pack and the fold.  `exps` is the int32 tile
+    exponent table [B*H*ceil(Sk/64)] the pack wrote (None when nothing was launched; of the first
+    min(Sk, Sq) keys under the causal mask, which hides the others from every query);
     `exact_path_taken(exps)` tells whether some query block took the exact fp32 path."""
     return _launch(q, k, v, scale, causal, return_lse, V_EXPONENT_MAX)
 
@@ -236,7 +326,8 @@ def _launch_short(q, k, v, scale, causal, return_lse):
     return out, lse
 
 
-def _launch(q, k, v, scale, causal, return_lse, e_max: int, w64: bool | None = None):
+def _launch(q, k, v, scale, causal, return_lse, e_max: int, w64: bool | None = None,
+            waves: int | None = None, per: int | None = None):
     """The launches with the exact path's threshold as a parameter: e_max = -1 sends every
     query block through the exact fp32 path (the tests compare the two paths with it).
     `w64=False` runs the compiler-scheduled 32-queries-per-wave kernel at head dim 128 instead
@@ -247,36 +338,53 @@ def _launch(q, k, v, scale, causal, return_lse, e_max: int, w64: bool | None = N
     if done:
         return out, lse, None
     B, H, Sq, D = q.shape
-    if w64 is None:
-        w64 = use_w64(D, causal, Sq, k.shape[2])
+    if w64 is None and waves is None:
+        w64, waves, per = _fold_plan(B * H, Sq, k.shape[2], D, bool(causal))
     q, k, v = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)
     if k.stride(2) >= K_ROW_STRIDE_MAX:
         k = k.contiguous()
     if q.stride(2) >= Q_ROW_STRIDE_MAX:
         q = q.contiguous()
     device = q.device.index if q.device.index is not None else torch.cuda.current_device()
-    Sk = k.shape[2]
+    Sk = min(k.shape[2], Sq) if causal else k.shape[2]    # no query sees a key past the last query
     ntiles = (Sk + BLOCK_N - 1) // BLOCK_N
     # V^T tile images (fp16, MFMA operand order) and one power-of-two exponent per tile
     vt = torch.empty((B * H * ntiles * D * BLOCK_N,), dtype=torch.float16, device=q.device)
     exps = torch.empty((B * H * ntiles,), dtype=torch.int32, device=q.device)
-    prog = _program(D, causal, q.dtype, w64)
+    prog = _program(D, causal, q.dtype, w64, waves)
     pack = prog.kernel(attention_pack_kernel_name(D, q.dtype),
                        (hip.PTR,) * 3 + (hip.I32,) * 2 + (hip.I64,) * 3, 256, device)
-    fold = prog.kernel(attention_kernel_name(D, causal, q.dtype, attention_w64(D, w64)),
-                       (hip.PTR,) * 7 + (hip.I32,) * 3 + (hip.I64,) * 9 + (hip.I32, hip.F32),
-                       attention_fold_threads(D, w64), device)
+    w64 = attention_w64(D, w64)
+    name = attention_kernel_name(D, causal, q.dtype, w64, waves)
+    fold = prog.kernel(name, (hip.PTR,) * 7 + (hip.I32,) * 3 + (hip.I64,) * 9 + (hip.I32, hip.F32)
+                       + (() if w64 else (hip.PTR,) * 2 + (hip.I32,) * 2),
+                       attention_fold_threads(D, w64, waves), device)
     stream = hip.current_stream(q.device)
     pack.launch((B * H * ntiles,),
                 (v.data_ptr(), vt.data_ptr(), exps.data_ptr(), H, Sk,
                  v.stride(0), v.stride(1), v.stride(2)), stream)
-    bm = attention_block_m(D, w64)
+    bm = attention_block_m(D, w64, waves)
     nqb = (Sq + bm - 1) // bm
-    fold.launch((nqb * B * H,),
+    lse_ptr = lse.data_ptr() if lse is not None else 0
+    parts, rows, po, pml = 1, B * H * Sq, 0, 0
+    if not w64:
+        most = -(-(min(Sk, nqb * bm) if causal else Sk) // BLOCK_N)   # tiles of the longest block
+        per = min(per or most, most)
+        parts = -(-most // per)
+        if parts > 1:     # fp32 O, then (max, sum), of every part and query
+            state = torch.empty(parts * rows * (D + 2), dtype=torch.float32, device=q.device)
+            po = state.data_ptr()
+            pml = po + 4 * parts * rows * D
+    fold.launch((nqb * B * H * parts,),
                 (q.data_ptr(), k.data_ptr(), vt.data_ptr(), exps.data_ptr(), v.data_ptr(),
-                 out.data_ptr(), lse.data_ptr() if lse is not None else 0, H, Sq, Sk,
+                 out.data_ptr(), lse_ptr, H, Sq, Sk,
                  q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
-                 v.stride(0), v.stride(1), v.stride(2), int(e_max), scale * LOG2E), stream)
+                 v.stride(0), v.stride(1), v.stride(2), int(e_max), scale * LOG2E)
+                + (() if w64 else (po, pml, parts, per)), stream)
+    if parts > 1:
+        merge = prog.kernel(name + "_merge", (hip.PTR,) * 4 + (hip.I64,) + (hip.I32,) * 3, 256, device)
+        merge.launch((-(-rows * (D // 4) // 256),),
+                     (po, pml, out.data_ptr(), lse_ptr, rows, Sq, Sk, per), stream)
     return out, lse, exps
 
 

@@ -561,20 +561,22 @@ def attention_w64(head_dim: int, w64: bool | None = None) -> bool:
     return head_dim == 128 if w64 is None else (w64 and head_dim == 128)
 
 
-def attention_waves(head_dim: int, w64: bool | None = None) -> int:
+def attention_waves(head_dim: int, w64: bool | None = None, waves: int | None = None) -> int:
+    """Wave64s per fold workgroup: the 64-query kernel has 4; the 32-query one `waves`, by default
+    two per SIMD up to head dim 128 and one at 256, where O^T and Q^T alone take 192 registers."""
     if attention_w64(head_dim, w64):
         return 4
-    return 8 if head_dim <= 128 else 4
+    return waves or (8 if head_dim <= 128 else 4)
 
 
-def attention_fold_threads(head_dim: int, w64: bool | None = None) -> int:
-    return 64 * attention_waves(head_dim, w64)
+def attention_fold_threads(head_dim: int, w64: bool | None = None, waves: int | None = None) -> int:
+    return 64 * attention_waves(head_dim, w64, waves)
 
 
-def attention_block_m(head_dim: int, w64: bool | None = None) -> int:
+def attention_block_m(head_dim: int, w64: bool | None = None, waves: int | None = None) -> int:
     """Queries per fold workgroup."""
     per_wave = 64 if attention_w64(head_dim, w64) else 32
-    return per_wave * attention_waves(head_dim, w64)
+    return per_wave * attention_waves(head_dim, w64, waves)
 
 
 ATTN_DTYPES = {"bfloat16": ("bf16", "__bf16"), "float16": ("f16", "_Float16")}
@@ -588,26 +590,36 @@ def _attn_dtype(dtype) -> tuple[str, str]:
 
 
 def emit_attention_source(head_dim: int, causal: bool, dtype="bfloat16",
-                          waves_per_eu: int | None = None, w64: bool | None = None) -> str:
+                          waves_per_eu: int | None = None, w64: bool | None = None,
+                          waves: int | None = None) -> str:
     """hiprtc unit of the online-softmax attention fold (no reference counterpart): the
     logsumexp repair exp(s - s2) applied per key tile to (m, l, O).  Holds two kernels: the
     V^T tile packer and the fold itself (with its exact fallback for out-of-range V)."""
     if head_dim not in ATTN_HEAD_DIMS:
         raise NotImplementedError("attention fold supports head_dim 64, 128 and 256")
     w64 = attention_w64(head_dim, w64)
-    wpe = attention_waves(head_dim, w64) // 4 if waves_per_eu is None else waves_per_eu
-    threads = attention_fold_threads(head_dim, w64)
+    # the registers of two waves per SIMD up to head dim 128 (of one for the 64-query kernel)
+    wpe = (2 if head_dim <= 128 and not w64 else 1) if waves_per_eu is None else waves_per_eu
+    threads = attention_fold_threads(head_dim, w64, waves)
     tag, ctype = _attn_dtype(dtype)
-    name = attention_kernel_name(head_dim, causal, dtype, w64)
+    name = attention_kernel_name(head_dim, causal, dtype, w64, waves)
     pack = attention_pack_kernel_name(head_dim, dtype)
     cz = "true" if causal else "false"
     if w64:
         from neptune_codegen.attention_asm import asm_macro
         prefix = asm_macro(causal, tag) + "\n"
         call = f"  nep::attention_fwd_w64<{ctype}, {cz}>("
+        more, merge = ("", ""), ""
     else:
         prefix = ""
-        call = f"  nep::attention_fwd<{ctype}, {head_dim}, {cz}>("
+        more = (", float* po, float* pml, int parts, int per", ", po, pml, parts, per")
+        bm = attention_block_m(head_dim, False, waves)
+        merge = (f'extern "C" __global__ void __launch_bounds__(256) {name}_merge(const float* po, '
+                 "const float* pml, void* o, float* lse, long long rows, int sq, int sk, int per) {\n"
+                 f"  nep::attention_parts_merge<{ctype}, {head_dim}, {cz}, {bm}>(po, pml, ({ctype}*)o, "
+                 "lse, rows, sq, sk, per);\n}\n")
+        call = (f"  nep::attention_fwd<{ctype}, {head_dim}, {cz}, "
+                f"{attention_waves(head_dim, False, waves)}>(")
     return "\n".join([
         "// AUTO-GENERATED by neptune_codegen (HIP emitter) -- do not edit.\n"
         f"// online-softmax attention fold: head_dim={head_dim}, causal={causal}, {tag} inputs; "
@@ -620,16 +632,21 @@ def emit_attention_source(head_dim: int, causal: bool, dtype="bfloat16",
         f'extern "C" __global__ void __launch_bounds__({threads}, {wpe}) {name}(const void* q, const void* k, '
         "const void* vt, const int* exps, const void* v, void* o, float* lse, int heads, int sq, "
         "int sk, long long qsb, long long qsh, long long qss, long long ksb, long long ksh, "
-        "long long kss, long long vsb, long long vsh, long long vss, int e_max, float scale_log2) {\n"
+        f"long long kss, long long vsb, long long vsh, long long vss, int e_max, float scale_log2{more[0]}) {{\n"
         + call + f"(const {ctype}*)q, "
         f"(const {ctype}*)k, (const nep::u16*)vt, exps, (const {ctype}*)v, ({ctype}*)o, lse, heads, "
-        "sq, sk, qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, e_max, scale_log2);\n}\n"])
+        f"sq, sk, qsb, qsh, qss, ksb, ksh, kss, vsb, vsh, vss, e_max, scale_log2{more[1]});\n}}\n",
+        merge])
 
 
-def attention_kernel_name(head_dim: int, causal: bool, dtype="bfloat16", w64: bool = False) -> str:
-    """The fold's symbol; the 64-queries-per-wave kernel carries a `_w64` suffix."""
+def attention_kernel_name(head_dim: int, causal: bool, dtype="bfloat16", w64: bool = False,
+                          waves: int | None = None) -> str:
+    """The fold's symbol; the 64-queries-per-wave kernel carries a `_w64` suffix, the 32-query one
+    its waves where they are not the default."""
     tag, _ = _attn_dtype(dtype)
     suffix = "_w64" if attention_w64(head_dim, w64) and w64 else ""
+    if not suffix and waves and waves != attention_waves(head_dim, False):
+        suffix = f"_x{waves}"
     return f"attention_fold_{tag}_d{head_dim}_{'causal' if causal else 'full'}{suffix}"
 
 

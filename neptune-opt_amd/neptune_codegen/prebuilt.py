@@ -72,13 +72,18 @@ def _segment_programs():
 
 
 def _attention_programs():
-    from neptune_codegen.attention import _program
+    from neptune_codegen.attention import _program, _short_program
 
-    # head dim 128: both fold kernels (attention.use_w64 picks one by shape)
-    return [_program(128, c, dt, w) for c in (True, False) for dt in ("bfloat16", "float16")
-            for w in (True, False)] + [
-        _program(64, True), _program(64, False), _program(64, False, "float16"),
-        _program(256, True), _program(256, False), _program(256, True, "float16")]
+    # head dim 128: the 64-queries-per-wave kernel beside the 8- and 4-wave ones; 64: 8 and 4 waves;
+    # 256: 4 waves (attention._fold_choice picks by shape); the short-query kernels of each
+    out = []
+    for dt in ("bfloat16", "float16"):
+        for causal in (True, False):
+            out.append(_program(128, causal, dt, True, 8))
+            for dim, waves in ((128, 8), (128, 4), (64, 8), (64, 4), (256, 4)):
+                out.append(_program(dim, causal, dt, False, waves))
+            out += [_short_program(dim, causal, dt) for dim in (64, 128, 256)]
+    return out
 
 
 def programs():

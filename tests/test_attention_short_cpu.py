@@ -15,3 +15,22 @@ def test_short_chunks_cover_the_keys_once():
     assert A.short_chunks(1, 128) == (1, 4)
     assert A.short_chunks(512, 3000)[0] == 1          # the heads fill the chip
     assert A.short_chunks(1, 1 << 20)[0] == A.SHORT_MAX_CHUNKS
+
+
+def test_fold_choice_is_launchable():
+    """Every choice is a kernel that exists, with parts that cover the keys and fit the scratch."""
+    for dim in (64, 128, 256):
+        for causal in (True, False):
+            for bh in (1, 8, 36, 128, 1000):
+                for sq, sk in ((17, 17), (100, 4000), (300, 300), (4096, 4096), (5000, 90)):
+                    cost, (w64, waves, per) = A._fold_choice(bh, sq, sk, dim, causal)
+                    assert cost > 0 and waves in ((8, 4) if dim <= 128 else (4,))
+                    assert not w64 or (dim == 128 and A.use_w64(dim, causal, sq, sk))
+                    if per is not None:
+                        most = -(-(min(sq, sk) if causal else sk) // A.BLOCK_N)
+                        assert waves == 4 and 2 <= per < most
+                        assert -(-most // per) * bh * sq * (dim + 2) * 4 <= A.MAX_STATE_BYTES
+    # a full chip keeps whole keys and the largest blocks; few heads over long keys are split
+    assert A._fold_choice(128, 4096, 4096, 128, True)[1] == (True, 8, None)
+    assert A._fold_choice(36, 100, 4000, 128, False)[1][2] is not None
+    assert A._short_wins(1, 16, 1 << 15, 128, False) and not A._short_wins(128, 4096, 4096, 128, True)
