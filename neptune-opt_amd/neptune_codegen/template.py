@@ -155,17 +155,46 @@ def compile_readout(name: str, values: dict | None = None, *, nan_posinf_rows: b
     return program
 
 
-def launch_readout(program: ReadoutProgram, x2, out, rows, ncols, block, num_warps) -> None:
-    """Launch a readout on the current stream: out [rows, ncols] contiguous."""
+def launch_readout(program: ReadoutProgram, x2, out, rows, ncols, block, num_warps):
+    """Launch a readout on the current stream: out [rows, ncols] contiguous.  Returns the kernel,
+    its grid and its arguments behind the two pointers."""
     import torch
 
     device = x2.device.index if x2.device.index is not None else torch.cuda.current_device()
     var = _fold_variant(x2, ncols, block, num_warps, resident=True)
     rpw = max(1, var.wg // var.tpr)
-    program.kernel(var, device, resident=ncols <= readout_tile(var)).launch(
-        (_grid_1d(rows, rpw),),
-        (x2.data_ptr(), out.data_ptr(), rows, ncols, x2.stride(0), x2.stride(1)),
-        hip.current_stream(x2.device))
+    kernel = program.kernel(var, device, resident=ncols <= readout_tile(var))
+    grid, tail = (_grid_1d(rows, rpw),), (rows, ncols, x2.stride(0), x2.stride(1))
+    kernel.launch(grid, (x2.data_ptr(), out.data_ptr()) + tail, hip.current_stream(x2.device))
+    return kernel, grid, tail
+
+
+_RUN_SEEN: dict = {}
+_RUN_SEEN_MAX = 4096
+
+
+def _fold_seen_key(x, options: tuple, params: dict):
+    """Key of a fold or readout call on a plain strided device tensor: everything the validation
+    and the launch choice read; None when the call takes the full path."""
+    import torch
+
+    if (type(x) is not torch.Tensor or not x.is_cuda or x.layout != torch.strided
+            or hip.recording_active()):
+        return None
+    try:
+        key = options + (x.dtype, x.device, x.shape, x.stride(), x.data_ptr() % 16,
+                         tuple(sorted((k, type(v).__name__, repr(v)) for k, v in params.items()))
+                         if params else ())
+        hash(key)
+    except TypeError:
+        return None
+    return key
+
+
+def _remember(key, launch) -> None:
+    if len(_RUN_SEEN) >= _RUN_SEEN_MAX:
+        _RUN_SEEN.clear()
+    _RUN_SEEN[key] = launch
 
 
 def run_readout(name: str, x, *, nan_posinf_rows: bool = True, block: int | None = None,
@@ -173,10 +202,19 @@ def run_readout(name: str, x, *, nan_posinf_rows: bool = True, block: int | None
     """phi(x) - r over the last dimension, r the row's exponential fold (fp32), rounded once to
     x.dtype: for logsumexp, log_softmax(x, -1).  With nan_posinf_rows a row containing +inf
     reads out NaN, as the reference's log_softmax lowering does (lowering.py:92-98).  Fresh
-    contiguous output of x's shape and dtype; Fake/meta tensors return metadata only."""
+    contiguous output of x's shape and dtype; Fake/meta tensors return metadata only.  A call whose
+    tensor layout, options and parameters were seen before reuses that call's kernel and launch
+    shape, as `run` does."""
     import torch
     from torch._subclasses.fake_tensor import FakeTensor
 
+    seen = _fold_seen_key(x, ("readout", name, bool(nan_posinf_rows), block, num_warps), params)
+    entry = _RUN_SEEN.get(seen) if seen is not None else None
+    if entry is not None:
+        kernel, grid, tail = entry
+        out = torch.empty(x.shape, device=x.device, dtype=x.dtype)
+        kernel.launch(grid, (x.data_ptr(), out.data_ptr()) + tail, hip.current_stream(x.device))
+        return out
     metadata = isinstance(x, FakeTensor) or x.device.type == "meta"
     _validate_row_last(x, metadata=metadata)
     program = compile_readout(name, params, nan_posinf_rows=nan_posinf_rows)
@@ -190,7 +228,9 @@ def run_readout(name: str, x, *, nan_posinf_rows: bool = True, block: int | None
         cfg = best_config(rows, ncols, x.dtype, x.device)
         block = cfg[0] if block is None else block
         num_warps = cfg[1] if num_warps is None else num_warps
-    launch_readout(program, x2, out, rows, ncols, block, num_warps)
+    launch = launch_readout(program, x2, out, rows, ncols, block, num_warps)
+    if seen is not None and x2.data_ptr() == x.data_ptr():
+        _remember(seen, launch)
     return out
 
 
@@ -367,10 +407,6 @@ def launch_reduction(kernel, plan, x2, out, rows, ncols, block, num_warps, *, wr
     return kp, grid_p, tail_p, km, grid_m, tail_m, rows * nparts
 
 
-_RUN_SEEN: dict = {}
-_RUN_SEEN_MAX = 4096
-
-
 def run(name: str, x, block: int | None = None, num_warps: int | None = None,
         keepdim: bool = False, plan: str = "serial", **params):
     """Reduce the last dimension of `x` with the generated fold `name`.
@@ -389,15 +425,9 @@ def run(name: str, x, block: int | None = None, num_warps: int | None = None,
 
     from neptune_codegen.skeleton import param_defaults
 
-    seen = None
-    if type(x) is torch.Tensor and x.is_cuda and not hip.recording_active():
-        try:
-            seen = (name, plan, x.dtype, x.device, tuple(x.shape), tuple(x.stride()),
-                    x.data_ptr() % 16, block, num_warps, keepdim,
-                    tuple(sorted((k, type(v).__name__, repr(v)) for k, v in params.items())))
-            entry = _RUN_SEEN.get(seen)
-        except TypeError:
-            seen, entry = None, None
+    seen = _fold_seen_key(x, (name, plan, block, num_warps, keepdim), params)
+    if seen is not None:
+        entry = _RUN_SEEN.get(seen)
         if entry is not None:
             out = torch.empty(entry[0], device=x.device, dtype=x.dtype)
             stream = hip.current_stream(x.device)
@@ -438,9 +468,7 @@ def run(name: str, x, block: int | None = None, num_warps: int | None = None,
         num_warps = cfg[1] if num_warps is None else num_warps
     launch = launch_reduction(kernel, plan, x2, out, rows, ncols, block, num_warps)
     if seen is not None and launch is not None and x2.data_ptr() == x.data_ptr():
-        if len(_RUN_SEEN) >= _RUN_SEEN_MAX:
-            _RUN_SEEN.clear()
-        _RUN_SEEN[seen] = (tuple(out.shape),) + tuple(launch)
+        _remember(seen, (tuple(out.shape),) + tuple(launch))
     return out
 
 

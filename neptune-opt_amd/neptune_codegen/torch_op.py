@@ -418,34 +418,48 @@ def _spans_program() -> hip.Program:
         return _SPANS_PROGRAM
 
 
+def _spans_launch(lengths):
+    """(number of lengths, blocks, block-sum kernel, scan kernel) of the prefix sum of contiguous
+    `lengths`."""
+    import torch
+
+    from neptune_codegen.emitters import SPAN_BLOCK
+
+    n = lengths.shape[0]
+    tag = "i32" if lengths.dtype == torch.int32 else "i64"
+    device = lengths.device.index if lengths.device.index is not None else torch.cuda.current_device()
+    prog = _spans_program()
+    args = (hip.PTR, hip.I64, hip.PTR, hip.PTR)
+    return (n, (n + SPAN_BLOCK - 1) // SPAN_BLOCK,
+            prog.kernel(f"segment_spans_sums_{tag}", args, 256, device),
+            prog.kernel(f"segment_spans_scan_{tag}", args, 256, device))
+
+
+def _run_spans(launch, lengths, status_ptr: int):
+    """int64 spans [0, cumsum(lengths)] by `launch`; the first kernel also sets a non-null status
+    word to 1."""
+    import torch
+
+    n, nblocks, sums_kernel, scan_kernel = launch
+    work = torch.empty(n + 1 + nblocks, dtype=torch.int64, device=lengths.device)
+    spans = work.data_ptr()
+    sums = spans + 8 * (n + 1)
+    stream = hip.current_stream(lengths.device)
+    sums_kernel.launch((nblocks,), (lengths.data_ptr(), n, sums, status_ptr), stream)
+    scan_kernel.launch((nblocks,), (lengths.data_ptr(), n, sums, spans), stream)
+    return work[:n + 1]
+
+
 def _device_spans(data, segments, *, offsets, status=None):
     """[start, end) boundaries for the fused-validation launch: offsets as given, lengths as an
     int64 prefix sum (the same values `_segment_spans` builds) by two HIP launches -- block
     sums, then a per-block scan on top of the preceding blocks; no asserts here (the segment
     kernel checks the spans).  With lengths, the first launch also sets `status` (one int32)
     to 1; returns (spans, status set)."""
-    import torch
-
-    from neptune_codegen.emitters import SPAN_BLOCK
-
     if offsets:
         return segments, False
     lengths = segments.contiguous()
-    n = lengths.shape[0]
-    spans = torch.empty(n + 1, dtype=torch.int64, device=segments.device)
-    nblocks = (n + SPAN_BLOCK - 1) // SPAN_BLOCK
-    sums = hip.scratch(torch.empty(nblocks, dtype=torch.int64, device=segments.device))
-    tag = "i32" if lengths.dtype == torch.int32 else "i64"
-    device = segments.device.index if segments.device.index is not None else torch.cuda.current_device()
-    prog = _spans_program()
-    stream = hip.current_stream(segments.device)
-    prog.kernel(f"segment_spans_sums_{tag}", (hip.PTR, hip.I64, hip.PTR, hip.PTR), 256,
-                device).launch((nblocks,), (lengths.data_ptr(), n, sums.data_ptr(),
-                                            status.data_ptr() if status is not None else 0),
-                               stream)
-    prog.kernel(f"segment_spans_scan_{tag}", (hip.PTR, hip.I64, hip.PTR, hip.PTR), 256,
-                device).launch((nblocks,), (lengths.data_ptr(), n, sums.data_ptr(),
-                                            spans.data_ptr()), stream)
+    spans = _run_spans(_spans_launch(lengths), lengths, status.data_ptr() if status is not None else 0)
     return spans, status is not None
 
 
@@ -457,12 +471,13 @@ def _launch_segment(name, data, segments, params, plan, *, wrapper=None):
     Otherwise the spans are built and asserted exactly as `_segment_spans` does."""
     import torch
 
-    # CSR offsets seen before with the same tensor layout and parameters: the validation, the
-    # variant and the launch shape are what that call found; only the output allocation, the
-    # launch (span checks inside) and the assert on the armed status word remain
+    # Offsets or lengths seen before with the same tensor layout and parameters: the validation, the
+    # variant and the launch shapes are what that call found; only the allocations, the launches
+    # (span checks inside) and the assert on the armed status word remain
     key = None
-    if (params["offsets"] and type(data) is torch.Tensor and type(segments) is torch.Tensor
-            and data.is_cuda and not hip.recording_active()):
+    if (type(data) is torch.Tensor and type(segments) is torch.Tensor and data.is_cuda
+            and data.layout == torch.strided and segments.layout == torch.strided
+            and not hip.recording_active()):
         try:
             key = (name, plan, tuple(sorted((k, type(v).__name__, repr(v)) for k, v in params.items())),
                    data.dtype, data.device, tuple(data.shape), tuple(data.stride()),
@@ -473,9 +488,10 @@ def _launch_segment(name, data, segments, params, plan, *, wrapper=None):
             key, entry = None, None
         status = _armed_status(data.device) if entry is not None else None
         if status is not None:
-            out_shape, kernel, grid, tail = entry
+            out_shape, spans_launch, kernel, grid, tail = entry
             out = torch.empty(out_shape, dtype=data.dtype, device=data.device)
-            kernel.launch(grid, (data.data_ptr(), segments.data_ptr(), out.data_ptr()) + tail,
+            spans = segments if spans_launch is None else _run_spans(spans_launch, segments, 0)
+            kernel.launch(grid, (data.data_ptr(), spans.data_ptr(), out.data_ptr()) + tail,
                           hip.current_stream(data.device))
             torch._assert_async(status, DESCRIPTOR_MESSAGE)
             return out
@@ -501,12 +517,13 @@ def _launch_segment(name, data, segments, params, plan, *, wrapper=None):
         launch = launch_segment_kernel(compile_segment_reduction(name, params, plan), flat, spans,
                                        out, status=status, cover=cover)
         torch._assert_async(status, DESCRIPTOR_MESSAGE)
-        if (key is not None and flat.data_ptr() == data.data_ptr() and spans is segments
-                and status is _STATUS.get(data.device.index if data.device.index is not None
+        if (key is not None and flat.data_ptr() == data.data_ptr()
+                and (params["offsets"] or segments.is_contiguous()) and status is _STATUS.get(data.device.index if data.device.index is not None
                                           else torch.cuda.current_device())):
             if len(_SEG_SEEN) >= 4096:
                 _SEG_SEEN.clear()
-            _SEG_SEEN[key] = (tuple(out.shape),) + launch
+            spans_launch = None if params["offsets"] else _spans_launch(segments)
+            _SEG_SEEN[key] = (tuple(out.shape), spans_launch) + launch
         return out
     _segment_spans(data, segments, offsets=params["offsets"], unsafe=params["unsafe"])
     return out
