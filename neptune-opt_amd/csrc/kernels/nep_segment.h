@@ -256,6 +256,7 @@ __device__ __forceinline__ i64 wave_sum_i64(i64 v) {
 }
 
 // Sum over the workgroup, returned to every thread.
+template <int THREADS = kSpanThreads>
 __device__ __forceinline__ i64 block_sum_i64(i64 v, i64* lds) {
   v = wave_sum_i64(v);
   const int wave = threadIdx.x >> 6;
@@ -264,7 +265,7 @@ __device__ __forceinline__ i64 block_sum_i64(i64 v, i64* lds) {
   __syncthreads();
   i64 total = 0;
 #pragma unroll
-  for (int w = 0; w < kSpanThreads / 64; ++w) total += lds[w];
+  for (int w = 0; w < THREADS / 64; ++w) total += lds[w];
   return total;
 }
 
@@ -310,6 +311,37 @@ __device__ __forceinline__ void spans_scan(const L* __restrict__ lengths, i64 n,
   for (i64 b = threadIdx.x; b < (i64)blockIdx.x; b += kSpanThreads) before += sums[b];
   before = block_sum_i64(before, lds);
   const i64 base = (i64)blockIdx.x * kSpanBlock + (i64)threadIdx.x * kSpanPer;
+  i64 run[kSpanPer];
+  i64 acc = 0;
+#pragma unroll
+  for (int k = 0; k < kSpanPer; ++k) {
+    acc += base + k < n ? (i64)lengths[base + k] : 0;
+    run[k] = acc;
+  }
+  const i64 offset = before + block_exclusive_i64(acc, lds);
+#pragma unroll
+  for (int k = 0; k < kSpanPer; ++k)
+    if (base + k < n) spans[base + k + 1] = offset + run[k];
+  if (blockIdx.x == 0 && threadIdx.x == 0) spans[0] = 0;
+}
+
+// The same in one launch: each workgroup of 1024 threads sums every length before its own 4096
+// itself, which for a few blocks costs less than a launch.
+constexpr int kSpanDirectThreads = 1024;
+constexpr i64 kSpanDirectBlock = (i64)kSpanDirectThreads * kSpanPer;
+template <class L>
+__device__ __forceinline__ void spans_direct(const L* __restrict__ lengths, i64 n,
+                                             i64* __restrict__ spans, int* __restrict__ status) {
+  __shared__ i64 lds[kSpanDirectThreads / 64];
+  if (status != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *status = 1;
+  i64 before = 0;
+#pragma unroll 2
+  for (i64 b = threadIdx.x; b < (i64)blockIdx.x * kSpanDirectBlock; b += kSpanDirectBlock) {
+#pragma unroll
+    for (int k = 0; k < kSpanPer; ++k) before += (i64)lengths[b + k * kSpanDirectThreads];
+  }
+  before = block_sum_i64<kSpanDirectThreads>(before, lds);
+  const i64 base = (i64)blockIdx.x * kSpanDirectBlock + (i64)threadIdx.x * kSpanPer;
   i64 run[kSpanPer];
   i64 acc = 0;
 #pragma unroll

@@ -525,6 +525,7 @@ def emit_segment_source(name: str, *, initial=None, offsets=False, plan="serial"
 
 
 SPAN_BLOCK = 256 * 4           # lengths per workgroup of the spans kernels (nep_segment.h)
+SPAN_DIRECT_THREADS = 1024     # threads of the one-launch spans kernel, 4 lengths each
 
 
 def emit_segment_spans_source() -> str:
@@ -541,6 +542,10 @@ def emit_segment_spans_source() -> str:
             f'extern "C" __global__ void __launch_bounds__(256) segment_spans_scan_{tag}('
             "const void* lengths, long long n, const long long* sums, long long* spans) {\n"
             f"  nep::spans_scan<{ctype}>((const {ctype}*)lengths, n, sums, spans);\n}}\n")
+        parts.append(
+            f'extern "C" __global__ void __launch_bounds__({SPAN_DIRECT_THREADS}) segment_spans_direct_{tag}('
+            "const void* lengths, long long n, long long* spans, int* status) {\n"
+            f"  nep::spans_direct<{ctype}>((const {ctype}*)lengths, n, spans, status);\n}}\n")
     return "\n".join(parts)
 
 
