@@ -155,3 +155,49 @@ def test_ragged_l2_exact_division_of_tiny_and_huge_norms():
     norm = x.square().sum(-1, True).sqrt().clamp_min(1e-6)
     assert torch.equal(got[1], torch.zeros(width)) and torch.equal(got[0], torch.zeros(width))
     assert _ulps(got[2:], (x / norm)[2:], torch.float32) <= 8
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("name", ["logsumexp", "softcap_lse", "stable_l2", "rmsnorm_max", "linear_attn"])
+def test_few_long_rows(name, dtype):
+    """Few rows over up to 1024 lanes and 16 wavefronts each, aligned and ragged."""
+    params = {"rmsnorm_max": {"eps": 1e-6}, "softcap_lse": {"beta": 0.5}}.get(name, {})
+    for rows, width, offset in ((1, 65536, 0), (3, 65537, 1), (16, 8192, 0), (2, 262144, 0)):
+        x, dev = _rows(rows, width, dtype, offset, 0)
+        if name == "linear_attn":
+            x = x.abs()          # a signed sum cancels: its relative error is not bounded
+            dev.copy_(x)
+        print(f"few rows {name} {dtype} {rows}x{width}+{offset}", flush=True)
+        got = CG.run(name, dev, **params).cpu().float()
+        rtol, atol = TOL[dtype]
+        torch.testing.assert_close(got, R.reference(name, x, **params), rtol=rtol, atol=atol)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("name", ["variance", "std"])
+def test_two_pass_rows_held_and_read_twice(name, dtype):
+    """Rows around the widest that 1024 lanes hold (8 and 16 slots each), and wider ones."""
+    top = 65536 if dtype == torch.float32 else 131072
+    for width, offset in ((top // 2, 0), (top // 2 + 1, 1), (top, 0), (top - 1, 3), (top + 8, 0),
+                          (2 * top + 5, 0)):
+        x, dev = _rows(3, width, dtype, offset, 0)
+        _say(f"two-pass {name} {dtype} width={width} offset={offset}")
+        got = CG.run(name, dev).cpu().float()
+        rtol, atol = TOL[dtype]
+        torch.testing.assert_close(got, R.reference(name, x), rtol=rtol, atol=atol)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_log_softmax_rows_of_16_slots(dtype):
+    """Rows that 1024 lanes hold with up to 16 slots each, with NaN and +inf rows among them."""
+    top = 65536 if dtype == torch.float32 else 131072
+    for width, offset in ((top // 2 + 8, 0), (top, 0), (top - 3, 1)):
+        x, dev = _rows(4, width, dtype, offset, 0)
+        x[1, width // 3] = float("inf")
+        x[2, width - 1] = float("nan")
+        dev.copy_(x)
+        _say(f"log_softmax 16 slots {dtype} width={width} offset={offset}")
+        got = CG.run_log_softmax(dev).cpu().float()
+        rtol, atol = TOL[dtype]
+        torch.testing.assert_close(got[::3], torch.log_softmax(x[::3].float(), -1), rtol=rtol, atol=atol)
+        assert torch.isnan(got[1:3]).all()
