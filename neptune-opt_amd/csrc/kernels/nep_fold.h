@@ -311,7 +311,8 @@ __device__ __forceinline__ float finalize_state(const State& s, float n) {
 }
 
 // ---------------------------------------------------------------- fast exponential path
-template <class St, int TPR, int UNROLL, int VECTOR>
+// CACHED: for a row that is read again, so that its second reading finds it in the caches.
+template <class St, int TPR, int UNROLL, int VECTOR, bool CACHED = false>
 __device__ __forceinline__ void load_raw(RawTile<St, UNROLL, VECTOR>& r,
                                          const typename St::T* row, i64 stride_col, i64 tile,
                                          i64 c1, int t) {
@@ -323,8 +324,9 @@ __device__ __forceinline__ void load_raw(RawTile<St, UNROLL, VECTOR>& r,
     if constexpr (VECTOR) {
       // a uniform base plus a 32-bit lane offset (the tile is below 2^31 elements)
       const u32 f = St::kNegInfWord;
-      r.w[u] = r.ok[u] ? load16(row + tile + (u32)((u * TPR + t) * TL::VEC))
-                       : u32x4{f, f, f, f};
+      const typename St::T* p = row + tile + (u32)((u * TPR + t) * TL::VEC);
+      if constexpr (CACHED) r.w[u] = r.ok[u] ? load16_cached(p) : u32x4{f, f, f, f};
+      else r.w[u] = r.ok[u] ? load16(p) : u32x4{f, f, f, f};
     } else {
       r.s[u] = r.ok[u] ? St::load(row + e * stride_col) : -kInf;
     }
@@ -440,11 +442,12 @@ __device__ __forceinline__ LogLane log_row_lane(const typename St::T* row, i64 s
   typename Span<St, TPR, VECTOR>::Rest rest;   // issued first: its latency is the first tile's
   if constexpr (VECTOR == kRagged) sp.load_rest(rest, row, t);
   RawTile<St, UNROLL, VECTOR> cur;
-  load_raw<St, TPR, UNROLL, VECTOR>(cur, row, stride_col, sp.v0, sp.v1, t);
+  load_raw<St, TPR, UNROLL, VECTOR, CENTERED>(cur, row, stride_col, sp.v0, sp.v1, t);
   for (i64 tile = sp.v0; tile < sp.v1; tile += TL::TILE) {
     RawTile<St, UNROLL, VECTOR> nxt;
     const bool more = tile + TL::TILE < sp.v1;
-    if (more) load_raw<St, TPR, UNROLL, VECTOR>(nxt, row, stride_col, tile + TL::TILE, sp.v1, t);
+    if (more)
+      load_raw<St, TPR, UNROLL, VECTOR, CENTERED>(nxt, row, stride_col, tile + TL::TILE, sp.v1, t);
     log_fold_tile<F, St, TPR, UNROLL, VECTOR, CENTERED>(s, cur, n);
     if (more) cur = nxt;
   }
@@ -764,13 +767,73 @@ __device__ __forceinline__ void fold_split_merge(const float* __restrict__ pm,
   if (live && lane == 0) St::store(out + row, finalize_state<F>(s, (float)ncols));
 }
 
+// A raw tile that lies in [v0, v1) whole: loads without per-slot bounds.
+template <class St, int TPR, int UNROLL, int VECTOR, bool CACHED>
+__device__ __forceinline__ void load_whole(RawTile<St, UNROLL, VECTOR>& r,
+                                           const typename St::T* row, i64 stride_col, i64 tile,
+                                           int t) {
+  typedef Tiles<St, TPR, UNROLL, VECTOR> TL;
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u) {
+    r.ok[u] = true;
+    if constexpr (VECTOR) {
+      const typename St::T* p = row + tile + (u32)((u * TPR + t) * TL::VEC);
+      if constexpr (CACHED) r.w[u] = load16_cached(p);
+      else r.w[u] = load16(p);
+    } else {
+      r.s[u] = St::load(row + (tile + u * TPR + t) * stride_col);
+    }
+  }
+}
+
+// fn(element) over the valid elements of a raw tile.
+template <class St, int UNROLL, int VECTOR, class F>
+__device__ __forceinline__ void each(const RawTile<St, UNROLL, VECTOR>& r, F fn) {
+  constexpr int VEC = VECTOR ? St::kVec : 1;
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u) {
+    if (!r.ok[u]) continue;
+    float v[VEC];
+    if constexpr (VECTOR) St::unpack(r.w[u], v);
+    else v[0] = r.s[u];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) fn(v[j]);
+  }
+}
+
+// fn over one lane's elements of the vectors of a row, the next tile's loads in flight while this
+// one's are used.
+template <class St, int TPR, int UNROLL, int VECTOR, bool CACHED, class F>
+__device__ __forceinline__ void each_of_row(const typename St::T* row, i64 stride_col, i64 v0,
+                                            i64 v1, int t, F fn) {
+  constexpr i64 TILE = Tiles<St, TPR, UNROLL, VECTOR>::TILE;
+  RawTile<St, UNROLL, VECTOR> cur, nxt;
+  i64 tile = v0;
+  if (tile + TILE <= v1) {
+    load_whole<St, TPR, UNROLL, VECTOR, CACHED>(cur, row, stride_col, tile, t);
+    for (; tile + 2 * TILE <= v1; tile += TILE) {
+      load_whole<St, TPR, UNROLL, VECTOR, CACHED>(nxt, row, stride_col, tile + TILE, t);
+      each(cur, fn);
+      cur = nxt;
+    }
+    each(cur, fn);
+    tile += TILE;
+  }
+  if (tile < v1) {
+    load_raw<St, TPR, UNROLL, VECTOR, CACHED>(cur, row, stride_col, tile, v1, t);
+    each(cur, fn);
+  }
+}
+
 // Two-pass plan (template.py:62-103): pass 1 reduces the producer over the row, pass 2 the
-// term with the producer held constant.  The second pass re-reads the row.
-template <class F, class St, int TPR, int UNROLL, int VECTOR, int WG>
+// term with the producer held constant.  RESIDENT: the row fits in one tile (host) and stays in
+// registers as raw words, so it crosses HBM once; otherwise the second pass reads it again,
+// through the caches where it still is there.  The two are separate kernels so that each is
+// allocated the registers of its own path.
+template <class F, class St, int TPR, int UNROLL, int VECTOR, int WG, bool RESIDENT>
 __device__ __forceinline__ void fold_two_pass(const typename St::T* __restrict__ x,
                                               typename St::T* __restrict__ out, i64 rows,
                                               i64 ncols, i64 stride_row, i64 stride_col) {
-  typedef Tiles<St, TPR, UNROLL, VECTOR> TL;
   typedef RowComm<TPR> RC;
   constexpr int RPW = WG / TPR;
   __shared__ float lds[WG / 64];
@@ -781,51 +844,30 @@ __device__ __forceinline__ void fold_two_pass(const typename St::T* __restrict__
   const i64 c1 = live ? ncols : 0;
   const float n = (float)ncols;
   const int wave = threadIdx.x >> 6, first = (wave / RC::WPR) * RC::WPR;
-  // A row that fits in one tile stays in registers: pass 2 reads what pass 1 loaded, so the
-  // row crosses HBM once (same values, same order as reading it twice).
   const Span<St, TPR, VECTOR> sp(rp, 0, c1);
-  constexpr int RU = Span<St, TPR, VECTOR>::RU;
-  const bool resident = ncols <= TL::TILE;
-  float keep[TL::K];
-  bool kept[UNROLL];
-  // a ragged row's last elements, held from here to the second pass
+  RawTile<St, RESIDENT ? UNROLL : 1, VECTOR> keep;
+  // a ragged row's other elements, held from here to the second pass
   typename Span<St, TPR, VECTOR>::Rest rest;
   if constexpr (VECTOR == kRagged) sp.load_rest(rest, rp, t);
   // pass 1: the producer
   float m = F::kProducerSum ? 0.0f : -kInf;
-  if (resident) {
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      kept[u] = TL::load_slot(rp, stride_col, sp.v0, sp.v1, t, u, keep);
-      if (!kept[u]) continue;
-#pragma unroll
-      for (int j = 0; j < TL::VEC; ++j) {
-        const float o = F::phi(keep[u * TL::VEC + j], n);
-        m = F::kProducerSum ? (m + o) : __builtin_fmaxf(m, o);
-      }
-    }
+  auto produce = [&](float v) {
+    const float o = F::phi(v, n);
+    m = F::kProducerSum ? (m + o) : __builtin_fmaxf(m, o);
+  };
+  if constexpr (RESIDENT) {
+    if (sp.v1 - sp.v0 == Tiles<St, TPR, UNROLL, VECTOR>::TILE)
+      load_whole<St, TPR, UNROLL, VECTOR, false>(keep, rp, stride_col, sp.v0, t);
+    else
+      load_raw<St, TPR, UNROLL, VECTOR>(keep, rp, stride_col, sp.v0, sp.v1, t);
+    each(keep, produce);
+    // 16-bit rows of many slots are unpacked again in the second pass instead of being held as
+    // fp32 in between, which would leave one workgroup per CU (or spill, with 16 slots)
+    if constexpr (UNROLL * Tiles<St, TPR, UNROLL, VECTOR>::VEC > (TPR >= 1024 ? 64 : 32)) reopen(keep);
   } else {
-    for (i64 tile = sp.v0; tile < sp.v1; tile += TL::TILE) {
-      float v[TL::K];
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        if (!TL::load_slot(rp, stride_col, tile, sp.v1, t, u, v)) continue;
-#pragma unroll
-        for (int j = 0; j < TL::VEC; ++j) {
-          const float o = F::phi(v[u * TL::VEC + j], n);
-          m = F::kProducerSum ? (m + o) : __builtin_fmaxf(m, o);
-        }
-      }
-    }
+    each_of_row<St, TPR, UNROLL, VECTOR, true>(rp, stride_col, sp.v0, sp.v1, t, produce);
   }
-  if constexpr (VECTOR == kRagged) {
-#pragma unroll
-    for (int u = 0; u < RU; ++u) {
-      if (!rest.ok[u]) continue;
-      const float o = F::phi(rest.s[u], n);
-      m = F::kProducerSum ? (m + o) : __builtin_fmaxf(m, o);
-    }
-  }
+  if constexpr (VECTOR == kRagged) each(rest, produce);
   m = F::kProducerSum ? group_sum<RC::G>(m) : group_max<RC::G>(m);
   if constexpr (RC::WPR > 1) {
     if (lane_id() == 0) lds[wave] = m;
@@ -839,38 +881,16 @@ __device__ __forceinline__ void fold_two_pass(const typename St::T* __restrict__
   }
   // pass 2: the term at the final producer value
   float acc = consumer_init<F>();
-  if (resident) {
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      if (!kept[u]) continue;
-#pragma unroll
-      for (int j = 0; j < TL::VEC; ++j) {
-        const float tv = F::term(keep[u * TL::VEC + j], m, n);
-        acc = F::kConsumerMax ? __builtin_fmaxf(acc, tv) : (acc + tv);
-      }
-    }
+  auto consume = [&](float v) {
+    const float tv = F::term(v, m, n);
+    acc = F::kConsumerMax ? __builtin_fmaxf(acc, tv) : (acc + tv);
+  };
+  if constexpr (RESIDENT) {
+    each(keep, consume);
   } else {
-    for (i64 tile = sp.v0; tile < sp.v1; tile += TL::TILE) {
-      float v[TL::K];
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        if (!TL::load_slot(rp, stride_col, tile, sp.v1, t, u, v)) continue;
-#pragma unroll
-        for (int j = 0; j < TL::VEC; ++j) {
-          const float tv = F::term(v[u * TL::VEC + j], m, n);
-          acc = F::kConsumerMax ? __builtin_fmaxf(acc, tv) : (acc + tv);
-        }
-      }
-    }
+    each_of_row<St, TPR, UNROLL, VECTOR, false>(rp, stride_col, sp.v0, sp.v1, t, consume);
   }
-  if constexpr (VECTOR == kRagged) {
-#pragma unroll
-    for (int u = 0; u < RU; ++u) {
-      if (!rest.ok[u]) continue;
-      const float tv = F::term(rest.s[u], m, n);
-      acc = F::kConsumerMax ? __builtin_fmaxf(acc, tv) : (acc + tv);
-    }
-  }
+  if constexpr (VECTOR == kRagged) each(rest, consume);
   acc = F::kConsumerMax ? group_max<RC::G>(acc) : group_sum<RC::G>(acc);
   if constexpr (RC::WPR > 1) {
     if (lane_id() == 0) lds[wave] = acc;

@@ -212,6 +212,7 @@ class FoldVariant:
     unroll: int = 4     # slots per lane per tile
     waves: int = 4      # wave64s per workgroup (at least one row)
     ragged: bool = False    # vector rows of any alignment and width (nep_device.h kRagged)
+    resident: bool = False  # two-pass folds: one tile holds the row, which stays in registers
 
     @property
     def wg(self) -> int:
@@ -223,7 +224,7 @@ class FoldVariant:
 
     def tag(self) -> str:
         return (f"{dtype_tag(self.dtype)[0]}_{access_tag(self.vector, self.ragged)}{self.tpr}"
-                f"u{self.unroll}w{self.waves}")
+                f"u{self.unroll}w{self.waves}{'k' if self.resident else ''}")
 
 
 _FOLD_ARGS_SERIAL = ("const void* x, void* out, long long rows, long long ncols, "
@@ -241,7 +242,7 @@ def _fold_kernel(sk: Skeleton, plan: str, part: str, var: FoldVariant) -> tuple[
         sig = _FOLD_ARGS_SERIAL
     elif plan == "two_pass":
         name = f"{sk.name}_two_pass_{var.tag()}"
-        body = (f"nep::fold_two_pass<{tmpl}>((const {st}::T*)x, ({st}::T*)out, rows, ncols, "
+        body = (f"nep::fold_two_pass<{tmpl}, {str(var.resident).lower()}>((const {st}::T*)x, ({st}::T*)out, rows, ncols, "
                 "stride_row, stride_col);")
         sig = _FOLD_ARGS_SERIAL
     elif part == "partial":
@@ -332,7 +333,8 @@ def emit_readout_source(sk: Skeleton, values: dict | None = None, *, variants: t
         _, st = dtype_tag(var.dtype)
         for resident in (True, False):
             name = readout_kernel_name(sk, var, nan_posinf_rows, resident)
-            if name in seen:
+            # more than 8 slots per lane are only ever taken by rows they hold
+            if name in seen or (var.unroll > 8 and not resident):
                 continue
             seen.add(name)
             parts.append(

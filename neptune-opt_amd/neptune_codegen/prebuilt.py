@@ -5,6 +5,8 @@ tensors (data pointer 0, always aligned) reproduce the variants a real launch pi
 """
 from __future__ import annotations
 
+import dataclasses
+
 
 def _fold_programs():
     import torch
@@ -29,9 +31,10 @@ def _fold_programs():
         params = {**param_defaults(name), **({"eps": 1e-6} if name == "rmsnorm_max" else {})}
         prog = compile_skeleton(name, params)
         sk = prog.sk
-        out.append(prog.program(_fold_variant(x2, 4096, block, warps, resident=sk.two_pass,
-                                              merge_heavy=not sk.is_log and not sk.two_pass,
-                                              heavy_phi=prog.heavy_phi)))
+        var = _fold_variant(x2, 4096, block, warps, resident=sk.two_pass,
+                            merge_heavy=not sk.is_log and not sk.two_pass,
+                            heavy_phi=prog.heavy_phi)
+        out.append(prog.program(dataclasses.replace(var, resident=sk.two_pass)))
     from neptune_codegen.template import compile_readout
 
     xw = torch.empty((16384, 32000), device="meta", dtype=torch.bfloat16)

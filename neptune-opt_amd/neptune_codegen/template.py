@@ -24,6 +24,8 @@ from neptune_codegen.emitters import (BASE_OPTIONS, NO_CONTRACT, FoldVariant, Ro
 from neptune_codegen.skeleton import SKELETONS, all_registered, param_defaults
 
 MAX_SPLIT_PARTS = 4096
+# Slots per lane of a row held in registers by 1024 lanes: 64 VGPRs of the 128 such a lane has.
+RESIDENT_UNROLL = 16
 _CACHE: dict = {}
 _STATE_CACHE: dict = {}
 _STATE_SEEN: dict = {}
@@ -357,7 +359,9 @@ def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: in
             unroll *= 2
         while tpr * unroll * per_slot < ncols and tpr < MAX_TPR:
             tpr *= 2
-    if per_slot == 8 and (merge_heavy or resident) and not split_block and tpr == 64:
+        if unroll * tpr * per_slot < ncols <= RESIDENT_UNROLL * tpr * per_slot and vector:
+            unroll = RESIDENT_UNROLL
+    if per_slot == 8 and (merge_heavy or resident) and not split_block and tpr == 64 and slots >= 256:
         waves = 1              # one row per 64-lane workgroup (bf16 8192 wide: 54.0 -> 48.7 us)
     if not split_block and type(ncols) is int:
         # as many tiles as before, each with no more slots than the row needs
