@@ -197,7 +197,8 @@ def _fold_plan(bh, sq, sk, head_dim, causal):
 def _short_wins(bh: int, sq: int, sk: int, head_dim: int, causal: bool) -> bool:
     """Whether the short-query kernels run a call: always up to 16 queries; beyond, where they are
     estimated 15% cheaper (bf16 causal B*H=8 s=512 13.3 us against 17.5, d=256 causal B*H=16 s=100
-    9.8 against 18.4; B*H=96 s=1000 d=64 full 34 against 21)."""
+    9.8 against 18.4; B*H=12 s=1000 d=64 full 34 against 21; B*H=160 sq=35 sk=5120 196 against
+    189 on 256-query blocks)."""
     if sq <= SHORT_MAX_SQ:
         return True
     seen = min(sq, sk) if causal else sk
@@ -205,9 +206,11 @@ def _short_wins(bh: int, sq: int, sk: int, head_dim: int, causal: bool) -> bool:
             + bh * seen * head_dim * 4 / PACK_BYTES_PER_US)
     units = bh * -(-sq // ATTN_SHORT_BLOCK_M)
     chunks, per = short_chunks(units, seen)
-    short = (SHORT_LAUNCH_US + -(-units * chunks // SHORT_RESIDENT[head_dim])
-             * (SHORT_BLOCK_US + -(-per // ATTN_SHORT_WAVES) * SHORT_PASS_US[head_dim])
-             + (MERGE_US if chunks > 1 else 0.0))
+    wait = (SHORT_LAUNCH_US + -(-units * chunks // SHORT_RESIDENT[head_dim])
+            * (SHORT_BLOCK_US + -(-per // ATTN_SHORT_WAVES) * SHORT_PASS_US[head_dim]))
+    # a full chip passes a 32-key tile per CU in SHORT_TILE_US at head dim 128, whatever is resident
+    busy = units * -(-seen // ATTN_SHORT_TILE) / CUS * SHORT_TILE_US * head_dim / 128
+    short = max(wait, busy) + (MERGE_US if chunks > 1 else 0.0)
     return 1.15 * short < fold
 
 
@@ -273,7 +276,8 @@ def _seen_key(q, k, v, scale, causal, return_lse):
     """Key of a call on plain strided device tensors, or None where the call takes the full path."""
     import torch
 
-    if hip.recording_active():
+    # a scale whose printed form may not be its value (a tensor) takes the full path
+    if hip.recording_active() or not (scale is None or type(scale) in (int, float)):
         return None
     key = [type(scale).__name__, repr(scale), bool(causal), bool(return_lse)]
     for t in (q, k, v):

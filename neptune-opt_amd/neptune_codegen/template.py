@@ -182,7 +182,8 @@ def _fold_seen_key(x, options: tuple, params: dict):
     import torch
 
     if (type(x) is not torch.Tensor or not x.is_cuda or x.layout != torch.strided
-            or hip.recording_active()):
+            or hip.recording_active()
+            or params and any(type(v) not in (int, float, bool) for v in params.values())):
         return None
     try:
         key = options + (x.dtype, x.device, x.shape, x.stride(), x.data_ptr() % 16,
