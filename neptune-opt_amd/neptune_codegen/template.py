@@ -164,7 +164,7 @@ def launch_readout(program: ReadoutProgram, x2, out, rows, ncols, block, num_war
     import torch
 
     device = x2.device.index if x2.device.index is not None else torch.cuda.current_device()
-    var = _fold_variant(x2, ncols, block, num_warps, resident=True)
+    var = _fold_variant(x2, ncols, block, num_warps, resident=True, readout=True)
     rpw = max(1, var.wg // var.tpr)
     kernel = program.kernel(var, device, resident=ncols <= readout_tile(var))
     grid, tail = (_grid_1d(rows, rpw),), (rows, ncols, x2.stride(0), x2.stride(1))
@@ -294,7 +294,7 @@ def _is_ragged(x2, ncols: int, vec: int) -> bool:
 
 def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: int = 0,
                   resident: bool = False, merge_heavy: bool = False,
-                  heavy_phi: bool = False) -> FoldVariant:
+                  heavy_phi: bool = False, readout: bool = False) -> FoldVariant:
     """Launch shape: 16-byte loads when the layout allows, lanes per row from BLOCK (a tile
     wider than the workgroup's lanes gives each lane up to MAX_UNROLL slots first), workgroup =
     max(64 * num_warps, lanes per row).  Three fold classes then adjust it (serial plan only):
@@ -340,7 +340,9 @@ def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: in
     per_slot = vec if vector else 1
     if merge_heavy and not split_block and per_slot == 8:
         # 16-bit rows: at most one wavefront per row, several short tiles per lane
-        tpr = min(64, max(16, 1 << max(0, (max(1, ncols // 128) - 1).bit_length())))
+        # (at least two slots each: bf16 131072 x 64 12.8 us on 16 lanes, 7.1 on 4)
+        least = min(16, 1 << max(0, (-(-ncols // 16) - 1).bit_length()))
+        tpr = min(64, max(least, 1 << max(0, (max(1, ncols // 128) - 1).bit_length())))
         unroll = MAX_UNROLL if ncols >= WIDE_16BIT_ROW else UNROLL
     elif (merge_heavy or heavy_phi) and not split_block and per_slot == 4:
         # fp32 rows: 8 slots per lane on the same lanes, then lanes given up while a tile would
@@ -352,7 +354,17 @@ def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: in
         while tpr > 64 and unroll < MAX_UNROLL:
             tpr //= 2
             unroll *= 2
-    if resident and not split_block:
+    slots = -(-ncols // per_slot) if type(ncols) is int else 256
+    if (resident and vector and not split_block and slots < 256 and x2.shape[0] >= 8
+            and (readout or per_slot == 8)):
+        # Short rows: 1 slot per lane up to 8 slots, else 2 or 3, whichever idles fewer lanes (the
+        # shape below is one generation of wavefronts that loads, then stores).  60 MB, cold:
+        # log_softmax bf16 131072 x 64 17.9 -> 8.4 us, x 200 31.4 -> 21.9, 30000 x 1000 24.3 ->
+        # 21.8, fp32 131072 x 64 16.7 -> 12.9, 75000 x 200 24.9 -> 21.5; variance bf16 131072 x 64
+        # 8.1 -> 5.7 (fp32 75000 x 200 11.8 -> 12.4: two-pass fp32 rows keep their shape).
+        unroll = 1 if slots <= 8 else min((2, 3), key=lambda n: n << max(0, (-(-slots // n) - 1).bit_length()))
+        tpr = 1 << max(0, (-(-slots // unroll) - 1).bit_length())
+    elif resident and not split_block:
         if per_slot == 8:      # 16-bit rows: lanes first (up to 512), then slots
             unroll = UNROLL
             tpr = min(512, 1 << max(0, (-(-ncols // (UNROLL * per_slot)) - 1).bit_length()))
@@ -622,6 +634,15 @@ def _row_variant(flat, gamma, width: int, *, tile: int | None = None) -> RowVari
     width 8192: 4 slots 87.4 / 88.6, 8 slots 89.0 / 90.5;
     width 16384: 8 slots 88.4 / 89.0, 4 slots 89.0 / 88.9.
 
+    Rows of fewer than 256 slots take the 2 to 5 slots per lane that leave the fewest lanes idle
+    (ragged 16-bit rows 2 to 4, fp32 ones 2: 30000 x 151 10.1 us, 3 slots 10.5, one element per load 10.9), rows of up to 8 slots one: with 8 a wavefront holds so many rows that a whole input is
+    one generation of wavefronts, which loads, then stores.  64 MB inputs, cold, RMSNorm /
+    L2-normalize: bf16 131072 x 64 38.4 / 38.8 -> 9.6 / 8.2 us, x 128 33.3 / 37.3 -> 13.8 / 13.5,
+    32000 x 1000 29.3 / 31.7 -> 24.1 / 23.9; fp32 131072 x
+    64 31.2 / 34.3 -> 13.6 / 13.5, 62500 x 256 24.9 / 24.9 -> 23.3 / 23.7.  fp32 rows of 512 to
+    1024 slots take 4 (7812 x 2048 24.7 / 25.3 -> 23.9 / 23.6).  Fewer than 8 rows are one or two
+    workgroups whichever way and keep the shape above.
+
     Ragged rows (nep_device.h Span; gamma of unit stride, any alignment) take 2 slots in fp32 and
     4 in 16 bits, 8 above 4096 elements: fp32 L2 20000 x 2999 78.7 us (3 slots 82.0, 6 84.4),
     bf16 RMSNorm 32768 x 1001 27.3 (2 slots 27.2, 8 32.0), fp16 8192 x 8191 50.3 (4 slots 54.4).
@@ -641,6 +662,14 @@ def _row_variant(flat, gamma, width: int, *, tile: int | None = None) -> RowVari
         nv = 4 if slots >= 256 else 2
     if ragged:
         nv = 2 if vec == 4 else (4 if slots <= 512 else 8)
+    if vector and (ragged or flat.shape[0] >= 8):
+        if slots <= 8:
+            nv = 1
+        elif slots < 256 and not (ragged and vec == 4):
+            nv = min((2, 3, 4) if ragged else (2, 3, 4, 5),
+                     key=lambda n: n << max(0, (-(-slots // n) - 1).bit_length()))
+        elif vec == 4 and 512 <= slots <= 1024 and not ragged:
+            nv = 4
     if tile is not None:
         nv = 2 if vector else 8
     tpr = 1 << max(0, (max(1, -(-slots // nv)) - 1).bit_length())
