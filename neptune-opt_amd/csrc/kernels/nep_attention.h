@@ -398,12 +398,13 @@ __device__ void attention_exact_rows(const T* __restrict__ qp, const T* __restri
 
 // kAttnWaves wave64s of 32 queries: 8 share each staged tile among most queries, 4 make twice the
 // workgroups where 8 leave CUs idle or uneven.
-// A head's keys may be split into `parts` of `per` tiles: each workgroup takes one part of one
+// PARTS: a head's keys are split into `parts` of `per` tiles: each workgroup takes one part of one
 // query block, and a block that has more than one part leaves its unnormalised fp32 state
 // (O, m, l) for attention_parts_merge (causal blocks differ in their parts).  Both are for calls
 // whose time is their longest workgroup's: bf16 full, 36 heads x 100 queries x 4000 keys, d=128
 // 108 us with 8 waves, 92 with 4, 44 in 6 parts; causal, 8 heads x 4096 103, 84, 63.
-template <typename T, int D, bool CAUSAL, int kAttnWaves>
+// (Its own kernel: the part's bounds in the unsplit loop cost head dim 256 causal 5%.)
+template <typename T, int D, bool CAUSAL, int kAttnWaves, bool PARTS>
 __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* __restrict__ k,
                                               const u16* __restrict__ vt,
                                               const int* __restrict__ exps,
@@ -432,16 +433,17 @@ __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* 
   __shared__ __attribute__((aligned(1024))) unsigned char vbuf1[TILE];
 
   const int nqb = (sq + kAttnBM - 1) / kAttnBM;
-  const int bh_count = gridDim.x / (nqb * parts);
+  const int bh_count = gridDim.x / (PARTS ? nqb * parts : nqb);
   const int id = blockIdx.x / bh_count;
-  const int qb = nqb - 1 - id / parts;      // heaviest query block first
-  const int part = id % parts;
+  const int qb = nqb - 1 - (PARTS ? id / parts : id);   // heaviest query block first
+  const int part = PARTS ? id % parts : 0;
   const int bh = blockIdx.x % bh_count;
   int kv_end = sk;
   if constexpr (CAUSAL) kv_end = min(sk, (qb + 1) * kAttnBM);
   const int block_tiles = (kv_end + kAttnBN - 1) / kAttnBN;
-  const int t0 = part * per, ntiles = min(block_tiles, t0 + per);
-  if (t0 >= block_tiles) return;            // a causal block with fewer parts
+  const int t0 = PARTS ? part * per : 0;
+  const int ntiles = PARTS ? min(block_tiles, t0 + per) : block_tiles;
+  if (PARTS && t0 >= block_tiles) return;   // a causal block with fewer parts
   const int b = bh / heads, h = bh % heads;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -623,13 +625,19 @@ __device__ __forceinline__ void attention_fwd(const T* __restrict__ q, const T* 
   }
   T* orow0 = o + (i64)bh * sq * D;
   float* lse_row0 = lse != nullptr ? lse + (i64)bh * sq : nullptr;
-  const bool whole = per >= block_tiles;
+  const bool whole = !PARTS || per >= block_tiles;
   const i64 part_row0 = ((i64)part * bh_count + bh) * sq;
   if (exact) {
-    attention_exact_rows<T, D, CAUSAL, kAttnWaves>(
-        qp, kp, v + b * vsb + h * vsh, orow0, lse_row0, sq, sk, q0, qss, kss, vss, scale_log2,
-        t0 * kAttnBN, ntiles * kAttnBN, whole ? nullptr : po + part_row0 * D,
-        whole ? nullptr : pml + 2 * part_row0);
+    if constexpr (PARTS) {
+      attention_exact_rows<T, D, CAUSAL, kAttnWaves>(
+          qp, kp, v + b * vsb + h * vsh, orow0, lse_row0, sq, sk, q0, qss, kss, vss, scale_log2,
+          t0 * kAttnBN, ntiles * kAttnBN, whole ? nullptr : po + part_row0 * D,
+          whole ? nullptr : pml + 2 * part_row0);
+    } else {
+      attention_exact_rows<T, D, CAUSAL, kAttnWaves>(qp, kp, v + b * vsb + h * vsh, orow0,
+                                                     lse_row0, sq, sk, q0, qss, kss, vss,
+                                                     scale_log2);
+    }
     return;
   }
   if (!whole) {

@@ -69,15 +69,15 @@ def use_w64(head_dim: int, causal: bool, sq: int, sk: int) -> bool:
 
 
 def _program(head_dim: int, causal: bool, dtype="bfloat16", w64: bool | None = None,
-             waves: int | None = None) -> hip.Program:
+             waves: int | None = None, parts: bool = False) -> hip.Program:
     w64 = attention_w64(head_dim, w64)
-    key = (head_dim, causal, str(dtype), w64, waves)
+    key = (head_dim, causal, str(dtype), w64, waves, parts)
     with _lock:
         prog = _PROGRAMS.get(key)
         if prog is None:
-            prog = hip.Program(emit_attention_source(head_dim, causal, dtype, w64=w64, waves=waves),
-                               f"{attention_kernel_name(head_dim, causal, dtype, w64, waves)}.hip",
-                               BASE_OPTIONS)
+            name = attention_kernel_name(head_dim, causal, dtype, w64, waves, parts)
+            prog = hip.Program(emit_attention_source(head_dim, causal, dtype, w64=w64, waves=waves,
+                                                     parts=parts), f"{name}.hip", BASE_OPTIONS)
             _PROGRAMS[key] = prog
         return prog
 
@@ -454,15 +454,7 @@ def _launch_fold(q, k, v, scale, causal, return_lse, e_max, w64=None, waves=None
     # V^T tile images (fp16, MFMA operand order) and one power-of-two exponent per tile
     call.exps = B * H * ntiles * D * BLOCK_N * 2
     call.nbytes = call.exps + B * H * ntiles * 4
-    prog = _program(D, causal, q.dtype, w64, waves)
-    pack = prog.kernel(attention_pack_kernel_name(D, q.dtype),
-                       (hip.PTR,) * 3 + (hip.I32,) * 2 + (hip.I64,) * 3, 256, device)
-    call.pack = (pack, (B * H * ntiles,), (H, Sk, v.stride(0), v.stride(1), v.stride(2)))
     w64 = attention_w64(D, w64)
-    name = attention_kernel_name(D, causal, q.dtype, w64, waves)
-    fold = prog.kernel(name, (hip.PTR,) * 7 + (hip.I32,) * 3 + (hip.I64,) * 9 + (hip.I32, hip.F32)
-                       + (() if w64 else (hip.PTR,) * 2 + (hip.I32,) * 2),
-                       attention_fold_threads(D, w64, waves), device)
     bm = attention_block_m(D, w64, waves)
     nqb = (Sq + bm - 1) // bm
     parts, rows = 1, B * H * Sq
@@ -470,10 +462,18 @@ def _launch_fold(q, k, v, scale, causal, return_lse, e_max, w64=None, waves=None
         most = -(-(min(Sk, nqb * bm) if causal else Sk) // BLOCK_N)   # tiles of the longest block
         per = min(per or most, most)
         parts = -(-most // per)
+    prog = _program(D, causal, q.dtype, w64, waves, parts > 1)
+    pack = prog.kernel(attention_pack_kernel_name(D, q.dtype),
+                       (hip.PTR,) * 3 + (hip.I32,) * 2 + (hip.I64,) * 3, 256, device)
+    call.pack = (pack, (B * H * ntiles,), (H, Sk, v.stride(0), v.stride(1), v.stride(2)))
+    name = attention_kernel_name(D, causal, q.dtype, w64, waves, parts > 1)
+    fold = prog.kernel(name, (hip.PTR,) * 7 + (hip.I32,) * 3 + (hip.I64,) * 9 + (hip.I32, hip.F32)
+                       + ((hip.PTR,) * 2 + (hip.I32,) * 2 if parts > 1 else ()),
+                       attention_fold_threads(D, w64, waves), device)
     call.fold = (fold, (nqb * B * H * parts,),
                  (H, Sq, Sk, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1),
                   k.stride(2), v.stride(0), v.stride(1), v.stride(2), int(e_max), scale * LOG2E),
-                 () if w64 else (parts, per))
+                 (parts, per) if parts > 1 else ())
     if parts > 1:
         call.add_state(parts, rows, D)
         merge = prog.kernel(name + "_merge", (hip.PTR,) * 4 + (hip.I64,) + (hip.I32,) * 3, 256, device)

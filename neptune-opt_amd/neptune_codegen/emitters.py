@@ -598,7 +598,7 @@ def _attn_dtype(dtype) -> tuple[str, str]:
 
 def emit_attention_source(head_dim: int, causal: bool, dtype="bfloat16",
                           waves_per_eu: int | None = None, w64: bool | None = None,
-                          waves: int | None = None) -> str:
+                          waves: int | None = None, parts: bool = False) -> str:
     """hiprtc unit of the online-softmax attention fold (no reference counterpart): the
     logsumexp repair exp(s - s2) applied per key tile to (m, l, O).  Holds two kernels: the
     V^T tile packer and the fold itself (with its exact fallback for out-of-range V)."""
@@ -609,7 +609,7 @@ def emit_attention_source(head_dim: int, causal: bool, dtype="bfloat16",
     wpe = (2 if head_dim <= 128 and not w64 else 1) if waves_per_eu is None else waves_per_eu
     threads = attention_fold_threads(head_dim, w64, waves)
     tag, ctype = _attn_dtype(dtype)
-    name = attention_kernel_name(head_dim, causal, dtype, w64, waves)
+    name = attention_kernel_name(head_dim, causal, dtype, w64, waves, parts)
     pack = attention_pack_kernel_name(head_dim, dtype)
     cz = "true" if causal else "false"
     if w64:
@@ -619,14 +619,16 @@ def emit_attention_source(head_dim: int, causal: bool, dtype="bfloat16",
         more, merge = ("", ""), ""
     else:
         prefix = ""
-        more = (", float* po, float* pml, int parts, int per", ", po, pml, parts, per")
-        bm = attention_block_m(head_dim, False, waves)
-        merge = (f'extern "C" __global__ void __launch_bounds__(256) {name}_merge(const float* po, '
-                 "const float* pml, void* o, float* lse, long long rows, int sq, int sk, int per) {\n"
-                 f"  nep::attention_parts_merge<{ctype}, {head_dim}, {cz}, {bm}>(po, pml, ({ctype}*)o, "
-                 "lse, rows, sq, sk, per);\n}\n")
+        more, merge = ("", ", nullptr, nullptr, 1, 0"), ""
+        if parts:
+            more = (", float* po, float* pml, int parts, int per", ", po, pml, parts, per")
+            bm = attention_block_m(head_dim, False, waves)
+            merge = (f'extern "C" __global__ void __launch_bounds__(256) {name}_merge(const float* po, '
+                     "const float* pml, void* o, float* lse, long long rows, int sq, int sk, int per) {\n"
+                     f"  nep::attention_parts_merge<{ctype}, {head_dim}, {cz}, {bm}>(po, pml, "
+                     f"({ctype}*)o, lse, rows, sq, sk, per);\n}}\n")
         call = (f"  nep::attention_fwd<{ctype}, {head_dim}, {cz}, "
-                f"{attention_waves(head_dim, False, waves)}>(")
+                f"{attention_waves(head_dim, False, waves)}, {str(parts).lower()}>(")
     return "\n".join([
         "// AUTO-GENERATED by neptune_codegen (HIP emitter) -- do not edit.\n"
         f"// online-softmax attention fold: head_dim={head_dim}, causal={causal}, {tag} inputs; "
@@ -647,13 +649,15 @@ def emit_attention_source(head_dim: int, causal: bool, dtype="bfloat16",
 
 
 def attention_kernel_name(head_dim: int, causal: bool, dtype="bfloat16", w64: bool = False,
-                          waves: int | None = None) -> str:
+                          waves: int | None = None, parts: bool = False) -> str:
     """The fold's symbol; the 64-queries-per-wave kernel carries a `_w64` suffix, the 32-query one
-    its waves where they are not the default."""
+    its waves where they are not the default, and `_parts` where it takes parts of the keys."""
     tag, _ = _attn_dtype(dtype)
     suffix = "_w64" if attention_w64(head_dim, w64) and w64 else ""
     if not suffix and waves and waves != attention_waves(head_dim, False):
         suffix = f"_x{waves}"
+    if parts:
+        suffix += "_parts"
     return f"attention_fold_{tag}_d{head_dim}_{'causal' if causal else 'full'}{suffix}"
 
 

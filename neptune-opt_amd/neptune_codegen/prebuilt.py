@@ -85,6 +85,8 @@ def _attention_programs():
             out.append(_program(128, causal, dt, True, 8))
             for dim, waves in ((128, 8), (128, 4), (64, 8), (64, 4), (256, 4)):
                 out.append(_program(dim, causal, dt, False, waves))
+                if waves == 4:
+                    out.append(_program(dim, causal, dt, False, waves, True))
             out += [_short_program(dim, causal, dt) for dim in (64, 128, 256)]
     return out
 
