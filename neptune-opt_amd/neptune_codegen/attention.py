@@ -107,7 +107,8 @@ SHORT_MAX_SQ = 16
 # `short_chunks` takes the cheapest count; against a sweep of 1 to 64 chunks over fourteen shapes
 # it is within 4% of the best but for two (d=64, 4 chunks 25 us for 8 at 20.6; sq=1 sk=8192 B*H=1
 # 12.4 for 10.7).  At B*H=32 sk=32768 1 chunk takes 556 us, 8 take 87 and 64 take 94.
-SHORT_MAX_CHUNKS = 64
+# No split makes more than 4096 workgroups (16 per CU, states of at most 68 MB).
+SHORT_MAX_CHUNKS, SHORT_MAX_WORKGROUPS = 64, 4096
 SHORT_TILE_US, SHORT_MERGE_US, SHORT_CHUNK_US = 0.6, 3.0, 0.05
 CUS = 256
 
@@ -122,7 +123,7 @@ def short_chunks(units: int, sk: int) -> tuple[int, int]:
         return (rounds * -(-tiles // chunks) * SHORT_TILE_US
                 + (SHORT_MERGE_US + chunks * SHORT_CHUNK_US if chunks > 1 else 0.0))
 
-    most = max(1, min(SHORT_MAX_CHUNKS, tiles // ATTN_SHORT_WAVES))
+    most = max(1, min(SHORT_MAX_CHUNKS, tiles // ATTN_SHORT_WAVES, SHORT_MAX_WORKGROUPS // units))
     chunks = min(range(1, most + 1), key=cost)
     per = -(-tiles // chunks)
     return -(-tiles // per), per
@@ -257,7 +258,9 @@ def run_attention(q, k, v, *, scale: float | None = None, causal: bool = True,
     if call is not None:
         out, lse, _ = call.run(q, k, v)
         return (out, lse) if return_lse else out
-    if _takes_short(q, k, causal):
+    if key is None and _is_metadata(q):    # shapes may be symbolic: no launch is chosen
+        out, lse, _, _ = _outputs(q, k, v, scale, return_lse)
+    elif _takes_short(q, k, causal):
         out, lse, call = _launch_short(q, k, v, scale, causal, return_lse)
     else:
         out, lse, _, call, _ = _launch_fold(q, k, v, scale, causal, return_lse, V_EXPONENT_MAX)
@@ -355,12 +358,17 @@ def launch_attention(q, k, v, *, scale: float | None = None, causal: bool = True
     return _launch(q, k, v, scale, causal, return_lse, V_EXPONENT_MAX)
 
 
+def _is_metadata(q) -> bool:
+    from torch._subclasses.fake_tensor import FakeTensor
+
+    return isinstance(q, FakeTensor) or q.device.type == "meta"
+
+
 def _outputs(q, k, v, scale, return_lse):
     """(out, lse or None, scale, whether nothing is to be launched) after validation."""
     import torch
-    from torch._subclasses.fake_tensor import FakeTensor
 
-    metadata = isinstance(q, FakeTensor) or q.device.type == "meta"
+    metadata = _is_metadata(q)
     shape = validate_attention_inputs(q, k, v, metadata=metadata)
     out = torch.empty(shape, dtype=q.dtype, device=q.device)
     lse = torch.empty(shape[:3], dtype=torch.float32, device=q.device) if return_lse else None

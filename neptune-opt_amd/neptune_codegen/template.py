@@ -176,23 +176,25 @@ _RUN_SEEN: dict = {}
 _RUN_SEEN_MAX = 4096
 
 
-def _fold_seen_key(x, options: tuple, params: dict):
-    """Key of a fold or readout call on a plain strided device tensor: everything the validation
-    and the launch choice read; None when the call takes the full path."""
+def _fold_seen(x, options: tuple, params: dict):
+    """(key, launch seen under it or None) of a fold or readout call on a plain strided device
+    tensor: the key is everything the validation and the launch choice read, and None when the
+    call takes the full path."""
     import torch
 
     if (type(x) is not torch.Tensor or not x.is_cuda or x.layout != torch.strided
-            or hip.recording_active()
-            or params and any(type(v) not in (int, float, bool) for v in params.values())):
-        return None
+            or hip.recording_active()):
+        return None, None
+    key = options + (x.dtype, x.device, x.shape, x.stride(), x.data_ptr() % 16)
+    for name in sorted(params):
+        value = params[name]
+        if type(value) not in (int, float, bool):    # its printed form may not be its value
+            return None, None
+        key += (name, type(value), repr(value))
     try:
-        key = options + (x.dtype, x.device, x.shape, x.stride(), x.data_ptr() % 16,
-                         tuple(sorted((k, type(v).__name__, repr(v)) for k, v in params.items()))
-                         if params else ())
-        hash(key)
-    except TypeError:
-        return None
-    return key
+        return key, _RUN_SEEN.get(key)
+    except TypeError:                                # an option that cannot be hashed
+        return None, None
 
 
 def _remember(key, launch) -> None:
@@ -212,8 +214,7 @@ def run_readout(name: str, x, *, nan_posinf_rows: bool = True, block: int | None
     import torch
     from torch._subclasses.fake_tensor import FakeTensor
 
-    seen = _fold_seen_key(x, ("readout", name, bool(nan_posinf_rows), block, num_warps), params)
-    entry = _RUN_SEEN.get(seen) if seen is not None else None
+    seen, entry = _fold_seen(x, ("readout", name, bool(nan_posinf_rows), block, num_warps), params)
     if entry is not None:
         kernel, grid, tail = entry
         out = torch.empty(x.shape, device=x.device, dtype=x.dtype)
@@ -472,24 +473,22 @@ def run(name: str, x, block: int | None = None, num_warps: int | None = None,
 
     from neptune_codegen.skeleton import param_defaults
 
-    seen = _fold_seen_key(x, (name, plan, block, num_warps, keepdim), params)
-    if seen is not None:
-        entry = _RUN_SEEN.get(seen)
-        if entry is not None:
-            out = torch.empty(entry[0], device=x.device, dtype=x.dtype)
-            stream = hip.current_stream(x.device)
-            if plan == "serial":
-                _, kern, grid, tail = entry
-                kern.launch(grid, (x.data_ptr(), out.data_ptr()) + tail, stream)
-                return out
-            _, kp, grid_p, tail_p, km, grid_m, tail_m, count = entry
-            # one allocation holds the four partial arrays (m, acc: fp32; seen, status: int32)
-            parts = torch.empty(4 * count, device=x.device, dtype=torch.float32)
-            base = parts.data_ptr()
-            ptrs = (base, base + 4 * count, base + 8 * count, base + 12 * count)
-            kp.launch(grid_p, (x.data_ptr(),) + ptrs + tail_p, stream)
-            km.launch(grid_m, ptrs + (out.data_ptr(),) + tail_m, stream)
+    seen, entry = _fold_seen(x, (name, plan, block, num_warps, keepdim), params)
+    if entry is not None:
+        out = torch.empty(entry[0], device=x.device, dtype=x.dtype)
+        stream = hip.current_stream(x.device)
+        if plan == "serial":
+            _, kern, grid, tail = entry
+            kern.launch(grid, (x.data_ptr(), out.data_ptr()) + tail, stream)
             return out
+        _, kp, grid_p, tail_p, km, grid_m, tail_m, count = entry
+        # one allocation holds the four partial arrays (m, acc: fp32; seen, status: int32)
+        parts = torch.empty(4 * count, device=x.device, dtype=torch.float32)
+        base = parts.data_ptr()
+        ptrs = (base, base + 4 * count, base + 8 * count, base + 12 * count)
+        kp.launch(grid_p, (x.data_ptr(),) + ptrs + tail_p, stream)
+        km.launch(grid_m, ptrs + (out.data_ptr(),) + tail_m, stream)
+        return out
     metadata = isinstance(x, FakeTensor) or x.device.type == "meta"
     _validate_row_last(x, metadata=metadata)
     params = {**param_defaults(name), **(params or {})}

@@ -34,3 +34,25 @@ def test_fold_choice_is_launchable():
     assert A._fold_choice(128, 4096, 4096, 128, True)[1] == (True, 8, None)
     assert A._fold_choice(36, 100, 4000, 128, False)[1][2] is not None
     assert A._short_wins(1, 16, 1 << 15, 128, False) and not A._short_wins(128, 4096, 4096, 128, True)
+
+
+def test_metadata_calls_choose_no_launch():
+    """Meta and fake tensors, symbolic sizes among them, return shapes only."""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.symbolic_shapes import ShapeEnv
+
+    q = torch.empty(2, 3, 5, 64, dtype=torch.bfloat16, device="meta")
+    out, lse = A.run_attention(q, q, q, causal=False, return_lse=True)
+    assert out.shape == q.shape and lse.shape == q.shape[:3] and lse.dtype == torch.float32
+    mode = FakeTensorMode(shape_env=ShapeEnv())
+    real = torch.empty(2, 3, 40, 64, dtype=torch.bfloat16)
+    fake = mode.from_tensor(real)
+    with mode:
+        assert A.run_attention(fake, fake, fake).shape == real.shape
+
+
+def test_short_chunks_bound_the_scratch():
+    for units in (1, 100, 257, 480, 4096, 4097, 100000):
+        chunks, _ = A.short_chunks(units, 1 << 20)
+        assert chunks == 1 or chunks * units <= A.SHORT_MAX_WORKGROUPS
