@@ -43,6 +43,7 @@ BLOCK_M = 256           # queries per fold workgroup up to head dim 128 (8 waves
 BLOCK_N = 64            # keys per tile (one V^T image per tile)
 K_ROW_STRIDE_MAX = 1 << 24   # K rows are addressed with 32-bit byte offsets within a tile
 Q_ROW_STRIDE_MAX = 1 << 22   # head dim 128: Q rows, with 32-bit byte offsets within 256 rows
+ANY_STRIDE = 1 << 62         # read with 64-bit addresses
 # V^T tiles are fp16 images of v * 2^-e, e the tile's exponent (0 below 2^15).  A tile value
 # below 2^(e - 14) keeps only an absolute precision of 2^(e - 25), which bounds the error it
 # adds to O; e <= 13 keeps that under 2^-12, a quarter of the bf16 absolute tolerance.  Blocks
@@ -113,19 +114,25 @@ SHORT_TILE_US, SHORT_MERGE_US, SHORT_CHUNK_US = 0.6, 3.0, 0.05
 CUS = 256
 
 
-@functools.lru_cache(maxsize=4096)
 def short_chunks(units: int, sk: int) -> tuple[int, int]:
     """(chunks, tiles per chunk) of a head's keys for `units` (head, query block) pairs."""
-    tiles = -(-sk // ATTN_SHORT_TILE)
+    return _tile_chunks(units, -(-sk // ATTN_SHORT_TILE))
 
-    def cost(chunks):
-        rounds = -(-units * chunks // CUS)
-        return (rounds * -(-tiles // chunks) * SHORT_TILE_US
-                + (SHORT_MERGE_US + chunks * SHORT_CHUNK_US if chunks > 1 else 0.0))
 
+@functools.lru_cache(maxsize=4096)
+def _tile_chunks(units: int, tiles: int) -> tuple[int, int]:
+    # kept by tiles: a key range that grows token by token is searched once in 32 calls
     most = max(1, min(SHORT_MAX_CHUNKS, tiles // ATTN_SHORT_WAVES, SHORT_MAX_WORKGROUPS // units))
-    chunks = min(range(1, most + 1), key=cost)
-    per = -(-tiles // chunks)
+    best, cost = 1, -(-units // CUS) * tiles * SHORT_TILE_US
+    least = max(units * tiles / CUS, -(-tiles // most))     # passes of any split
+    for chunks in range(2, most + 1):
+        merge = SHORT_MERGE_US + chunks * SHORT_CHUNK_US
+        if least * SHORT_TILE_US + merge >= cost:
+            break                                # nor is any larger count cheaper
+        us = -(-units * chunks // CUS) * -(-tiles // chunks) * SHORT_TILE_US + merge
+        if us < cost:
+            best, cost = chunks, us
+    per = -(-tiles // best)
     return -(-tiles // per), per
 
 
@@ -145,24 +152,42 @@ SHORT_PASS_US = {64: 1.2, 128: 1.8, 256: 2.5}
 SHORT_RESIDENT = {64: 1024, 128: 512, 256: 256}
 
 
-def _fold_cost(bh, sq, sk, head_dim, causal, bm, tile_us, per):
+def _fold_blocks(sq, sk, causal, bm):
+    """(query blocks, blocks whose last tile is on the causal diagonal, tiles of the longest block,
+    tiles of all blocks) of a head, with query blocks of `bm`."""
+    nqb, tiles, step = -(-sq // bm), -(-sk // BLOCK_N), bm // BLOCK_N
+    if not causal:
+        return nqb, 0, tiles, nqb * tiles
+    rising = min(nqb, tiles // step)             # block i sees min(tiles, step * (i + 1))
+    return (nqb, rising, min(tiles, step * nqb),
+            step * rising * (rising + 1) // 2 + (nqb - rising) * tiles)
+
+
+def _fold_items(blocks, per, step):
+    """Workgroups of a head with its blocks in parts of `per` tiles."""
+    nqb, rising, longest, _ = blocks
+    items = (nqb - rising) * -(-longest // per)
+    for k in range(-(-step * rising // per)):    # rising blocks that have a part k
+        items += rising - k * per // step
+    return items
+
+
+def _fold_cost(bh, sq, head_dim, causal, bm, blocks, tile_us, per):
     """us of the fold (and merge) with query blocks of `bm` and keys in parts of `per` tiles."""
-    nqb = -(-sq // bm)
-    blocks = [-(-(min(sk, (i + 1) * bm) if causal else sk) // BLOCK_N) for i in range(nqb)]
-    per = min(per, blocks[-1])
-    items = bh * sum(-(-t // per) for t in blocks)
+    nqb, _, longest, total = blocks
+    per = min(per, longest)
+    items = bh * _fold_items(blocks, per, bm // BLOCK_N)
     if causal:     # heaviest first: the last items to finish are about half a part apart
-        tiles = max(per, bh * sum(blocks) / CUS + per / 2)
+        tiles = max(per, bh * total / CUS + per / 2)
     else:
         tiles = -(-items // CUS) * per
     cost = tile_us * tiles + BLOCK_US * max(1.0, items / CUS)
-    if per < blocks[-1]:
+    if per < longest:
         state = 2 * 4 * items * sq / nqb * head_dim    # written and read, fp32
         cost += MERGE_US + state / STATE_BYTES_PER_US
     return cost
 
 
-@functools.lru_cache(maxsize=4096)
 def _fold_choice(bh: int, sq: int, sk: int, head_dim: int, causal: bool) -> tuple:
     """(us, (w64, waves, tiles per part or None)) of the cheapest fold after the V^T pack.
 
@@ -172,21 +197,36 @@ def _fold_choice(bh: int, sq: int, sk: int, head_dim: int, causal: bool) -> tupl
     sq=100 sk=4000 108 / 92 / 44; causal B*H=8 s=4096 103 / 84 / 63; full B*H=64 sq=333 sk=2000
     67 / 57 / 59; causal B*H=128 s=1500 122 / 117 / 162; full B*H=128 s=512 33 / 34 / 64; causal
     B*H=128 s=4096 592 / 645 / -; d=64 causal B*H=1 s=6000 110 / 82 / 28; d=256 full B*H=16 s=700
-    - / 45 / 43."""
+    - / 45 / 43.
+
+    Found once for the sizes of the same tile counts, so that lengths that change from call to call
+    are not searched anew."""
+    us, waves, per = _tile_choice(bh, -(-sq // BLOCK_N), -(-sk // BLOCK_N), head_dim, causal)
+    return us, (waves == 8 and use_w64(head_dim, causal, sq, sk), waves, per)
+
+
+@functools.lru_cache(maxsize=4096)
+def _tile_choice(bh: int, sq_tiles: int, sk_tiles: int, head_dim: int, causal: bool) -> tuple:
+    """(us, waves, tiles per part or None) of the cheapest fold."""
+    sq, sk = sq_tiles * BLOCK_N, sk_tiles * BLOCK_N
     most = -(-(min(sk, sq) if causal else sk) // BLOCK_N)
     big = TILE_256_US[head_dim]
     best = None
     if big is not None:
         tile_us = big[0] + big[1] * min(1.0, bh * -(-sq // 256) / CUS)
-        best = (_fold_cost(bh, sq, sk, head_dim, causal, 256, tile_us, most + 4),
-                (use_w64(head_dim, causal, sq, sk), 8, None))
+        best = (_fold_cost(bh, sq, head_dim, causal, 256, _fold_blocks(sq, sk, causal, 256), tile_us,
+                           most + 4), 8, None)
+    blocks, tile_us = _fold_blocks(sq, sk, causal, 128), TILE_128_US[head_dim]
+    # the passes, workgroups and merge of any split
+    least = tile_us * (bh * blocks[3] / CUS) + BLOCK_US * max(1.0, bh * blocks[0] / CUS) + MERGE_US
     for parts in (1, 2, 3, 4, 6, 8, 12, 16):
         per = -(-most // parts)
-        if parts > 1 and (per < 2 or parts * bh * sq * (head_dim + 2) * 4 > MAX_STATE_BYTES):
+        if parts > 1 and (per < 2 or parts * bh * sq * (head_dim + 2) * 4 > MAX_STATE_BYTES
+                          or least >= best[0]):
             break
-        cost = _fold_cost(bh, sq, sk, head_dim, causal, 128, TILE_128_US[head_dim], per if parts > 1 else most + 4)
+        cost = _fold_cost(bh, sq, head_dim, causal, 128, blocks, tile_us, per if parts > 1 else most + 4)
         if best is None or cost < best[0]:
-            best = (cost, (False, 4, per if parts > 1 else None))
+            best = (cost, 4, per if parts > 1 else None)
     return best
 
 
@@ -194,18 +234,52 @@ def _fold_plan(bh, sq, sk, head_dim, causal):
     return _fold_choice(bh, sq, sk, head_dim, causal)[1]
 
 
-@functools.lru_cache(maxsize=4096)
+_KERNELS: dict = {}
+
+
+def _kernels(device, head_dim, causal, dtype, short, w64=None, waves=None, parts=False) -> tuple:
+    """(pack or None, fold, merge or None) of one kind of call, fetched once per device."""
+    key = (device, head_dim, causal, dtype, short, w64, waves, parts)
+    found = _KERNELS.get(key)
+    if found is not None:
+        return found
+    if short:
+        names = attention_short_kernel_names(head_dim, causal, dtype)
+        prog = _short_program(head_dim, causal, dtype)
+        found = (None,
+                 prog.kernel(names[0], (hip.PTR,) * 7 + (hip.I32,) * 6 + (hip.I64,) * 9 + (hip.F32,),
+                             64 * ATTN_SHORT_WAVES, device),
+                 prog.kernel(names[1], (hip.PTR,) * 4 + (hip.I64, hip.I32), 256, device))
+    else:
+        prog = _program(head_dim, causal, dtype, w64, waves, parts)
+        name = attention_kernel_name(head_dim, causal, dtype, w64, waves, parts)
+        found = (prog.kernel(attention_pack_kernel_name(head_dim, dtype),
+                             (hip.PTR,) * 3 + (hip.I32,) * 2 + (hip.I64,) * 3, 256, device),
+                 prog.kernel(name, (hip.PTR,) * 7 + (hip.I32,) * 3 + (hip.I64,) * 9 + (hip.I32, hip.F32)
+                             + ((hip.PTR,) * 2 + (hip.I32,) * 2 if parts else ()),
+                             attention_fold_threads(head_dim, w64, waves), device),
+                 prog.kernel(name + "_merge", (hip.PTR,) * 4 + (hip.I64,) + (hip.I32,) * 3, 256, device)
+                 if parts else None)
+    _KERNELS[key] = found
+    return found
+
+
 def _short_wins(bh: int, sq: int, sk: int, head_dim: int, causal: bool) -> bool:
     """Whether the short-query kernels run a call: always up to 16 queries; beyond, where they are
     estimated 15% cheaper (bf16 causal B*H=8 s=512 13.3 us against 17.5, d=256 causal B*H=16 s=100
     9.8 against 18.4; B*H=12 s=1000 d=64 full 34 against 21; B*H=160 sq=35 sk=5120 196 against
     189 on 256-query blocks)."""
-    if sq <= SHORT_MAX_SQ:
-        return True
+    return sq <= SHORT_MAX_SQ or _short_cheaper(bh, -(-sq // ATTN_SHORT_BLOCK_M),
+                                                -(-sk // ATTN_SHORT_TILE), head_dim, causal)
+
+
+@functools.lru_cache(maxsize=4096)
+def _short_cheaper(bh: int, sq_blocks: int, sk_tiles: int, head_dim: int, causal: bool) -> bool:
+    sq, sk = sq_blocks * ATTN_SHORT_BLOCK_M, sk_tiles * ATTN_SHORT_TILE
     seen = min(sq, sk) if causal else sk
     fold = (_fold_choice(bh, sq, sk, head_dim, causal)[0] + PACK_US
             + bh * seen * head_dim * 4 / PACK_BYTES_PER_US)
-    units = bh * -(-sq // ATTN_SHORT_BLOCK_M)
+    units = bh * sq_blocks
     chunks, per = short_chunks(units, seen)
     wait = (SHORT_LAUNCH_US + -(-units * chunks // SHORT_RESIDENT[head_dim])
             * (SHORT_BLOCK_US + -(-per // ATTN_SHORT_WAVES) * SHORT_PASS_US[head_dim]))
@@ -218,31 +292,38 @@ def _short_wins(bh: int, sq: int, sk: int, head_dim: int, causal: bool) -> bool:
 def validate_attention_inputs(q, k, v, *, metadata: bool = False):
     import torch
 
+    strided, dtypes = torch.strided, (torch.bfloat16, torch.float16)
     for t, nm in ((q, "q"), (k, "k"), (v, "v")):
-        if t.layout != torch.strided:
+        if t.layout != strided:
             raise TypeError(f"attention {nm} must be strided")
         if t.ndim != 4:
             raise ValueError(f"attention {nm} must be [batch, heads, seq, head_dim]")
-        if t.dtype not in (torch.bfloat16, torch.float16):
+        if t.dtype not in dtypes:
             raise TypeError(f"attention fold supports bfloat16 and float16 inputs, got {t.dtype} for {nm}")
         if not metadata and t.device.type != "cuda":
             raise ValueError("attention execution requires a ROCm (cuda) device")
-    if k.shape != v.shape or q.shape[0] != k.shape[0] or q.shape[1] != k.shape[1] or q.shape[3] != k.shape[3]:
+    qs, ks = q.shape, k.shape
+    if ks != v.shape or qs[0] != ks[0] or qs[1] != ks[1] or qs[3] != ks[3]:
         raise ValueError(f"attention shapes do not match: q {tuple(q.shape)}, k {tuple(k.shape)}, v {tuple(v.shape)}")
     if k.dtype != q.dtype or v.dtype != q.dtype:
         raise TypeError(f"attention q, k, v must share one dtype, got {q.dtype}, {k.dtype}, {v.dtype}")
     if q.device != k.device or q.device != v.device:
         raise ValueError("attention tensors must be on the same device")
-    if q.shape[3] not in ATTN_HEAD_DIMS:
+    if qs[3] not in ATTN_HEAD_DIMS:
         raise NotImplementedError("attention fold supports head_dim 64, 128 and 256")
-    if k.shape[2] == 0:
+    if ks[2] == 0:
         raise ValueError("attention needs at least one key")
-    return tuple(q.shape)
+    return tuple(qs)
 
 
-def _kernel_ready(t):
-    ok = (t.stride(3) == 1 and all(s % 8 == 0 for s in t.stride()[:3]) and t.data_ptr() % 16 == 0)
-    return t if ok else t.contiguous()
+def _operand(t, row_stride_max):
+    """(t, or its contiguous copy where a kernel cannot read its rows; batch, head, row strides)."""
+    sb, sh, ss, sd = t.stride()
+    if (sd == 1 and sb % 8 == 0 and sh % 8 == 0 and ss % 8 == 0 and ss < row_stride_max
+            and t.data_ptr() % 16 == 0):
+        return t, (sb, sh, ss)
+    t = t.contiguous()
+    return t, t.stride()[:3]
 
 
 def run_attention(q, k, v, *, scale: float | None = None, causal: bool = True,
@@ -259,7 +340,7 @@ def run_attention(q, k, v, *, scale: float | None = None, causal: bool = True,
         out, lse, _ = call.run(q, k, v)
         return (out, lse) if return_lse else out
     if key is None and _is_metadata(q):    # shapes may be symbolic: no launch is chosen
-        out, lse, _, _ = _outputs(q, k, v, scale, return_lse)
+        out, lse, _, _ = _outputs(q, k, v, scale, return_lse, True)
     elif _takes_short(q, k, causal):
         out, lse, call = _launch_short(q, k, v, scale, causal, return_lse)
     else:
@@ -282,12 +363,15 @@ def _seen_key(q, k, v, scale, causal, return_lse):
     # a scale whose printed form may not be its value (a tensor) takes the full path
     if hip.recording_active() or not (scale is None or type(scale) in (int, float)):
         return None
-    key = [type(scale).__name__, repr(scale), bool(causal), bool(return_lse)]
+    plain, strided = torch.Tensor, torch.strided
     for t in (q, k, v):
-        if type(t) is not torch.Tensor or not t.is_cuda or t.layout != torch.strided:
+        if type(t) is not plain or not t.is_cuda or t.layout != strided:
             return None
-        key += (t.dtype, t.device, t.shape, t.stride(), t.data_ptr() % 16)
-    return tuple(key)
+    # (a NaN scale equals no key, and is refused)
+    return (type(scale), scale, bool(causal), bool(return_lse),
+            q.dtype, q.device, q.shape, q.stride(), q.data_ptr() % 16,
+            k.dtype, k.device, k.shape, k.stride(), k.data_ptr() % 16,
+            v.dtype, v.device, v.shape, v.stride(), v.data_ptr() % 16)
 
 
 class _Call:
@@ -343,10 +427,10 @@ class _Call:
 
 def _takes_short(q, k, causal) -> bool:
     """Whether the call runs the short-query kernels (calls to be refused do not matter here)."""
-    if q.ndim != 4 or k.ndim != 4 or q.shape[3] not in ATTN_HEAD_DIMS or 0 in q.shape or 0 in k.shape:
+    qs, ks = q.shape, k.shape
+    if len(qs) != 4 or len(ks) != 4 or qs[3] not in ATTN_HEAD_DIMS or 0 in qs or 0 in ks:
         return False
-    B, H, Sq, D = q.shape
-    return _short_wins(B * H, Sq, k.shape[2], D, bool(causal))
+    return _short_wins(qs[0] * qs[1], qs[2], ks[2], qs[3], bool(causal))
 
 
 def launch_attention(q, k, v, *, scale: float | None = None, causal: bool = True,
@@ -364,11 +448,10 @@ def _is_metadata(q) -> bool:
     return isinstance(q, FakeTensor) or q.device.type == "meta"
 
 
-def _outputs(q, k, v, scale, return_lse):
+def _outputs(q, k, v, scale, return_lse, metadata):
     """(out, lse or None, scale, whether nothing is to be launched) after validation."""
     import torch
 
-    metadata = _is_metadata(q)
     shape = validate_attention_inputs(q, k, v, metadata=metadata)
     out = torch.empty(shape, dtype=q.dtype, device=q.device)
     lse = torch.empty(shape[:3], dtype=torch.float32, device=q.device) if return_lse else None
@@ -385,36 +468,27 @@ def _launch_short(q, k, v, scale, causal, return_lse):
     was copied."""
     import torch
 
-    out, lse, scale, done = _outputs(q, k, v, scale, return_lse)
+    out, lse, scale, done = _outputs(q, k, v, scale, return_lse, False)
     if done:
         return out, lse, None
     B, H, Sq, D = q.shape
     given = (q, k, v)
-    q, k, v = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)
-    if k.stride(2) >= K_ROW_STRIDE_MAX:
-        k = k.contiguous()
-    if v.stride(2) >= K_ROW_STRIDE_MAX:
-        v = v.contiguous()
+    (q, qs), (k, ks), (v, vs) = (_operand(q, ANY_STRIDE), _operand(k, K_ROW_STRIDE_MAX),
+                                 _operand(v, K_ROW_STRIDE_MAX))
     device = q.device.index if q.device.index is not None else torch.cuda.current_device()
     Sk = k.shape[2]
     nqb = -(-Sq // ATTN_SHORT_BLOCK_M)
     chunks, per = short_chunks(B * H * nqb, min(Sk, Sq) if causal else Sk)
     rows = B * H * Sq
     call = _Call(q.shape, return_lse)
-    names = attention_short_kernel_names(D, causal, q.dtype)
-    prog = _short_program(D, causal, q.dtype)
-    fold = prog.kernel(names[0], (hip.PTR,) * 7 + (hip.I32,) * 6 + (hip.I64,) * 9 + (hip.F32,),
-                       64 * ATTN_SHORT_WAVES, device)
+    _, fold, merge = _kernels(device, D, bool(causal), q.dtype, True)
     call.fold = (fold, (-(-B * H * chunks // 8) * nqb * 8,),
-                 (B, H, Sq, Sk, chunks, per, q.stride(0), q.stride(1), q.stride(2),
-                  k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2),
-                  scale * LOG2E), ())
+                 (B, H, Sq, Sk, chunks, per) + qs + ks + vs + (scale * LOG2E,), ())
     if chunks > 1:
         call.add_state(chunks, rows, D)
-        merge = prog.kernel(names[1], (hip.PTR,) * 4 + (hip.I64, hip.I32), 256, device)
         call.merge = (merge, (rows,), (rows, chunks))
     call.run(q, k, v, out, lse)
-    return out, lse, call if _same(given, (q, k, v)) else None
+    return out, lse, call if q is given[0] and k is given[1] and v is given[2] else None
 
 
 def _launch(q, k, v, scale, causal, return_lse, e_max: int, w64: bool | None = None,
@@ -427,6 +501,8 @@ def _launch(q, k, v, scale, causal, return_lse, e_max: int, w64: bool | None = N
     when the keys are whole."""
     import torch
 
+    if _is_metadata(q):
+        return _outputs(q, k, v, scale, return_lse, True)[:2] + (None,)
     out, lse, work, call, tiles = _launch_fold(q, k, v, scale, causal, return_lse, e_max, w64, waves, per)
     if work is None:
         return out, lse, None
@@ -434,27 +510,20 @@ def _launch(q, k, v, scale, causal, return_lse, e_max: int, w64: bool | None = N
     return out, lse, exps
 
 
-def _same(given, used) -> bool:
-    return all(a is b for a, b in zip(given, used))
-
-
 def _launch_fold(q, k, v, scale, causal, return_lse, e_max, w64=None, waves=None, per=None):
     """(out, lse or None, workspace, call, (offset, count) of the exponents) of the V^T pack and
     the fold; the call is None where an input was copied."""
     import torch
 
-    out, lse, scale, done = _outputs(q, k, v, scale, return_lse)
+    out, lse, scale, done = _outputs(q, k, v, scale, return_lse, False)
     if done:
         return out, lse, None, None, None
     B, H, Sq, D = q.shape
     if w64 is None and waves is None:
         w64, waves, per = _fold_plan(B * H, Sq, k.shape[2], D, bool(causal))
     given = (q, k, v)
-    q, k, v = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)
-    if k.stride(2) >= K_ROW_STRIDE_MAX:
-        k = k.contiguous()
-    if q.stride(2) >= Q_ROW_STRIDE_MAX:
-        q = q.contiguous()
+    (q, qs), (k, ks), (v, vs) = (_operand(q, Q_ROW_STRIDE_MAX), _operand(k, K_ROW_STRIDE_MAX),
+                                 _operand(v, ANY_STRIDE))
     device = q.device.index if q.device.index is not None else torch.cuda.current_device()
     Sk = min(k.shape[2], Sq) if causal else k.shape[2]    # no query sees a key past the last query
     ntiles = (Sk + BLOCK_N - 1) // BLOCK_N
@@ -470,25 +539,17 @@ def _launch_fold(q, k, v, scale, causal, return_lse, e_max, w64=None, waves=None
         most = -(-(min(Sk, nqb * bm) if causal else Sk) // BLOCK_N)   # tiles of the longest block
         per = min(per or most, most)
         parts = -(-most // per)
-    prog = _program(D, causal, q.dtype, w64, waves, parts > 1)
-    pack = prog.kernel(attention_pack_kernel_name(D, q.dtype),
-                       (hip.PTR,) * 3 + (hip.I32,) * 2 + (hip.I64,) * 3, 256, device)
-    call.pack = (pack, (B * H * ntiles,), (H, Sk, v.stride(0), v.stride(1), v.stride(2)))
-    name = attention_kernel_name(D, causal, q.dtype, w64, waves, parts > 1)
-    fold = prog.kernel(name, (hip.PTR,) * 7 + (hip.I32,) * 3 + (hip.I64,) * 9 + (hip.I32, hip.F32)
-                       + ((hip.PTR,) * 2 + (hip.I32,) * 2 if parts > 1 else ()),
-                       attention_fold_threads(D, w64, waves), device)
+    pack, fold, merge = _kernels(device, D, bool(causal), q.dtype, False, w64, waves, parts > 1)
+    call.pack = (pack, (B * H * ntiles,), (H, Sk) + vs)
     call.fold = (fold, (nqb * B * H * parts,),
-                 (H, Sq, Sk, q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1),
-                  k.stride(2), v.stride(0), v.stride(1), v.stride(2), int(e_max), scale * LOG2E),
+                 (H, Sq, Sk) + qs + ks + vs + (int(e_max), scale * LOG2E),
                  (parts, per) if parts > 1 else ())
     if parts > 1:
         call.add_state(parts, rows, D)
-        merge = prog.kernel(name + "_merge", (hip.PTR,) * 4 + (hip.I64,) + (hip.I32,) * 3, 256, device)
         call.merge = (merge, (-(-rows * (D // 4) // 256),), (rows, Sq, Sk, per))
     _, _, work = call.run(q, k, v, out, lse)
-    return (out, lse, work, call if _same(given, (q, k, v)) else None,
-            (call.exps, B * H * ntiles))
+    copied = q is not given[0] or k is not given[1] or v is not given[2]
+    return out, lse, work, None if copied else call, (call.exps, B * H * ntiles)
 
 
 def exact_path_taken(exps) -> bool:
