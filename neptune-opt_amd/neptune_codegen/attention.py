@@ -337,14 +337,14 @@ def run_attention(q, k, v, *, scale: float | None = None, causal: bool = True,
     key = _seen_key(q, k, v, scale, causal, return_lse)
     call = _SEEN.get(key) if key is not None else None
     if call is not None:
-        out, lse, _ = call.run(q, k, v)
+        out, lse = call.run(q, k, v)
         return (out, lse) if return_lse else out
     if key is None and _is_metadata(q):    # shapes may be symbolic: no launch is chosen
         out, lse, _, _ = _outputs(q, k, v, scale, return_lse, True)
     elif _takes_short(q, k, causal):
         out, lse, call = _launch_short(q, k, v, scale, causal, return_lse)
     else:
-        out, lse, _, call, _ = _launch_fold(q, k, v, scale, causal, return_lse, V_EXPONENT_MAX)
+        out, lse, call, _ = _launch_fold(q, k, v, scale, causal, return_lse, V_EXPONENT_MAX)
     if key is not None and call is not None:
         if len(_SEEN) >= _SEEN_MAX:
             _SEEN.clear()
@@ -387,8 +387,8 @@ class _Call:
         self.rows_bytes = 0                  # behind the states' O
         self.pack = self.fold = self.merge = None    # (kernel, grid, further arguments)
 
-    def run(self, q, k, v, out=None, lse=None):
-        """(out, lse or None, workspace or None)."""
+    def run(self, q, k, v, out=None, lse=None, exps=None):
+        """(out, lse or None); the tile exponents go to `exps` where it is given."""
         import torch
 
         if out is None:
@@ -408,15 +408,15 @@ class _Call:
             kernel.launch(grid, (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse_ptr,
                                  po, pml) + rest, stream)
         else:
-            exps = base + self.exps
+            exps_ptr = base + self.exps if exps is None else exps.data_ptr()
             pack, pack_grid, pack_rest = self.pack
-            pack.launch(pack_grid, (v.data_ptr(), base, exps) + pack_rest, stream)
-            kernel.launch(grid, (q.data_ptr(), k.data_ptr(), base, exps, v.data_ptr(), out.data_ptr(),
+            pack.launch(pack_grid, (v.data_ptr(), base, exps_ptr) + pack_rest, stream)
+            kernel.launch(grid, (q.data_ptr(), k.data_ptr(), base, exps_ptr, v.data_ptr(), out.data_ptr(),
                                  lse_ptr) + rest + ((po, pml) + tail if tail else ()), stream)
         if self.merge is not None:
             merge, merge_grid, merge_rest = self.merge
             merge.launch(merge_grid, (po, pml, out.data_ptr(), lse_ptr) + merge_rest, stream)
-        return out, lse, work
+        return out, lse
 
     def add_state(self, parts, rows, head_dim):
         """Workspace of `parts` fp32 states (O, then (max, sum)) of every query row."""
@@ -499,25 +499,22 @@ def _launch(q, k, v, scale, causal, return_lse, e_max: int, w64: bool | None = N
     compiler-scheduled 32-queries-per-wave kernel (8 waves, or `waves`; the keys in parts of
     `per` tiles), whose results at head dim 128 equal the instruction-scheduled one's bit for bit
     when the keys are whole."""
-    import torch
-
     if _is_metadata(q):
         return _outputs(q, k, v, scale, return_lse, True)[:2] + (None,)
-    out, lse, work, call, tiles = _launch_fold(q, k, v, scale, causal, return_lse, e_max, w64, waves, per)
-    if work is None:
-        return out, lse, None
-    exps = work[tiles[0]:tiles[0] + 4 * tiles[1]].view(torch.int32)
+    out, lse, _, exps = _launch_fold(q, k, v, scale, causal, return_lse, e_max, w64, waves, per, True)
     return out, lse, exps
 
 
-def _launch_fold(q, k, v, scale, causal, return_lse, e_max, w64=None, waves=None, per=None):
-    """(out, lse or None, workspace, call, (offset, count) of the exponents) of the V^T pack and
-    the fold; the call is None where an input was copied."""
+def _launch_fold(q, k, v, scale, causal, return_lse, e_max, w64=None, waves=None, per=None,
+                 keep_exps=False):
+    """(out, lse or None, call, exponents or None) of the V^T pack and the fold; the call is None
+    where an input was copied.  With `keep_exps` the exponents are a tensor of their own: a caller
+    that holds on to them holds no workspace."""
     import torch
 
     out, lse, scale, done = _outputs(q, k, v, scale, return_lse, False)
     if done:
-        return out, lse, None, None, None
+        return out, lse, None, None
     B, H, Sq, D = q.shape
     if w64 is None and waves is None:
         w64, waves, per = _fold_plan(B * H, Sq, k.shape[2], D, bool(causal))
@@ -547,9 +544,10 @@ def _launch_fold(q, k, v, scale, causal, return_lse, e_max, w64=None, waves=None
     if parts > 1:
         call.add_state(parts, rows, D)
         call.merge = (merge, (-(-rows * (D // 4) // 256),), (rows, Sq, Sk, per))
-    _, _, work = call.run(q, k, v, out, lse)
+    exps = torch.empty(B * H * ntiles, dtype=torch.int32, device=q.device) if keep_exps else None
+    call.run(q, k, v, out, lse, exps)
     copied = q is not given[0] or k is not given[1] or v is not given[2]
-    return out, lse, work, None if copied else call, (call.exps, B * H * ntiles)
+    return out, lse, None if copied else call, exps
 
 
 def exact_path_taken(exps) -> bool:
