@@ -16,7 +16,8 @@ import threading
 
 from neptune_codegen import hip
 from neptune_codegen.autotune import (MAX_TPR, MAX_UNROLL, UNROLL, WIDE_16BIT_ROW, best_config,
-                                      lanes_per_row, parameter_identity, parameter_tag, vec_of)
+                                      default_config, lanes_per_row, parameter_identity,
+                                      parameter_tag, vec_of)
 from neptune_codegen.emitters import (BASE_OPTIONS, NO_CONTRACT, FoldVariant, RowVariant,
                                       check_supported, emit_kernel_source, emit_readout_source,
                                       emit_rms_state_source, fold_kernel_name,
@@ -409,6 +410,20 @@ def _few_rows(var: FoldVariant, rows: int, ncols: int) -> FoldVariant:
     return dataclasses.replace(var, tpr=tpr, unroll=unroll)
 
 
+def _serial_variant(kernel, x2, rows, ncols, block, num_warps) -> FoldVariant:
+    """A serial fold's launch shape.  A configuration other than the default one of the shape --
+    asked for by the caller, fixed in an operator's name, or measured into the launch table --
+    keeps its lanes per row; the default one has them spread where the rows are few."""
+    sk = kernel.sk
+    var = _fold_variant(x2, ncols, block, num_warps, resident=sk.two_pass,
+                        merge_heavy=not sk.is_log and not sk.two_pass, heavy_phi=kernel.heavy_phi)
+    if sk.two_pass:
+        return dataclasses.replace(var, resident=ncols <= readout_tile(var))
+    if (block, num_warps) == default_config(rows, ncols, x2.dtype):
+        return _few_rows(var, rows, ncols)
+    return var
+
+
 def _grid_1d(items: int, per_wg: int) -> int:
     return max(1, (items + per_wg - 1) // per_wg)
 
@@ -421,14 +436,7 @@ def launch_reduction(kernel, plan, x2, out, rows, ncols, block, num_warps, *, wr
     device = x2.device.index if x2.device.index is not None else torch.cuda.current_device()
     stream = hip.current_stream(x2.device)
     if plan == "serial":
-        sk = kernel.sk
-        var = _fold_variant(x2, ncols, block, num_warps, resident=sk.two_pass,
-                            merge_heavy=not sk.is_log and not sk.two_pass,
-                            heavy_phi=kernel.heavy_phi)
-        if sk.two_pass:
-            var = dataclasses.replace(var, resident=ncols <= readout_tile(var))
-        else:
-            var = _few_rows(var, rows, ncols)
+        var = _serial_variant(kernel, x2, rows, ncols, block, num_warps)
         k = kernel.kernel(var, "", device)
         rpw = max(1, var.wg // var.tpr)
         grid = (_grid_1d(rows, rpw),)
@@ -461,7 +469,8 @@ def run(name: str, x, block: int | None = None, num_warps: int | None = None,
 
     Rank >= 1 returns x.shape[:-1] (keepdim appends a 1).  Real execution needs a ROCm device
     and float16/bfloat16/float32; Fake/meta tensors return metadata only.  Declared parameter
-    defaults are filled for anything not passed.
+    defaults are filled for anything not passed.  `block` and `num_warps` default to the launch
+    table's choice; what they mean for a fold's class is in `_fold_variant`.
 
     A call on a plain device tensor whose (fold, plan, dtype, device, shape, strides, 16-byte
     alignment, launch options, parameter types and values) were seen before reuses that call's
