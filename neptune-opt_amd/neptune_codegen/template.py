@@ -189,9 +189,13 @@ def _fold_seen(x, options: tuple, params: dict):
     key = options + (x.dtype, x.device, x.shape, x.stride(), x.data_ptr() % 16)
     for name in sorted(params):
         value = params[name]
-        if type(value) not in (int, float, bool):    # its printed form may not be its value
-            return None, None
-        key += (name, type(value), repr(value))
+        kind = type(value)
+        if kind not in (int, float, bool):           # the binary64 value that a kernel is made for
+            try:                                     # (its printed form may be another)
+                value = float(value)
+            except (TypeError, ValueError, OverflowError, RuntimeError):
+                return None, None
+        key += (name, kind, repr(value))
     try:
         return key, _RUN_SEEN.get(key)
     except TypeError:                                # an option that cannot be hashed
