@@ -364,6 +364,9 @@ def _segment_spans(data, segments, *, offsets, unsafe):
     return spans
 
 
+MOST_LANES = (1 << 32) - 256
+
+
 def _segment_variant(flat, spans, channels: int) -> SegmentVariant:
     """Channel words per lane and token rows per step.  A lane's adds are ordered, so a segment's
     rows are only in flight together, never split over lanes: with few (segment, chunk) lanes
@@ -388,10 +391,12 @@ def _segment_variant(flat, spans, channels: int) -> SegmentVariant:
         words = 2 if waves < 4096 else 4
     while words > 1 and channels * size < 4 * words:
         words //= 2
+    # a launch has fewer than 2^32 lanes: the widest chunks where narrow ones make more
+    while words < 4 and channels * size >= 8 * words and nseg * -(-channels * size // (4 * words)) > MOST_LANES:
+        words *= 2
     per_lane = 4 * words // size
     chunks = -(-channels // per_lane)
-    if (channels < per_lane or (flat.stride(1) != 1 and channels > 1)
-            or nseg * chunks > (1 << 32) - 256):
+    if channels < per_lane or (flat.stride(1) != 1 and channels > 1) or nseg * chunks > MOST_LANES:
         return SegmentVariant(dtype, span_dtype, False, 0, 4)
     aligned = (channels % per_lane == 0 and flat.stride(0) % per_lane == 0
                and flat.data_ptr() % (4 * words) == 0)
