@@ -66,6 +66,50 @@ __device__ __forceinline__ State merge_state(const State& A, const State& B) {
   return R;
 }
 
+// N states merged at once: each accumulator is transported once, to the coordinate of all of them,
+// and the transported ones meet in a tree.  Merged one after the other, N - 1 transports and sums
+// round in turn, which over the 8 or 16 waves of a spread row cost accuracy (relative error of
+// fp32 stable_l2, 64 rows x 32000, against 64 bits: 1.3e-7 on 4 waves one after the other, 2.5e-7
+// on 16).
+template <class F, int N>
+__device__ __forceinline__ State merge_states(const State* states) {
+  int seen = 0, status = 0;
+  float cm = 0.0f, one_m = 0.0f, one_acc = consumer_init<F>();
+  State s[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    s[i] = states[i];
+    status |= s[i].status;
+    if (s[i].seen == 0) continue;
+    cm = seen == 0 ? s[i].m : (F::kProducerSum ? (cm + s[i].m) : __builtin_fmaxf(cm, s[i].m));
+    one_m = s[i].m;
+    one_acc = s[i].acc;
+    ++seen;
+  }
+  const bool several = seen > 1;
+  const float qN = eff<F>(several ? cm : 1.0f);
+  float t[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const bool v = several && s[i].seen != 0;
+    const float q = eff<F>(v ? s[i].m : 1.0f);
+    t[i] = (v ? s[i].acc : 0.0f) * F::rho(q, qN);
+    if constexpr (F::kHasBias) t[i] += F::beta(q, qN);
+    if (!v) t[i] = consumer_init<F>();
+  }
+#pragma unroll
+  for (int step = 1; step < N; step *= 2)
+#pragma unroll
+    for (int i = 0; i < N; i += 2 * step)
+      t[i] = F::kConsumerMax ? __builtin_fmaxf(t[i], t[i + step]) : (t[i] + t[i + step]);
+  State R;
+  R.m = several ? cm : one_m;
+  R.acc = several ? t[0] : one_acc;
+  R.seen = seen > 0 ? 1 : 0;
+  R.status = status;
+  return R;
+}
+
 template <int S>
 __device__ __forceinline__ State partner_state(const State& s) {
   State o;
@@ -251,8 +295,9 @@ __device__ __forceinline__ void exact_tile(State& s, const typename St::T* row, 
   exact_fold<F, UNROLL, TL::VEC>(s, v, ok, n);
 }
 
-// A row's lane states merged (lanes in order, then waves in order), complete in every lane.
-template <class F, int TPR>
+// A row's lane states merged (lanes in order, then waves in order or, SPREAD, at once), complete
+// in every lane.
+template <class F, int TPR, bool SPREAD = false>
 __device__ __forceinline__ State row_state(State s, State* lds_state) {
   typedef RowComm<TPR> RC;
   s = group_merge<F, RC::G>(s);
@@ -261,6 +306,7 @@ __device__ __forceinline__ State row_state(State s, State* lds_state) {
     __syncthreads();
     if (lane_id() == 0) lds_state[wave] = s;
     __syncthreads();
+    if constexpr (SPREAD) return merge_states<F, RC::WPR>(lds_state + first);
     State r = lds_state[first];
 #pragma unroll
     for (int w = 1; w < RC::WPR; ++w) r = merge_state<F>(r, lds_state[first + w]);
@@ -280,7 +326,7 @@ __device__ __forceinline__ State empty_state() {
 }
 
 // Exact state of the columns [c0, c1) of one row, complete in every lane of the row.
-template <class F, class St, int TPR, int UNROLL, int VECTOR>
+template <class F, class St, int TPR, int UNROLL, int VECTOR, bool SPREAD = false>
 __device__ __forceinline__ State exact_row_state(const typename St::T* row, i64 stride_col,
                                                  i64 c0, i64 c1, int t, float n,
                                                  State* lds_state) {
@@ -294,7 +340,7 @@ __device__ __forceinline__ State exact_row_state(const typename St::T* row, i64 
     sp.load_rest(rest, row, t);
     exact_fold<F, Span<St, TPR, VECTOR>::RU, 1>(s, rest.s, rest.ok, n);
   }
-  return row_state<F, TPR>(s, lds_state);
+  return row_state<F, TPR, SPREAD>(s, lds_state);
 }
 
 // Final value of a row from its exact state (emitters.py:522-532 for exponential folds).
@@ -521,7 +567,8 @@ __device__ __forceinline__ float log_row_finish(LogLane s, const typename St::T*
   });
 }
 
-template <class F, class St, int TPR, int UNROLL, int VECTOR, bool CENTERED = false>
+template <class F, class St, int TPR, int UNROLL, int VECTOR, bool CENTERED = false,
+          bool SPREAD = false>
 __device__ __forceinline__ float row_result(const typename St::T* rp, i64 stride_col, i64 c1,
                                             int t, float n, State* lds_state,
                                             LogLane* lds_lane) {
@@ -531,13 +578,13 @@ __device__ __forceinline__ float row_result(const typename St::T* rp, i64 stride
     return log_row_finish<F, St, TPR, UNROLL, VECTOR>(s, rp, stride_col, c1, t, n, lds_state,
                                                       lds_lane);
   } else {
-    const State e = exact_row_state<F, St, TPR, UNROLL, VECTOR>(rp, stride_col, 0, c1, t, n,
-                                                                 lds_state);
+    const State e = exact_row_state<F, St, TPR, UNROLL, VECTOR, SPREAD>(rp, stride_col, 0, c1, t, n,
+                                                                        lds_state);
     return finalize_state<F>(e, n);
   }
 }
 
-template <class F, class St, int TPR, int UNROLL, int VECTOR, int WG>
+template <class F, class St, int TPR, int UNROLL, int VECTOR, int WG, bool SPREAD = false>
 __device__ __forceinline__ void fold_serial(const typename St::T* __restrict__ x,
                                             typename St::T* __restrict__ out, i64 rows,
                                             i64 ncols, i64 stride_row, i64 stride_col) {
@@ -552,7 +599,8 @@ __device__ __forceinline__ void fold_serial(const typename St::T* __restrict__ x
   const i64 c1 = live ? ncols : 0;
   const float n = (float)ncols;
   const float result =
-      row_result<F, St, TPR, UNROLL, VECTOR>(rp, stride_col, c1, t, n, lds_state, lds_lane);
+      row_result<F, St, TPR, UNROLL, VECTOR, false, SPREAD>(rp, stride_col, c1, t, n, lds_state,
+                                                            lds_lane);
   if (live && t == 0) St::store(out + row, result);
 }
 

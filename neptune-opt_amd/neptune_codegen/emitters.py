@@ -213,6 +213,7 @@ class FoldVariant:
     waves: int = 4      # wave64s per workgroup (at least one row)
     ragged: bool = False    # vector rows of any alignment and width (nep_device.h kRagged)
     resident: bool = False  # two-pass folds: one tile holds the row, which stays in registers
+    spread: bool = False    # serial folds: more waves than the row's default, merged at once
 
     @property
     def wg(self) -> int:
@@ -224,7 +225,7 @@ class FoldVariant:
 
     def tag(self) -> str:
         return (f"{dtype_tag(self.dtype)[0]}_{access_tag(self.vector, self.ragged)}{self.tpr}"
-                f"u{self.unroll}w{self.waves}{'k' if self.resident else ''}")
+                f"u{self.unroll}w{self.waves}{'k' if self.resident else ''}{'x' if self.spread else ''}")
 
 
 _FOLD_ARGS_SERIAL = ("const void* x, void* out, long long rows, long long ncols, "
@@ -237,7 +238,7 @@ def _fold_kernel(sk: Skeleton, plan: str, part: str, var: FoldVariant) -> tuple[
     tmpl = f"Fold, {st}, {var.tpr}, {var.unroll}, {var.access}, {var.wg}"
     if plan == "serial":
         name = f"{sk.name}_serial_{var.tag()}"
-        body = (f"nep::fold_serial<{tmpl}>((const {st}::T*)x, ({st}::T*)out, rows, ncols, "
+        body = (f"nep::fold_serial<{tmpl}{', true' if var.spread else ''}>((const {st}::T*)x, ({st}::T*)out, rows, ncols, "
                 "stride_row, stride_col);")
         sig = _FOLD_ARGS_SERIAL
     elif plan == "two_pass":

@@ -393,25 +393,27 @@ def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: in
 FEW_ROWS_LANES = 1 << 17
 
 
-def _few_rows(var: FoldVariant, rows: int, ncols: int) -> FoldVariant:
+def _few_rows(var: FoldVariant, rows: int, ncols: int, merge: bool = False) -> FoldVariant:
     """A serial fold's launch shape for few rows: lanes per row are doubled while all rows together
     leave most of the chip idle and each lane still has 4 slots of its row to load (with fewer the
     merge across wavefronts costs more than it saves: fp32 8 x 4096 3.4 us on 256 lanes, 4.9 on
     512).  Measured on MI355X, cold, before -> after: logsumexp fp32 1 x 262144 50 -> 22 us,
     256 x 32000 11.6 -> 9.0; stable_l2 bf16 4 x 262144 234 -> 21, 64 x 32000 34 -> 7.7,
     600 x 16384 19 -> 9.1; rmsnorm_max fp32 4 x 262144 50 -> 24; softcap_lse bf16 8 x 4096
-    5.5 -> 4.0.  With 2^16 lanes as the line stable_l2 bf16 256 x 32000 takes 12.5 us for 9.1, with
+    5.5 -> 4.0.  A second wavefront for an fp32 row of 64 lanes wants twice that (stable_l2 300 x
+    2048 3.13 us on one, 3.38 on two, and less exact: 8.9e-8 and 9.6e-8).  With 2^16 lanes as the line stable_l2 bf16 256 x 32000 takes 12.5 us for 9.1, with
     2^18 8.4, but logsumexp fp32 256 x 32000 9.7 for 9.0."""
     per_slot = vec_of(var.dtype) if var.vector else 1
     slots = -(-ncols // per_slot)
     tpr = var.tpr
-    while tpr < MAX_TPR and rows * tpr < FEW_ROWS_LANES and slots >= 8 * tpr:
+    while (tpr < MAX_TPR and rows * tpr < FEW_ROWS_LANES
+           and slots >= (16 if tpr == 64 and per_slot == 4 else 8) * tpr):
         tpr *= 2
     if tpr == var.tpr:
         return var
     per_lane = -(-slots // tpr)
     unroll = -(-per_lane // -(-per_lane // var.unroll))
-    return dataclasses.replace(var, tpr=tpr, unroll=unroll)
+    return dataclasses.replace(var, tpr=tpr, unroll=unroll, spread=merge and tpr > 64)
 
 
 def _serial_variant(kernel, x2, rows, ncols, block, num_warps) -> FoldVariant:
@@ -424,7 +426,7 @@ def _serial_variant(kernel, x2, rows, ncols, block, num_warps) -> FoldVariant:
     if sk.two_pass:
         return dataclasses.replace(var, resident=ncols <= readout_tile(var))
     if (block, num_warps) == default_config(rows, ncols, x2.dtype):
-        return _few_rows(var, rows, ncols)
+        return _few_rows(var, rows, ncols, merge=not sk.is_log)
     return var
 
 
