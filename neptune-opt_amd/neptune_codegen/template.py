@@ -406,7 +406,11 @@ def _few_rows(var: FoldVariant, rows: int, ncols: int, merge: bool = False) -> F
     per_slot = vec_of(var.dtype) if var.vector else 1
     slots = -(-ncols // per_slot)
     tpr = var.tpr
-    while (tpr < MAX_TPR and rows * tpr < FEW_ROWS_LANES
+    # 16-bit exponential rows stop at 512 lanes: the 128 registers of a lane among 1024 do not hold
+    # 8 slots in flight and the fold (28 to 40 spilled).  logsumexp bf16 22 x 235968 25.8 us on 256
+    # lanes, 18.8 on 512, 27.8 on 1024; 1 x 262144 22.1, 16.5, 25.1; 200 x 250000 31.5, 22.2, 34.4
+    most = MAX_TPR // 2 if per_slot == 8 and not merge else MAX_TPR
+    while (tpr < most and rows * tpr < FEW_ROWS_LANES
            and slots >= (16 if tpr == 64 and per_slot == 4 else 8) * tpr):
         tpr *= 2
     if tpr == var.tpr:
