@@ -165,7 +165,7 @@ def launch_readout(program: ReadoutProgram, x2, out, rows, ncols, block, num_war
     import torch
 
     device = x2.device.index if x2.device.index is not None else torch.cuda.current_device()
-    var = _fold_variant(x2, ncols, block, num_warps, resident=True, readout=True)
+    var = _fold_variant(x2, ncols, block, num_warps, resident=True, readout=True, by_rows=True)
     rpw = max(1, var.wg // var.tpr)
     kernel = program.kernel(var, device, resident=ncols <= readout_tile(var))
     grid, tail = (_grid_1d(rows, rpw),), (rows, ncols, x2.stride(0), x2.stride(1))
@@ -293,15 +293,26 @@ def _is_vector(x2, ncols: int, vec: int, extra_align: int = 0) -> bool:
 
 def _is_ragged(x2, ncols: int, vec: int) -> bool:
     """Rows of unit column stride and at least one vector wide, whatever their alignment: the
-    vectors inside the row are loaded whole (nep_fold.h Span, with both sides measured).  A
+    vectors inside the row are loaded whole (nep_device.h Span, with both sides measured).  A
     narrower row may hold no vector at all."""
     return x2.dim() == 2 and x2.stride(1) == 1 and ncols >= vec
 
 
+# Narrow rows that are few in all are one element per load: a launch of them is bound by its
+# latency, and the elements around the vectors make it longer.
+NARROW_ROW, FEW_ELEMENTS = 1024, 1 << 19
+
+
+def _is_small(x2, ncols: int) -> bool:
+    return type(ncols) is int and ncols < NARROW_ROW and x2.shape[0] * ncols < FEW_ELEMENTS
+
+
 def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: int = 0,
                   resident: bool = False, merge_heavy: bool = False,
-                  heavy_phi: bool = False, readout: bool = False) -> FoldVariant:
-    """Launch shape: 16-byte loads when the layout allows, lanes per row from BLOCK (a tile
+                  heavy_phi: bool = False, readout: bool = False,
+                  by_rows: bool = False) -> FoldVariant:
+    """Launch shape: 16-byte loads when the layout allows (`by_rows`: and pays for this many rows,
+    see `_is_small`), lanes per row from BLOCK (a tile
     wider than the workgroup's lanes gives each lane up to MAX_UNROLL slots first), workgroup =
     max(64 * num_warps, lanes per row).  Three fold classes then adjust it (serial plan only):
 
@@ -332,7 +343,7 @@ def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: in
     (bf16 and fp32)."""
     vec = vec_of(x2.dtype)
     vector = _is_vector(x2, ncols, vec, split_block)
-    ragged = not vector and _is_ragged(x2, ncols, vec)
+    ragged = not vector and _is_ragged(x2, ncols, vec) and not (by_rows and _is_small(x2, ncols))
     vector = vector or ragged
     if vector and split_block and split_block < vec:
         vector = ragged = False
@@ -426,7 +437,8 @@ def _serial_variant(kernel, x2, rows, ncols, block, num_warps) -> FoldVariant:
     keeps its lanes per row; the default one has them spread where the rows are few."""
     sk = kernel.sk
     var = _fold_variant(x2, ncols, block, num_warps, resident=sk.two_pass,
-                        merge_heavy=not sk.is_log and not sk.two_pass, heavy_phi=kernel.heavy_phi)
+                        merge_heavy=not sk.is_log and not sk.two_pass, heavy_phi=kernel.heavy_phi,
+                        by_rows=True)
     if sk.two_pass:
         return dataclasses.replace(var, resident=ncols <= readout_tile(var))
     if (block, num_warps) == default_config(rows, ncols, x2.dtype):
