@@ -402,18 +402,28 @@ def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: in
 
 # Lanes below which a launch's rows are spread over more of them (512 per CU).
 FEW_ROWS_LANES = 1 << 17
+CUS = 256
 
 
 def _few_rows(var: FoldVariant, rows: int, ncols: int, merge: bool = False) -> FoldVariant:
     """A serial fold's launch shape for few rows: lanes per row are doubled while all rows together
-    leave most of the chip idle and each lane still has 4 slots of its row to load (with fewer the
-    merge across wavefronts costs more than it saves: fp32 8 x 4096 3.4 us on 256 lanes, 4.9 on
-    512).  Measured on MI355X, cold, before -> after: logsumexp fp32 1 x 262144 50 -> 22 us,
-    256 x 32000 11.6 -> 9.0; stable_l2 bf16 4 x 262144 234 -> 21, 64 x 32000 34 -> 7.7,
-    600 x 16384 19 -> 9.1; rmsnorm_max fp32 4 x 262144 50 -> 24; softcap_lse bf16 8 x 4096
-    5.5 -> 4.0.  A second wavefront for an fp32 row of 64 lanes wants twice that (stable_l2 300 x
-    2048 3.13 us on one, 3.38 on two, and less exact: 8.9e-8 and 9.6e-8).  With 2^16 lanes as the line stable_l2 bf16 256 x 32000 takes 12.5 us for 9.1, with
-    2^18 8.4, but logsumexp fp32 256 x 32000 9.7 for 9.0."""
+    leave most of the chip idle and each lane keeps enough slots of its row to load (with fewer the
+    merge across wavefronts costs more than it saves).  Measured on MI355X, cold, us by lanes:
+
+    * 16-bit rows of a `merge` fold (a repair per butterfly level, few lanes to begin with): while
+      2^17 lanes in all are not reached.  stable_l2 bf16 64 x 32000 32.0 on 64 lanes, 18.7, 11.9,
+      8.6 on 512; 400 x 16384 20.1, 12.7, 9.0, 8.1; 200 x 185024 192 to 23.8 on 1024; past the
+      line, 800 x 32000 17.5 on 256, 20.5 on 512 (rmsnorm_max).
+    * The others are nearer to the loads' own time.  Beyond 256 lanes a row wants a CU of its own
+      and 12 slots per lane now: logsumexp bf16 256 x 65536 11.8 on 256, 10.7 on 512, but 257 x
+      65536 12.7, 15.7; fp32 stable_l2 64 x 16384 5.9, 5.6, but 64 x 8192 4.7, 4.9 (two rows on
+      a CU gain nothing either: 280 x 16384 8.4, 8.3, 400 x 32000 12.4, 13.0).  Beyond 512,
+      half a CU and 32 slots: logsumexp fp32 64 x 65536 11.9 on 512, 11.3 on 1024, but 64 x 32000
+      7.7, 8.0, and 200 x 65536 13.4, 14.1.  fp32 merge folds leave 128 lanes only so, too
+      (rmsnorm_max 256 x 4096 5.5, 5.1 on 256; 800 x 4096 7.1, 7.4).
+
+    A second wavefront for an fp32 row of 64 lanes wants 16 slots per lane (stable_l2 300 x 2048
+    3.13 us on one, 3.38 on two, and less exact: 8.9e-8 and 9.6e-8)."""
     per_slot = vec_of(var.dtype) if var.vector else 1
     slots = -(-ncols // per_slot)
     tpr = var.tpr
@@ -421,8 +431,19 @@ def _few_rows(var: FoldVariant, rows: int, ncols: int, merge: bool = False) -> F
     # 8 slots in flight and the fold (28 to 40 spilled).  logsumexp bf16 22 x 235968 25.8 us on 256
     # lanes, 18.8 on 512, 27.8 on 1024; 1 x 262144 22.1, 16.5, 25.1; 200 x 250000 31.5, 22.2, 34.4
     most = MAX_TPR // 2 if per_slot == 8 and not merge else MAX_TPR
-    while (tpr < most and rows * tpr < FEW_ROWS_LANES
-           and slots >= (16 if tpr == 64 and per_slot == 4 else 8) * tpr):
+
+    def pays(tpr):
+        if per_slot == 8 and merge:
+            return slots >= 8 * tpr
+        if tpr >= 512:
+            return 2 * rows <= CUS and slots >= 32 * tpr
+        if tpr >= 256:
+            return slots >= 12 * tpr and (rows <= CUS or (merge and slots <= 16 * tpr))
+        if merge and tpr >= 128 and rows > CUS:
+            return False
+        return slots >= (16 if tpr == 64 and per_slot == 4 else 8) * tpr
+
+    while tpr < most and rows * tpr < FEW_ROWS_LANES and pays(tpr):
         tpr *= 2
     if tpr == var.tpr:
         return var
@@ -665,11 +686,12 @@ def _row_variant(flat, gamma, width: int, *, tile: int | None = None) -> RowVari
     width 16384: 8 slots 88.4 / 89.0, 4 slots 89.0 / 88.9.
 
     Rows of fewer than 256 slots take the 2 to 5 slots per lane that leave the fewest lanes idle
-    (ragged 16-bit rows 2 to 4, fp32 ones 2: 30000 x 151 10.1 us, 3 slots 10.5, one element per load 10.9), rows of up to 8 slots one: with 8 a wavefront holds so many rows that a whole input is
-    one generation of wavefronts, which loads, then stores.  64 MB inputs, cold, RMSNorm /
+    (ragged 16-bit rows 2 to 4, fp32 ones 2: 30000 x 151 10.1 us, 3 slots 10.5, one element per
+    load 10.9), rows of up to 8 slots one: with 8 a wavefront holds so many rows that a whole input
+    is one generation of wavefronts, which loads, then stores.  64 MB inputs, cold, RMSNorm /
     L2-normalize: bf16 131072 x 64 38.4 / 38.8 -> 9.6 / 8.2 us, x 128 33.3 / 37.3 -> 13.8 / 13.5,
-    32000 x 1000 29.3 / 31.7 -> 24.1 / 23.9; fp32 131072 x
-    64 31.2 / 34.3 -> 13.6 / 13.5, 62500 x 256 24.9 / 24.9 -> 23.3 / 23.7.  fp32 rows of 512 to
+    32000 x 1000 29.3 / 31.7 -> 24.1 / 23.9; fp32 131072 x 64 31.2 / 34.3 -> 13.6 / 13.5,
+    62500 x 256 24.9 / 24.9 -> 23.3 / 23.7.  fp32 rows of 512 to
     1024 slots take 4 (7812 x 2048 24.7 / 25.3 -> 23.9 / 23.6).  Fewer than 8 rows are one or two
     workgroups whichever way and keep the shape above.
 
