@@ -378,7 +378,13 @@ def _segment_variant(flat, spans, channels: int) -> SegmentVariant:
     bf16 20000 x 20 x 100 23.8, 20.9, 20.2; bf16 3000 x 40 x 300 19.6, 18.1, 17.8;
     bf16 4096 x 16 x 64 6.4, 5.4, 8.5; bf16 300 x 200 x 512 17.4, 18.1, 24.3 (1/32 19.1);
     fp16 16 x 400 x 1024 20.0, 22.2, 30.0 (1/32 14.4); fp16 64 x 400 x 128 17.2, 19.5, 29.3
-    (1/32 12.8); fp32 347 x 13 x 246 4.1, 4.4, 4.9."""
+    (1/32 12.8); fp32 347 x 13 x 246 4.1, 4.4, 4.9.
+
+    Segments shorter than a step pay its tests per lane whatever they load, so on a full chip they
+    take wide chunks, and bf16 ones, whose adds round one by one, two words everywhere (1/16, 2/16,
+    4/16): fp16 60000 x 2 x 512 65.2, 46.6, 35.1, x 8 x 256 51.0, 47.7, 49.2; bf16 60000 x 4 x 256
+    45.3, 30.7, 28.4, x 11 x 256 83.0, 62.1, 64.5, 300 x 11 x 300 7.4, 6.5, 7.1; but fp16 1500 x 8
+    x 256 6.0, 6.4, 6.4."""
     dtype = str(flat.dtype).replace("torch.", "")
     span_dtype = str(spans.dtype).replace("torch.", "")
     size = flat.element_size()
@@ -389,6 +395,10 @@ def _segment_variant(flat, spans, channels: int) -> SegmentVariant:
         unroll = 32
     elif waves >= 2048 and channels * size % 256:
         words = 2 if waves < 4096 else 4
+    elif waves >= 8192 and nrows < 16 * nseg:
+        words = 4 if nrows < 6 * nseg else 2
+    if dtype == "bfloat16" and nrows < 16 * nseg:
+        words = max(words, 2)
     while words > 1 and channels * size < 4 * words:
         words //= 2
     # a launch has fewer than 2^32 lanes: the widest chunks where narrow ones make more
