@@ -145,6 +145,11 @@ TILE_256_US = {64: (1.1, 0.0), 128: (1.45, 0.6), 256: None}
 TILE_128_US = {64: 0.6, 128: 1.15, 256: 3.3}
 BLOCK_US, MERGE_US, STATE_BYTES_PER_US, PACK_US, PACK_BYTES_PER_US = 2.5, 6.0, 8e6, 4.0, 5e6
 MAX_STATE_BYTES = 256 << 20
+# Heads beyond the 256 MB of the last cache: a head's query blocks are a launch's width apart, so each
+# reads its K and V^T from HBM again, the fewer queries in a block, the more often (bf16 full, B*H=640
+# sq=601 sk=1184 d=128: 403 us with 256-query blocks, 474 with 128; B*H=1120 s=601 414 and 485; within
+# the cache, B*H=640 s=601, 241 and 215).  Causal blocks start with the longest and share more.
+CACHE_BYTES, CACHE_BYTES_PER_US = 256 << 20, 5.5e6
 # The short-query kernels: launch, a workgroup's start and end, its 4 waves' pass over 4 tiles of
 # 32 keys, and the workgroups the chip holds at once.
 SHORT_LAUNCH_US, SHORT_BLOCK_US = 3.0, 3.0
@@ -182,6 +187,9 @@ def _fold_cost(bh, sq, head_dim, causal, bm, blocks, tile_us, per):
     else:
         tiles = -(-items // CUS) * per
     cost = tile_us * tiles + BLOCK_US * max(1.0, items / CUS)
+    tile_bytes = bh * BLOCK_N * head_dim * 4           # of K and V^T, over the heads
+    if not causal and longest * tile_bytes > CACHE_BYTES:
+        cost = max(cost, total * tile_bytes / CACHE_BYTES_PER_US)
     if per < longest:
         state = 2 * 4 * items * sq / nqb * head_dim    # written and read, fp32
         cost += MERGE_US + state / STATE_BYTES_PER_US
