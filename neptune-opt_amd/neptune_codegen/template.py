@@ -373,14 +373,19 @@ def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: in
             unroll *= 2
     slots = -(-ncols // per_slot) if type(ncols) is int else 256
     if (resident and vector and not split_block and slots < 256 and x2.shape[0] >= 8
-            and (readout or per_slot == 8)):
+            and (readout or per_slot == 8)
+            and not (slots > 192 and x2.shape[0] * ncols < 1 << 22)):
         # Short rows: 1 slot per lane up to 8 slots, else 2 or 3, whichever idles fewer lanes (the
         # shape below is one generation of wavefronts that loads, then stores).  60 MB, cold:
         # log_softmax bf16 131072 x 64 17.9 -> 8.4 us, x 200 31.4 -> 21.9, 30000 x 1000 24.3 ->
         # 21.8, fp32 131072 x 64 16.7 -> 12.9, 75000 x 200 24.9 -> 21.5; variance bf16 131072 x 64
-        # 8.1 -> 5.7 (fp32 75000 x 200 11.8 -> 12.4: two-pass fp32 rows keep their shape).
+        # 8.1 -> 5.7 (fp32 75000 x 200 11.8 -> 12.4: two-pass fp32 rows keep their shape).  Rows of
+        # more than 192 slots need a second wave so, which few of them do not pay (log_softmax fp32
+        # 1000 x 1000 4.2 us on one wave of 4 slots, 4.5 on two of 2; 16384 x 1000 24.9, 23.8).
         unroll = 1 if slots <= 8 else min((2, 3), key=lambda n: n << max(0, (-(-slots // n) - 1).bit_length()))
         tpr = 1 << max(0, (-(-slots // unroll) - 1).bit_length())
+        if per_slot == 4 and unroll == 2 and _just_full(x2.shape[0] * tpr):
+            tpr, unroll = tpr // 2, 4
     elif resident and not split_block:
         if per_slot == 8:      # 16-bit rows: lanes first (up to 512), then slots
             unroll = UNROLL
@@ -398,6 +403,14 @@ def _fold_variant(x2, ncols: int, block: int, num_warps: int, *, split_block: in
         slots = -(-ncols // (tpr * per_slot))
         unroll = -(-slots // -(-slots // unroll))
     return FoldVariant(str(x2.dtype).replace("torch.", ""), vector, tpr, unroll, waves, ragged)
+
+
+def _just_full(lanes: int) -> bool:
+    """Launches that fill the last eighth of the 2^19 lanes the chip holds at once: the last
+    workgroups start when the first are done, so half the lanes with twice the slots are faster.
+    RMSNorm fp32 x 256, 2 slots / 4: 14 MB 7.0 / 6.9 us, 15 MB 7.6 / 7.0, 16.5 MB 8.2 / 7.1, 17 MB
+    8.6 / 8.7; bf16 x 256 14 MB 7.0 / 7.4, 16.5 MB 8.2 / 7.4, 17 MB 8.7 / 8.6."""
+    return 7 << 16 < lanes <= 1 << 19
 
 
 # Lanes below which a launch's rows are spread over more of them (512 per CU).
@@ -728,6 +741,14 @@ def _row_variant(flat, gamma, width: int, *, tile: int | None = None) -> RowVari
     while tpr > 1024:
         nv *= 2
         tpr = 1 << max(0, (max(1, -(-slots // nv)) - 1).bit_length())
+    if vector and tile is None:
+        # (16-bit rows of 128 slots up had 2 slots before the rule above, and are more exact so)
+        if nv == 2 and not ragged and (vec == 4 or slots < 128) and _just_full(flat.shape[0] * tpr):
+            tpr, nv = tpr // 2, 4
+        # ragged fp32 rows of 8 waves pay for their sum while the launch is short: RMSNorm x 3001, 512
+        # lanes / 256, 2 MB 4.0 / 4.1 us, 8 MB 5.9 / 5.6, 12 MB 7.6 / 7.0, 18 MB 10.2 / 10.0
+        elif ragged and vec == 4 and tpr == 512 and 1 << 18 < flat.shape[0] * tpr < 3 << 18:
+            tpr, nv = 256, 4
     nv = max(1, min(nv, -(-slots // tpr)))
     return RowVariant(str(flat.dtype).replace("torch.", ""), vector, tpr, nv, ragged)
 
