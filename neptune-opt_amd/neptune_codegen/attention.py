@@ -7,12 +7,14 @@ exp(s - s2) (tests/test_neptune_opt.py:347) applied per key tile to the running
 `is_causal=True` (query i sees keys j <= i).  The oracle is the closed form in fp32.
 
 Layout contract: q [B, H, Sq, D], k/v [B, H, Sk, D], D in {64, 128, 256}, one dtype (bf16 or
-fp16), unit stride on D; other strides are honoured (rows must be 16-byte aligned, otherwise the input is made
-contiguous).  Output is a fresh contiguous [B, H, Sq, D] tensor of the input dtype;
+fp16), unit stride on D; other strides are honoured (rows must be 16-byte aligned, otherwise the
+input is made contiguous).  Output is a fresh contiguous [B, H, Sq, D] tensor of the input dtype;
 `return_lse` adds the fp32 [B, H, Sq] natural-log logsumexp of the scaled, masked scores.
 
-Calls of at most 16 queries (decoding) run kernels of their own, which split a head's keys over
-workgroups and take P and V in fp32 (see SHORT_MAX_SQ); what follows is about the others.
+Calls of at most 16 queries (decoding), and longer ones that `_short_wins` estimates to be cheaper
+so (few heads, few keys), run kernels of their own: they split a head's keys over workgroups and
+take P and V in fp32 (see SHORT_MAX_SQ).  The MFMA path below is about the others; in both a hidden
+key's V reaches no query.
 
 Every input has a result; nothing is refused at run time and no device-side assert is used.
 The MFMA path feeds V to the P.V product as fp16 images scaled per 64-key tile by a power of
@@ -136,11 +138,12 @@ def _tile_chunks(units: int, tiles: int) -> tuple[int, int]:
     return -(-tiles // per), per
 
 
-# What `_fold_choice` and `_short_wins` price a call with, in us on MI355X, by head dim (fits of graph-replayed calls over
-# 24 shapes, cold): one workgroup's pass over a 64-key tile with a CU to itself -- the 256-query
-# kernels (two workgroups on a CU pass theirs hardly faster; at head dim 128 from 1.45 us on a
-# nearly empty chip to 2.05 on a full one, whose clock drops) and the 128-query one (4 waves x 32
-# queries) --, a workgroup's start and readout, and the merge launch with its state's traffic.
+# What `_fold_choice` and `_short_wins` price a call with, in us on MI355X, by head dim (fits of
+# graph-replayed calls over 24 shapes, cold): one workgroup's pass over a 64-key tile with a CU to
+# itself -- the 256-query kernels (two workgroups on a CU pass theirs hardly faster; at head dim 128
+# from 1.45 us on a nearly empty chip to 2.05 on a full one, whose clock drops) and the 128-query one
+# (4 waves x 32 queries) --, a workgroup's start and readout, and the merge launch with its state's
+# traffic.
 TILE_256_US = {64: (1.1, 0.0), 128: (1.45, 0.6), 256: None}
 TILE_128_US = {64: 0.6, 128: 1.15, 256: 3.3}
 BLOCK_US, MERGE_US, STATE_BYTES_PER_US, PACK_US, PACK_BYTES_PER_US = 2.5, 6.0, 8e6, 4.0, 5e6

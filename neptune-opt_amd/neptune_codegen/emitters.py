@@ -238,13 +238,15 @@ def _fold_kernel(sk: Skeleton, plan: str, part: str, var: FoldVariant) -> tuple[
     tmpl = f"Fold, {st}, {var.tpr}, {var.unroll}, {var.access}, {var.wg}"
     if plan == "serial":
         name = f"{sk.name}_serial_{var.tag()}"
-        body = (f"nep::fold_serial<{tmpl}{', true' if var.spread else ''}>((const {st}::T*)x, ({st}::T*)out, rows, ncols, "
+        spread = ", true" if var.spread else ""
+        body = (f"nep::fold_serial<{tmpl}{spread}>((const {st}::T*)x, ({st}::T*)out, rows, ncols, "
                 "stride_row, stride_col);")
         sig = _FOLD_ARGS_SERIAL
     elif plan == "two_pass":
         name = f"{sk.name}_two_pass_{var.tag()}"
-        body = (f"nep::fold_two_pass<{tmpl}, {str(var.resident).lower()}>((const {st}::T*)x, ({st}::T*)out, rows, ncols, "
-                "stride_row, stride_col);")
+        resident = str(var.resident).lower()
+        body = (f"nep::fold_two_pass<{tmpl}, {resident}>((const {st}::T*)x, ({st}::T*)out, rows, "
+                "ncols, stride_row, stride_col);")
         sig = _FOLD_ARGS_SERIAL
     elif part == "partial":
         name = f"{sk.name}_partial_{var.tag()}"

@@ -480,10 +480,10 @@ def _run_spans(launch, lengths, status_ptr: int):
 
 def _device_spans(data, segments, *, offsets, status=None):
     """[start, end) boundaries for the fused-validation launch: offsets as given, lengths as an
-    int64 prefix sum (the same values `_segment_spans` builds) by two HIP launches -- block
-    sums, then a per-block scan on top of the preceding blocks; no asserts here (the segment
-    kernel checks the spans).  With lengths, the first launch also sets `status` (one int32)
-    to 1; returns (spans, status set)."""
+    int64 prefix sum (the same values `_segment_spans` builds) by one HIP launch up to
+    SPAN_DIRECT_MAX lengths, by two beyond -- block sums, then a per-block scan on top of the
+    preceding blocks; no asserts here (the segment kernel checks the spans).  With lengths, the
+    first launch also sets `status` (one int32) to 1; returns (spans, status set)."""
     if offsets:
         return segments, False
     lengths = segments.contiguous()
@@ -545,9 +545,10 @@ def _launch_segment(name, data, segments, params, plan, *, wrapper=None):
         launch = launch_segment_kernel(compile_segment_reduction(name, params, plan), flat, spans,
                                        out, status=status, cover=cover)
         torch._assert_async(status, DESCRIPTOR_MESSAGE)
+        index = data.device.index if data.device.index is not None else torch.cuda.current_device()
         if (key is not None and flat.data_ptr() == data.data_ptr()
-                and (params["offsets"] or segments.is_contiguous()) and status is _STATUS.get(data.device.index if data.device.index is not None
-                                          else torch.cuda.current_device())):
+                and (params["offsets"] or segments.is_contiguous())
+                and status is _STATUS.get(index)):
             if len(_SEG_SEEN) >= 4096:
                 _SEG_SEEN.clear()
             spans_launch = None if params["offsets"] else _spans_launch(segments)
