@@ -382,9 +382,10 @@ def _segment_variant(flat, spans, channels: int) -> SegmentVariant:
 
     Segments shorter than a step pay its tests per lane whatever they load, so on a full chip they
     take wide chunks, and bf16 ones, whose adds round one by one, two words everywhere (1/16, 2/16,
-    4/16): fp16 60000 x 2 x 512 65.2, 46.6, 35.1, x 8 x 256 51.0, 47.7, 49.2; bf16 60000 x 4 x 256
-    45.3, 30.7, 28.4, x 11 x 256 83.0, 62.1, 64.5, 300 x 11 x 300 7.4, 6.5, 7.1; but fp16 1500 x 8
-    x 256 6.0, 6.4, 6.4."""
+    4/16; on a full chip also beside one whole step): fp16 60000 x 2 x 512 65.2, 46.6, 35.1, x 8 x 256 51.0, 47.7, 49.2; bf16 60000 x 4 x 256
+    45.3, 30.7, 28.4, x 11 x 256 83.0, 62.1, 64.5, 300 x 11 x 300 7.4, 6.5, 7.1, 6000 x 26 x 256
+    19.6, 18.1, 18.0; but fp16 1500 x 8 x 256 6.0, 6.4, 6.4.  Long fp32 segments keep one word below
+    4096 waves (1500 x 100 x 100 18.2, 19.8, 18.1)."""
     dtype = str(flat.dtype).replace("torch.", "")
     span_dtype = str(spans.dtype).replace("torch.", "")
     size = flat.element_size()
@@ -394,10 +395,10 @@ def _segment_variant(flat, spans, channels: int) -> SegmentVariant:
     if waves < 512 and nrows >= 64 * nseg:
         unroll = 32
     elif waves >= 2048 and channels * size % 256:
-        words = 2 if waves < 4096 else 4
+        words = 4 if waves >= 4096 else (1 if size == 4 and nrows >= 32 * nseg else 2)
     elif waves >= 8192 and nrows < 16 * nseg:
         words = 4 if nrows < 6 * nseg else 2
-    if dtype == "bfloat16" and nrows < 16 * nseg:
+    if dtype == "bfloat16" and (nrows < 16 * nseg or (waves >= 8192 and 16 * nseg < nrows < 32 * nseg)):
         words = max(words, 2)
     while words > 1 and channels * size < 4 * words:
         words //= 2

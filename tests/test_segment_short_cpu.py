@@ -22,7 +22,10 @@ def test_words_of_short_segments(dtype):
         assert _words(dtype, 60000, 6, channels) == 2
         assert _words(dtype, 60000, 15, channels) == 2
         assert _words(dtype, 60000, 16, channels) == 1
+        assert _words(dtype, 60000, 26, channels) == small
+        assert _words(dtype, 60000, 32, channels) == 1
         assert _words(dtype, 300, 4, channels) == small
         assert _words(dtype, 300, 40, channels) == 1
     assert _words(dtype, 300, 11, 300) == small
     assert _words(dtype, 25000, 11, 300) == 4
+    assert _words(torch.float32, 1500, 100, 100) == 1 and _words(torch.float32, 1500, 20, 100) == 2
