@@ -509,9 +509,8 @@ def _launch_segment(name, data, segments, params, plan, *, wrapper=None):
             and not hip.recording_active()):
         try:
             key = (name, plan, tuple(sorted((k, type(v).__name__, repr(v)) for k, v in params.items())),
-                   data.dtype, data.device, tuple(data.shape), tuple(data.stride()),
-                   data.data_ptr() % 16, segments.dtype, segments.device, tuple(segments.shape),
-                   tuple(segments.stride()))
+                   data.dtype, data.device, data.shape, data.stride(), data.data_ptr() % 16,
+                   segments.dtype, segments.device, segments.shape, segments.stride())
             entry = _SEG_SEEN.get(key)
         except TypeError:
             key, entry = None, None
